@@ -17,7 +17,14 @@ from pathlib import Path
 HERE = Path(__file__).resolve().parent
 CSRC = HERE / "csrc"
 OUT = HERE / "libpippin_hip.so"
-SOURCES = ["runtime.hip", "mlp.hip", "host_model.cpp", "mjcf.cpp", "meshes.cpp", "urdf.cpp"]
+# the step kernels' instances, one object each (step_kernels.hpp)
+INSTANCES = {"k1": (1, "DModel"), "k2": (2, "DModel"), "k4": (4, "DModel"), "ant": (4, "SpecAnt")}
+# (source, object name, extra flags), the slowest to compile first
+UNITS = [
+    (src, f"{src[:-4]}_{tag}.o", [f"-DPH_K={k}", f"-DPH_MT={mt}", f"-DPH_TAG={tag}"])
+    for src in ("step_inst.hip", "step_mlp_inst.hip") for tag, (k, mt) in INSTANCES.items()
+] + [(src, src + ".o", []) for src in
+     ("runtime.hip", "mlp.hip", "host_model.cpp", "mjcf.cpp", "meshes.cpp", "urdf.cpp")]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("PIPPIN_HIP_ARCH", "gfx950")
 FLAGS = [
@@ -49,22 +56,23 @@ def generate_specs(bdir: Path, verbose: bool = False) -> None:
 
 
 def build(verbose: bool = False) -> Path:
-    objs = []
+    from concurrent.futures import ThreadPoolExecutor
+
     bdir = HERE / "_build"
     bdir.mkdir(exist_ok=True)
     generate_specs(bdir, verbose)
-    procs = []
-    for src in SOURCES:  # compiled side by side
-        obj = bdir / (src + ".o")
+
+    def compile_unit(unit) -> str:
+        src, name, extra = unit
         lang = ["-x", "hip"] if src.endswith(".cpp") else []
-        cmd = [HIPCC, *FLAGS, *lang, "-I", str(bdir), "-c", str(CSRC / src), "-o", str(obj)]
+        cmd = [HIPCC, *FLAGS, *extra, *lang, "-I", str(bdir), "-c", str(CSRC / src), "-o", str(bdir / name)]
         if verbose:
             print(" ".join(cmd), flush=True)
-        procs.append((cmd, subprocess.Popen(cmd)))
-        objs.append(str(obj))
-    failed = [cmd for cmd, p in procs if p.wait() != 0]
-    if failed:
-        raise subprocess.CalledProcessError(1, failed[0])
+        subprocess.run(cmd, check=True)
+        return str(bdir / name)
+
+    with ThreadPoolExecutor(max_workers=min(8, os.cpu_count() or 1)) as pool:  # side by side
+        objs = list(pool.map(compile_unit, UNITS))
     tmp = OUT.with_suffix(".so.tmp")
     cmd = [HIPCC, *FLAGS, "-shared", "-o", str(tmp), *objs]
     subprocess.run(cmd, check=True)

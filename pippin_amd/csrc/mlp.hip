@@ -9,7 +9,7 @@
 
 #include "kstep.hpp"
 #include "mlp_host.hpp"
-#include "spec_models.hpp"
+#include "step_kernels.hpp"
 
 using namespace phk;
 
@@ -260,26 +260,12 @@ int pick_splits(int64_t B, int want) {
 
 namespace phm {
 
-const void* step_kernel(int K, int spec) {
-  if (spec == 1 && K == 4) return (const void*)k_step_mlp<4, SpecAnt>;
-  return K == 4 ? (const void*)k_step_mlp<4, DModel>
-                : K == 2 ? (const void*)k_step_mlp<2, DModel> : (const void*)k_step_mlp<1, DModel>;
-}
+const void* step_kernel(int K, int spec) { return mlp_kernel(K, spec); }
 
 void launch_step(int K, int spec, unsigned grid, size_t lds, hipStream_t st, const DModel* M, const DState* S,
                  int64_t begin, int64_t end, int64_t nstep, const double* ctrl, double* qpos_out) {
-  if (spec == 1 && K == 4)
-    hipLaunchKernelGGL((k_step_mlp<4, SpecAnt>), dim3(grid), dim3(64), lds, st, M, S, begin, end, nstep, ctrl,
-                       qpos_out);
-  else if (K == 4)
-    hipLaunchKernelGGL((k_step_mlp<4, DModel>), dim3(grid), dim3(64), lds, st, M, S, begin, end, nstep, ctrl,
-                       qpos_out);
-  else if (K == 2)
-    hipLaunchKernelGGL((k_step_mlp<2, DModel>), dim3(grid), dim3(64), lds, st, M, S, begin, end, nstep, ctrl,
-                       qpos_out);
-  else
-    hipLaunchKernelGGL((k_step_mlp<1, DModel>), dim3(grid), dim3(64), lds, st, M, S, begin, end, nstep, ctrl,
-                       qpos_out);
+  void* args[] = {&M, &S, &begin, &end, &nstep, &ctrl, &qpos_out};
+  (void)hipLaunchKernel(mlp_kernel(K, spec), dim3(grid), dim3(64), args, lds, st);
 }
 
 MlpW view(const Net& n, int mode) {

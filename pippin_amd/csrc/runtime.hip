@@ -22,20 +22,11 @@
 #include "kstep.hpp"
 #include "mlp_host.hpp"
 #include "spec_models.hpp"
+#include "step_kernels.hpp"
 
 using namespace phk;
 
 // ---------------------------------------------------------------- kernels
-static const void* step_kernel(int K, int spec) {
-  if (spec == 1 && K == 4) return (const void*)k_step<4, SpecAnt>;
-  return K == 4 ? (const void*)k_step<4, DModel> : K == 2 ? (const void*)k_step<2, DModel> : (const void*)k_step<1, DModel>;
-}
-static const void* ws_kernel(int K, int spec) {
-  if (spec == 1 && K == 4) return (const void*)k_step_ws<4, SpecAnt>;
-  return K == 4 ? (const void*)k_step_ws<4, DModel>
-                : K == 2 ? (const void*)k_step_ws<2, DModel> : (const void*)k_step_ws<1, DModel>;
-}
-
 // Kinematics only (poses after set(qpos) / reset), for listed envs or a range.
 __global__ void __launch_bounds__(64) k_kin(const DModel* __restrict__ Mp, const DState* __restrict__ Sp,
                                             int64_t begin, const int64_t* ids) {
