@@ -22,7 +22,8 @@ INSTANCES = {"k1": (1, "DModel"), "k2": (2, "DModel"), "k4": (4, "DModel"), "ant
 # (source, object name, extra flags), the slowest to compile first
 UNITS = [
     (src, f"{src[:-4]}_{tag}.o", [f"-DPH_K={k}", f"-DPH_MT={mt}", f"-DPH_TAG={tag}"])
-    for src in ("step_inst.hip", "step_mlp_inst.hip") for tag, (k, mt) in INSTANCES.items()
+    for src in ("step_inst.hip", "step_mlp_inst.hip", "pgs_inst.hip") for tag, (k, mt) in INSTANCES.items()
+    if src != "pgs_inst.hip" or mt == "DModel"
 ] + [(src, src + ".o", []) for src in
      ("runtime.hip", "mlp.hip", "host_model.cpp", "mjcf.cpp", "meshes.cpp", "urdf.cpp")]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

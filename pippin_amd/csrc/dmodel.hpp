@@ -96,6 +96,10 @@ struct DModel {
   int ncmax;  // contact capacity per env (the sum of per-pair maxima: never exceeded)
   int nrmax;  // row capacity per env (4 per contact for Newton, 3 for PGS, + limits + equalities)
   int nrl;    // rows kept in LDS; larger problems use the global row buffers
+  // PGS: the most dofs that one row and its M^-1 J^T can hold (the dof blocks of the two
+  // bodies of a pair, of a limited joint or of an equality), and the largest such block;
+  // 0 when a row can hold more than 16
+  int pgs_w, pgs_b;
   int hess_mfma;  // 1: Newton's dense Hessian J'DJ on the FP64 matrix cores (one env per wavefront only)
 
   gp<const int> body_parent, body_jntadr, body_jntnum, body_dofadr, body_dofnum, body_lastdof;

@@ -486,6 +486,25 @@ void init_dmodel_scalars(const HostModel& hm, int solver, int max_contacts, phk:
   M.ncmax = std::max(hm.ncmax, 1);
   if (max_contacts > 0) M.ncmax = std::min(M.ncmax, max_contacts);
   M.nrmax = std::max(4 * M.ncmax + 2 * hm.nlimited + d.neq, 1);
+  // the widest PGS row: the dof blocks it touches
+  {
+    auto block_of = [&](int dof) { return dof < 0 ? -1 : hm.dof_block[dof]; };
+    auto size_of = [&](int b) { return b < 0 ? 0 : hm.block_adr[b + 1] - hm.block_adr[b]; };
+    int w = 1, bmax = 1;
+    auto touch = [&](int a, int b) {
+      w = std::max(w, a == b ? size_of(a) : size_of(a) + size_of(b));
+      bmax = std::max(bmax, std::max(size_of(a), size_of(b)));
+    };
+    for (size_t i = 0; i < hm.pair_g1.size(); i++)
+      touch(block_of(hm.body_lastdof[hm.geom_body[hm.pair_g1[i]]]), block_of(hm.body_lastdof[hm.geom_body[hm.pair_g2[i]]]));
+    for (int j = 0; j < d.njnt; j++)
+      if (hm.jnt_limited[j]) touch(block_of(hm.jnt_dofadr[j]), -1);
+    for (int e = 0; e < d.neq; e++)
+      touch(block_of(hm.jnt_dofadr[hm.eq_joint1[e]]),
+            hm.eq_joint2[e] >= 0 ? block_of(hm.jnt_dofadr[hm.eq_joint2[e]]) : -1);
+    M.pgs_w = w <= 16 ? w : 0;
+    M.pgs_b = w <= 16 ? bmax : 0;
+  }
   // island scratch (newton.rs:378-473), only when several dof blocks exist
   M.isl_fstride = M.nblock > 1 ? d.nv * d.nv + M.nrmax * (d.nv + 2) + 4 * d.nv : 0;
   M.isl_istride = M.nblock > 1 ? 2 * M.nrmax + d.nv + 2 * M.nblock + 1 : 0;  // ints, in LDS (Layout::i_isl)

@@ -1489,8 +1489,9 @@ PHD void solve_serial(const Real* L, int nv, int s0, int e, Real* x) {
   }
 }
 
-// Row record of the PGS problem (HBM, 10 doubles per row).
-enum { PR_SEP = 0, PR_MU, PR_INVA, PR_LAM, PR_KIND, PR_NORMAL, PR_CONTACT };
+// Row record of the PGS problem (HBM, 10 doubles per row). PR_FLAGS and PR_B1
+// belong to packed rows (pgs_prepare_packed).
+enum { PR_SEP = 0, PR_MU, PR_INVA, PR_LAM, PR_KIND, PR_NORMAL, PR_CONTACT, PR_FLAGS, PR_B1, PR_MODE };
 enum { PK_NORMAL = 0, PK_FRICTION = 1, PK_BILATERAL = 2 };
 
 // Soft-constraint coefficients and stopping rule of the sweeps (solver.rs:44-50, :229-240).
@@ -1763,6 +1764,43 @@ PHD void pgs_apply_warm(const MT& M, const DState& S, Env& E, int nr, Real* v) {
   });
 }
 
+// Warm-start forces from the matching previous contact (solver.rs:253-289), left
+// in the row records.
+template <class X, class MT>
+PHD void pgs_match_warm(const MT& M, const DState& S, Env& E, Real* rw, int ncon) {
+  auto con = S.con + E.e * (int64_t)M.ncmax * CW;
+  auto cg = S.cgeom + E.e * (int64_t)M.ncmax * 3;
+  auto pcon = S.pcon + E.e * (int64_t)M.ncmax * CW;
+  auto pcg = S.pcgeom + E.e * (int64_t)M.ncmax * 3;
+  auto plam = S.plambda + E.e * (int64_t)M.ncmax * 3;
+  const int npc = S.npcon[E.e];
+  X::par(ncon, [&](int c) {
+    if (npc == 0) return;
+    auto cc = con + c * CW;
+    Real bd = 0.01 * 0.01;
+    int bi = -1;
+    V3 cp = ld3(cc);
+    for (int pi = 0; pi < npc; pi++) {
+      if (pcg[3 * pi] == cg[3 * c] && pcg[3 * pi + 1] == cg[3 * c + 1]) {
+        Real d2 = norm2(ld3(pcon + pi * CW) - cp);
+        if (d2 < bd) {
+          bd = d2;
+          bi = pi;
+        }
+      }
+    }
+    if (bi >= 0) {
+      V3 pt1, pt2, t1, t2;
+      contact_frame(pcon + bi * CW, &pt1, &pt2);
+      contact_frame(cc, &t1, &t2);
+      V3 f = pt1 * plam[3 * bi + 1] + pt2 * plam[3 * bi + 2];
+      rw[(3 * c) * 10 + PR_LAM] = plam[3 * bi];
+      rw[(3 * c + 1) * 10 + PR_LAM] = dot(f, t1);
+      rw[(3 * c + 2) * 10 + PR_LAM] = dot(f, t2);
+    }
+  });
+}
+
 // pgs_prepare returns the row count, 0 when there is nothing to solve (then v,
 // vpos and the history are final), or -1 when the rows overflowed. Without
 // apply_warm it stops with the warm-start forces in the row records, before
@@ -1882,36 +1920,7 @@ PHD int pgs_prepare(const MT& M, const DState& S, Env& E, Real* v, Real* vpos, b
     for (int k = 0; k < nv; k++) a += J[r * nv + k] * x[k];
     rw[r * 10 + PR_INVA] = a > 1e-12 ? 1.0 / a : 0.0;
   });
-  // warm start from the matching previous contact (solver.rs:253-289)
-  auto pcon = S.pcon + E.e * (int64_t)M.ncmax * CW;
-  auto pcg = S.pcgeom + E.e * (int64_t)M.ncmax * 3;
-  auto plam = S.plambda + E.e * (int64_t)M.ncmax * 3;
-  const int npc = S.npcon[E.e];
-  X::par(ncon, [&](int c) {
-    if (npc == 0) return;
-    auto cc = con + c * CW;
-    Real bd = 0.01 * 0.01;
-    int bi = -1;
-    V3 cp = ld3(cc);
-    for (int pi = 0; pi < npc; pi++) {
-      if (pcg[3 * pi] == cg[3 * c] && pcg[3 * pi + 1] == cg[3 * c + 1]) {
-        Real d2 = norm2(ld3(pcon + pi * CW) - cp);
-        if (d2 < bd) {
-          bd = d2;
-          bi = pi;
-        }
-      }
-    }
-    if (bi >= 0) {
-      V3 pt1, pt2, t1, t2;
-      contact_frame(pcon + bi * CW, &pt1, &pt2);
-      contact_frame(cc, &t1, &t2);
-      V3 f = pt1 * plam[3 * bi + 1] + pt2 * plam[3 * bi + 2];
-      rw[(3 * c) * 10 + PR_LAM] = plam[3 * bi];
-      rw[(3 * c + 1) * 10 + PR_LAM] = dot(f, t1);
-      rw[(3 * c + 2) * 10 + PR_LAM] = dot(f, t2);
-    }
-  });
+  pgs_match_warm<X>(M, S, E, rw, ncon);
   if (apply_warm) pgs_apply_warm<X>(M, S, E, nr, v);
   return nr;
 }
@@ -2000,27 +2009,18 @@ PHD int pgs_sweeps(const MT& M, const DState& S, Env& E, int nr, Real* v, Real* 
   return sweeps;
 }
 
-// The constraint force and the history for the next warm start, after the
-// sweeps over nr > 0 rows.
+// The history for the next warm start, after the sweeps over the rows. (The
+// reference also forms qfrc_constraint here, which nothing of a PGS step reads.)
 template <class X, class MT>
-PHD void pgs_finish(const MT& M, const DState& S, Env& E, int nr) {
-  const int nv = M.nv;
-  const Real h = M.timestep;
+PHD void pgs_finish(const MT& M, const DState& S, Env& E) {
   int* isc = E.si + M.L.i_iscal;
   auto con = S.con + E.e * (int64_t)M.ncmax * CW;
   auto cg = S.cgeom + E.e * (int64_t)M.ncmax * 3;
-  Real* J = (S.gjac + E.e * (int64_t)M.nrmax * nv).p;
   Real* rw = (S.grow + E.e * (int64_t)M.nrmax * 10).p;
   auto pcon = S.pcon + E.e * (int64_t)M.ncmax * CW;
   auto pcg = S.pcgeom + E.e * (int64_t)M.ncmax * 3;
   auto plam = S.plambda + E.e * (int64_t)M.ncmax * 3;
   const int ncon = isc[0];
-  // qfrc_constraint = sum_r J_r lambda_r / h, rows in order
-  X::par(nv, [&](int k) {
-    Real f = 0.0;
-    for (int r = 0; r < nr; r++) f += J[r * nv + k] * rw[r * 10 + PR_LAM] / h;
-    LD(qfrc_c)[k] = f;
-  });
   // history for the next warm start: this step's contacts and their forces
   X::par(ncon * CW, [&](int t) { pcon[t] = con[t]; });
   X::par(ncon, [&](int c) {
@@ -2032,12 +2032,477 @@ PHD void pgs_finish(const MT& M, const DState& S, Env& E, int nr) {
   X::par(1, [&](int) { S.npcon[E.e] = ncon; });
 }
 
+// ---------------- packed PGS rows ----------------
+// A row J_r and its M^-1 J_r^T are zero outside the dof blocks that the row
+// touches (for a contact the blocks of its two bodies). When that is at most
+// 16 dofs for every row of a model (DModel::pgs_w), the rows are kept packed:
+// `count` entries of J_r and of M^-1 J_r^T each, for the dofs a .. a + na - 1
+// of the lower block and b .. of the upper one, from `off` in the env's slice
+// of gjac and gmj. The words that were zeros do not move and are not summed:
+// a zero product added to a sum changes at most the sign of a zero, which no
+// later use depends on, unless a velocity or force is not finite; those cases
+// are handled where they arise (pgs_sweeps_rows).
+struct PgsRow {
+  int kind, hard, sub, a, na, b, count;
+  int64_t off;
+  PHD int dof(int l) const { return l < na ? a + l : b + (l - na); }
+};
+// kind 2 bits, hard 1 (separated row: its bias stays in the second phase),
+// sub 2 (rows after the contact's normal row), a, na, b 8 each, count 5, off 24
+PHD Real pgs_flags(const PgsRow& r) {
+  const int64_t w = (int64_t)r.kind | (int64_t)r.hard << 2 | (int64_t)r.sub << 3 | (int64_t)r.a << 8 |
+                    (int64_t)r.na << 16 | (int64_t)r.b << 24 | (int64_t)r.count << 32 | r.off << 40;
+  return __builtin_bit_cast(Real, w);
+}
+PHD PgsRow pgs_row(Real flags) {
+  const int64_t w = __builtin_bit_cast(int64_t, flags);
+  const int lo = (int)w, hi = (int)(w >> 32);
+  PgsRow r;
+  r.kind = lo & 3;
+  r.hard = (lo >> 2) & 1;
+  r.sub = (lo >> 3) & 3;
+  r.a = (lo >> 8) & 255;
+  r.na = (lo >> 16) & 255;
+  r.b = (lo >> 24) & 255;
+  r.count = hi & 255;
+  r.off = (int64_t)((unsigned)hi >> 8);
+  return r;
+}
+constexpr int64_t PGS_OFF_MAX = 1 << 24;
+
+// The dofs of a row on blocks k1 and k2 (-1: none).
+template <class MT>
+PHD void pgs_span(const MT& M, int k1, int k2, PgsRow* r) {
+  const int lo = k1 < 0 ? k2 : (k2 < 0 ? k1 : (k1 < k2 ? k1 : k2)), hi = k1 > k2 ? k1 : k2;
+  r->a = r->na = r->b = r->count = 0;
+  if (lo < 0) return;
+  r->a = M.block_adr[lo];
+  r->na = M.block_adr[lo + 1] - r->a;
+  r->count = r->na;
+  if (hi != lo) {
+    r->b = M.block_adr[hi];
+    r->count += M.block_adr[hi + 1] - r->b;
+  }
+}
+
+// (M + h D)^-1 x on one factored block of n <= NB dofs, on one lane in
+// registers, in the order of math.rs:449-463 (solve_serial). L points at the
+// block's first row, rows nv apart.
+template <int NB, class LP>
+PHD void pgs_solve_block(LP L, int nv, int n, Real* x) {
+#pragma unroll
+  for (int i = 0; i < NB; i++) {
+    if (i < n) {
+      Real s;
+      if (i < 8) {
+        s = 0.0;
+#pragma unroll
+        for (int k = 0; k < i; k++) s = s + L[i * nv + k] * x[k];
+      } else {
+        Real s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+#pragma unroll
+        for (int k = 0; k + 4 <= i; k += 4) {
+          s0 = s0 + L[i * nv + k] * x[k];
+          s1 = s1 + L[i * nv + k + 1] * x[k + 1];
+          s2 = s2 + L[i * nv + k + 2] * x[k + 2];
+          s3 = s3 + L[i * nv + k + 3] * x[k + 3];
+        }
+        s = (s0 + s1) + (s2 + s3);
+#pragma unroll
+        for (int k = i / 4 * 4; k < i; k++) s = s + L[i * nv + k] * x[k];
+      }
+      x[i] = (x[i] - s) / L[i * nv + i];
+    }
+  }
+#pragma unroll
+  for (int i = NB - 1; i >= 0; i--) {
+    if (i < n) {
+      x[i] = x[i] / L[i * nv + i];
+#pragma unroll
+      for (int k = 0; k < i; k++) x[k] = x[k] + -x[i] * L[i * nv + k];
+    }
+  }
+}
+
+// M^-1 J_r^T and the row's inverse effective mass, one row per lane. The
+// block solves run in registers; through the row's HBM slice, with every dof
+// block solved for every row, they took 76 us per step on the six-body pile.
+template <int NB, class X, class MT>
+PHD void pgs_packed_masses(const MT& M, Env& E, const Real* J, Real* mj, Real* rw, int nr) {
+  const int nv = M.nv;
+  X::par(nr, [&](int r) {
+    const PgsRow w = pgs_row(rw[r * 10 + PR_FLAGS]);
+    const Real* jr = J + w.off;
+    Real* mr = mj + w.off;
+    Real sum = rsum0();
+    for (int part = 0; part < 2; part++) {
+      const int o = part == 0 ? 0 : w.na, n = part == 0 ? w.na : w.count - w.na, s0 = part == 0 ? w.a : w.b;
+      if (n <= 0) continue;
+      Real x[NB], j[NB];
+#pragma unroll
+      for (int k = 0; k < NB; k++) {
+        j[k] = jr[o + (k < n ? k : n - 1)];
+        x[k] = j[k];
+      }
+      pgs_solve_block<NB>(LD(chol) + s0 * nv + s0, nv, n, x);
+#pragma unroll
+      for (int k = 0; k < NB; k++)
+        if (k < n) {
+          mr[o + k] = x[k];
+          sum += j[k] * x[k];
+        }
+    }
+    rw[r * 10 + PR_INVA] = sum > 1e-12 ? 1.0 / sum : 0.0;
+  });
+}
+
+template <class MT>
+PHD PgsConsts pgs_consts(const MT& M);
+
+// The bias of a row in the first phase (solver.rs:175-207), and whether the
+// row is separated.
+PHD Real pgs_bias(const PgsConsts& C, int kind, Real sep, int* hard) {
+  *hard = 0;
+  if (kind == PK_NORMAL) {
+    const Real sp = sep + C.slop;
+    *hard = sp > 0.0 ? 1 : 0;
+    return sp > 0.0 ? sp / C.h : rmax(C.bias_rate * sp, -C.max_bias);
+  }
+  return rclamp(C.bias_rate * sep, -C.max_bias, C.max_bias);
+}
+
+// Doubles that the packed rows of an env take in the sweeps' storage:
+// velocities with a spare one, PGS_REC per row, both entries of every row, and
+// 16 past the end for lanes beyond a row's entries.
+constexpr int PGS_REC = 6;
+PHD int64_t pgs_packed_doubles(int nv, int64_t nr, int64_t entries) {
+  return ((nv + 2) & ~1) + PGS_REC * nr + 2 * entries + 16;
+}
+
+// pgs_prepare with packed rows, stopping before the warm start moves v. Takes
+// the env when its rows fit `cap` doubles of the sweeps' storage and its mass
+// factor is finite; returns -2 when it does not, with nothing written that
+// pgs_prepare does not write again.
+template <class X, class MT>
+PHD int pgs_prepare_packed(const MT& M, const DState& S, Env& E, Real* v, Real* vpos, int64_t cap) {
+  const int nv = M.nv;
+  const Real h = M.timestep;
+  int* isc = E.si + M.L.i_iscal;
+  auto con = S.con + E.e * (int64_t)M.ncmax * CW;
+  auto cg = S.cgeom + E.e * (int64_t)M.ncmax * 3;
+  Real* J = (S.gjac + E.e * (int64_t)M.nrmax * nv).p;
+  Real* mj = (S.gmj + E.e * (int64_t)M.nrmax * nv).p;
+  Real* rw = (S.grow + E.e * (int64_t)M.nrmax * 10).p;
+  const Real* qpos = LD(qpos);
+  const int ncon = isc[0];
+  const PgsConsts C = pgs_consts(M);
+  int* coff = reinterpret_cast<int*>(LD(cact));  // per contact: entries of its J rows, then their offset
+  auto span_of = [&](int c, PgsRow* r) {
+    const int d1 = M.body_lastdof[M.geom_body[cg[3 * c]]], d2 = M.body_lastdof[M.geom_body[cg[3 * c + 1]]];
+    pgs_span(M, d1 < 0 ? -1 : M.dof_block[d1], d2 < 0 ? -1 : M.dof_block[d2], r);
+  };
+  // the limits within reach (solver.rs:92-113): each adds one row of its block
+  auto limit_seps = [&](int j, Real* seps) {
+    const int t = M.jnt_type[j];
+    if (!M.jnt_limited[j] || !(t == J_HINGE || t == J_SLIDE)) return 0;
+    const Real q = qpos[M.jnt_qposadr[j]];
+    const Real reach = M.margin + 2.0 * h * fabs(v[M.jnt_dofadr[j]]);
+    seps[0] = q - M.jnt_range[2 * j];
+    seps[1] = M.jnt_range[2 * j + 1] - q;
+    return (seps[0] < reach ? 1 : 0) + (seps[1] < reach ? 2 : 0);
+  };
+  X::par(ncon, [&](int c) {
+    PgsRow r{};
+    span_of(c, &r);
+    coff[c] = r.count;
+  });
+  X::par(1, [&](int) {
+    int64_t off = 0;
+    for (int c = 0; c < ncon; c++) {
+      const int n = coff[c];
+      coff[c] = (int)off;
+      off += 3 * n;
+    }
+    int nr = 3 * ncon;
+    bool fits = true;
+    auto add = [&](PgsRow w, Real sep, int kind) {
+      w.kind = kind;
+      w.sub = 0;
+      w.off = off;
+      Real* q = rw + nr * 10;
+      q[PR_SEP] = sep;
+      q[PR_MU] = 0.0;
+      q[PR_INVA] = 0.0;
+      q[PR_LAM] = 0.0;
+      q[PR_KIND] = kind;
+      q[PR_NORMAL] = 0;
+      q[PR_CONTACT] = -1;
+      q[PR_B1] = pgs_bias(C, kind, sep, &w.hard);
+      q[PR_FLAGS] = pgs_flags(w);
+      for (int k = 0; k < w.count; k++) J[off + k] = 0.0;
+      off += w.count;
+      nr++;
+    };
+    auto entry = [&](const PgsRow& w, int dof) { return dof < w.a + w.na && dof >= w.a ? dof - w.a : w.na + dof - w.b; };
+    for (int j = 0; j < M.njnt && fits; j++) {
+      Real seps[2];
+      const int f = limit_seps(j, seps);
+      for (int sg = 0; sg < 2; sg++)
+        if ((f >> sg) & 1) {
+          if (nr >= M.nrmax) {
+            fits = false;
+            break;
+          }
+          PgsRow w{};
+          const int da = M.jnt_dofadr[j];
+          pgs_span(M, M.dof_block[da], -1, &w);
+          J[off + entry(w, da)] = 0.0;
+          const int64_t o = off;
+          add(w, seps[sg], PK_NORMAL);
+          J[o + entry(w, da)] = sg == 0 ? 1.0 : -1.0;
+        }
+    }
+    for (int e = 0; e < M.neq && fits; e++) {
+      if (nr >= M.nrmax) {
+        fits = false;
+        break;
+      }
+      const int j1 = M.eq_j1[e], j2 = M.eq_j2[e];
+      auto c = M.eq_poly + 5 * e;
+      const Real q1 = qpos[M.jnt_qposadr[j1]] - M.qpos0[M.jnt_qposadr[j1]];
+      const int d1 = M.jnt_dofadr[j1], d2 = j2 >= 0 ? M.jnt_dofadr[j2] : -1;
+      PgsRow w{};
+      pgs_span(M, M.dof_block[d1], d2 < 0 ? -1 : M.dof_block[d2], &w);
+      Real poly = c[0], dpoly = 0.0;
+      if (j2 >= 0) {
+        const Real x = qpos[M.jnt_qposadr[j2]] - M.qpos0[M.jnt_qposadr[j2]];
+        poly = c[0] + x * (c[1] + x * (c[2] + x * (c[3] + x * c[4])));
+        dpoly = c[1] + x * (2.0 * c[2] + x * (3.0 * c[3] + x * 4.0 * c[4]));
+      }
+      const int64_t o = off;
+      add(w, q1 - poly, PK_BILATERAL);
+      J[o + entry(w, d1)] += 1.0;
+      if (d2 >= 0) J[o + entry(w, d2)] -= dpoly;
+    }
+    // a factor entry that is not finite shows in the diagonal of its row
+    for (int k = 0; k < nv; k++) fits = fits && rfinite(LD(chol)[k * nv + k]);
+    isc[9] = nr;
+    isc[10] = fits && off < PGS_OFF_MAX && pgs_packed_doubles(nv, nr, off) <= cap ? 1 : 0;
+  });
+  if (!isc[10]) return -2;
+  const int nr = isc[9];
+  if (nr == 0) {
+    X::par(nv, [&](int k) { vpos[k] = v[k]; });
+    X::par(1, [&](int) { S.npcon[E.e] = 0; });
+    return 0;
+  }
+  // contact frames, once per contact, in the narrow phase's staging area
+  auto frame = S.stage + E.e * (int64_t)M.npair * MAXHIT * CW;
+  X::par(ncon, [&](int c) {
+    auto cc = con + c * CW;
+    V3 t1, t2;
+    contact_frame(cc, &t1, &t2);
+    st3(frame + c * 6, t1);
+    st3(frame + c * 6 + 3, t2);
+    const int g1 = cg[3 * c], g2 = cg[3 * c + 1];
+    const Real mu = rmax(M.v_friction[(int64_t)E.var * M.ngeom + g1], M.v_friction[(int64_t)E.var * M.ngeom + g2]);
+    const Real sep = -cc[9];
+    PgsRow w{};
+    span_of(c, &w);
+    for (int r = 0; r < 3; r++) {
+      Real* q = rw + (3 * c + r) * 10;
+      w.kind = r == 0 ? PK_NORMAL : PK_FRICTION;
+      w.sub = r;
+      w.off = coff[c] + (int64_t)r * w.count;
+      w.hard = 0;
+      q[PR_SEP] = sep;
+      q[PR_MU] = mu;
+      q[PR_INVA] = 0.0;
+      q[PR_LAM] = 0.0;
+      q[PR_KIND] = w.kind;
+      q[PR_NORMAL] = 3 * c;
+      q[PR_CONTACT] = c;
+      q[PR_B1] = r == 0 ? pgs_bias(C, PK_NORMAL, sep, &w.hard) : mu;
+      q[PR_FLAGS] = pgs_flags(w);
+    }
+  });
+  // contact rows (solver.rs:67-91), one lane per contact and dof of its blocks
+  X::par(ncon * M.pgs_w, [&](int t) {
+    const int c = t / M.pgs_w, l = t % M.pgs_w;
+    auto cc = con + c * CW;
+    const int b1 = M.geom_body[cg[3 * c]], b2 = M.geom_body[cg[3 * c + 1]];
+    PgsRow w{};
+    span_of(c, &w);
+    if (l >= w.count) return;
+    const int dof = w.dof(l);
+    const V3 p = ld3(cc);
+    const V3 dirs[3] = {ld3(cc + 3), ld3(frame + c * 6), ld3(frame + c * 6 + 3)};
+    const SP cd = ldsp(LD(cdof) + 6 * dof);
+    const bool on2 = (M.body_chain[b2] >> dof) & 1, on1 = (M.body_chain[b1] >> dof) & 1;
+    const V3 pv = point_velocity(cd, p);
+    for (int r = 0; r < 3; r++) {
+      Real jv = 0.0;
+      if (on2) jv += 1.0 * dot(dirs[r], pv);
+      if (on1) jv += -1.0 * dot(dirs[r], pv);
+      J[coff[c] + (int64_t)r * w.count + l] = jv;
+    }
+  });
+  if (M.pgs_b <= 6) pgs_packed_masses<6, X>(M, E, J, mj, rw, nr);
+  else pgs_packed_masses<16, X>(M, E, J, mj, rw, nr);
+  pgs_match_warm<X>(M, S, E, rw, ncon);
+  return nr;
+}
+
+// A row's new force from jv = J_r v, its force lam and its normal row's force
+// (solver.rs:175-207); b1 is the first phase's bias, for friction rows mu.
+PHD Real pgs_packed_force(const PgsConsts& C, bool use_bias, int kind, int hard, Real inv_a, Real b1, Real lam, Real lam_n,
+                           Real jv) {
+  if (kind == PK_FRICTION) {
+    const Real bound = b1 * lam_n;
+    return rclamp(lam - inv_a * jv, -bound, bound);
+  }
+  const bool soft = use_bias && !hard;
+  const Real bias = use_bias || hard ? b1 : 0.0;
+  const Real ms = soft ? C.mass_scale : 1.0, is = soft ? C.impulse_scale : 0.0;
+  if (kind == PK_NORMAL) {
+    const Real delta = -inv_a * ms * (jv + bias) - is * lam;
+    return rmax(lam + delta, 0.0);
+  }
+  return lam - inv_a * ms * (jv + bias) - is * lam;
+}
+
+// |dlambda_r| / inv_a_r >= tol (solver.rs:229-240), by a product where that
+// decides: for inv_a > 2^-900 the products are exact to 2^-52.
+PHD Real pgs_tol_hi(const PgsConsts& C) { return C.tol * (1.0 + 0x1p-40); }
+PHD Real pgs_tol_lo(const PgsConsts& C) { return C.tol * (1.0 - 0x1p-40); }
+PHD bool pgs_reaches_tol(const PgsConsts& C, Real t, Real inv_a) {
+  const bool normal = inv_a > 0x1p-900;
+  if (normal && t > inv_a * pgs_tol_hi(C)) return true;
+  if (normal && t < inv_a * pgs_tol_lo(C)) return false;
+  return t / inv_a >= C.tol;
+}
+
+// The dofs outside a row's blocks take 0 * x of a force change x that is not finite.
+template <class X, class VP>
+PHD void pgs_spread(const PgsRow& w, int nv, Real x, VP v) {
+  X::each([&](int l) {
+    if (l == 0)
+      for (int k = 0; k < nv; k++)
+        if (!(k >= w.a && k < w.a + w.na) && !(w.count > w.na && k >= w.b && k < w.b + w.count - w.na)) v[k] += 0.0 * x;
+  });
+  X::order();
+}
+
+// The row records in HBM, as the general sweeps read them.
+struct PgsRecs {
+  Real* p;
+  PHD Real inva(int r) const { return p[r * 10 + PR_INVA]; }
+  PHD Real b1(int r) const { return p[r * 10 + PR_B1]; }
+  PHD Real lam(int r) const { return p[r * 10 + PR_LAM]; }
+  PHD Real flags(int r) const { return p[r * 10 + PR_FLAGS]; }
+};
+
+// The warm start (solver.rs:155-161) over packed rows.
+template <class X, class JP, class VP>
+PHD void pgs_warm_rows(JP mj, PgsRecs rec, int nr, int nv, VP v) {
+  for (int r = 0; r < nr; r++) {
+    const Real lam = rec.lam(r);
+    if (lam == 0.0) continue;
+    const PgsRow w = pgs_row(rec.flags(r));
+    X::each([&](int l) {
+      if (l < w.count) v[w.dof(l)] += mj[w.off + l] * lam;
+    });
+    X::order();
+    if (!rfinite(lam)) pgs_spread<X>(w, nv, lam, v);
+  }
+}
+
+// The Gauss-Seidel sweeps over packed rows (solver.rs:149-245) on the 16 lanes
+// of one row, one lane per entry of the current row. keep_vpos() runs between
+// the two phases. The forces are left in the records. Takes up the sweeps at
+// row at.r of sweep at.it of phase at.phase: k_pgs_sweeps_rows hands over here
+// when a force or velocity is not finite.
+struct PgsAt {
+  int phase, it, r;
+  bool moved;  // some row of this sweep changed a velocity by at least the tolerance
+};
+PHD int pgs_relax_sweeps(const PgsConsts& C) { return C.iterations / 3 > 2 ? C.iterations / 3 : 2; }
+template <class X, int W, class JP, class VP, class F>
+PHD void pgs_sweeps_rows(const PgsConsts& C, JP J, JP mj, PgsRecs rec, int nr, int nv, VP v, PgsAt at, F&& keep_vpos) {
+  using LV = typename X::LV;
+  // every velocity and force is finite (once one is not, it never is again)
+  bool vfin = true;
+  for (int k = 0; k < nv; k++) vfin = vfin && rfinite(v[k]);
+  for (int r = 0; r < nr; r++) vfin = vfin && rfinite(rec.lam(r));
+  // what a row needs that no earlier row changes, loaded one row ahead
+  struct Ahead {
+    Real inv_a, b1, lam;
+    PgsRow w;
+    LV j, m;
+  };
+  auto fetch = [&](int r) {
+    Ahead n;
+    n.inv_a = rec.inva(r);
+    n.b1 = rec.b1(r);
+    n.lam = rec.lam(r);
+    n.w = pgs_row(rec.flags(r));
+    n.j = X::gen([&](int l) { return l < n.w.count ? J[n.w.off + l] : 0.0; });
+    n.m = X::gen([&](int l) { return l < n.w.count ? mj[n.w.off + l] : 0.0; });
+    return n;
+  };
+  auto sweep = [&](bool use_bias, int r0, bool moved) {
+    Ahead next = fetch(r0 < nr ? r0 : 0);
+    for (int r = r0; r < nr; r++) {
+      const Ahead q = next;
+      const PgsRow& w = q.w;
+      const LV vv = X::gen([&](int l) { return v[l < w.count ? w.dof(l) : w.a]; });
+      const Real lam_n = rec.lam(r - w.sub);
+      next = fetch(r + 1 < nr ? r + 1 : r);
+      const Real inv_a = q.inv_a, lam = q.lam;
+      if (inv_a == 0.0) continue;
+      const LV p = X::sel([&](int l) { return l < w.count; }, q.j * vv, X::splat(0.0));
+      Real jv = X::template rowsum<W>(p, rsum0());
+      if (!vfin)  // 0 * v of the dofs outside the row's blocks
+        for (int k = 0; k < nv; k++)
+          if (!(k >= w.a && k < w.a + w.na) && !(w.count > w.na && k >= w.b && k < w.b + w.count - w.na)) jv += 0.0 * v[k];
+      const Real nw = pgs_packed_force(C, use_bias, w.kind, w.hard, inv_a, q.b1, lam, lam_n, jv);
+      const Real dl = nw - lam;
+      if (dl != 0.0) {
+        const LV vn = vv + q.m * dl;
+        X::each([&](int l) {
+          if (l < w.count) v[w.dof(l)] = X::at(vn, l);
+          if (l == 0) rec.p[r * 10 + PR_LAM] = nw;
+        });
+        X::order();
+        moved = moved || pgs_reaches_tol(C, fabs(dl), inv_a);
+        if (X::ballot([&](int l) { return l < w.count && !rfinite(X::at(vn, l)); })) vfin = false;
+        if (!rfinite(dl)) {
+          pgs_spread<X>(w, nv, dl, v);
+          vfin = false;
+        }
+      }
+    }
+    return moved;
+  };
+  for (int phase = at.phase; phase < 2; phase++) {
+    const int limit = phase == 0 ? C.iterations : pgs_relax_sweeps(C);
+    for (int it = at.it; it < limit; it++) {
+      const bool moved = sweep(phase == 0, at.r, at.moved);
+      at.r = 0;
+      at.moved = false;
+      if (!moved) break;
+    }
+    at.it = 0;
+    if (phase == 0) keep_vpos();
+  }
+}
+
 template <class X, class MT>
 PHD void pgs_solve(const MT& M, const DState& S, Env& E, Real* v, Real* vpos) {
   const int nr = pgs_prepare<X>(M, S, E, v, vpos);
   if (nr <= 0) return;
   pgs_sweeps<X>(M, S, E, nr, v, vpos);
-  pgs_finish<X>(M, S, E, nr);
+  pgs_finish<X>(M, S, E);
 }
 
 // ---------------- integrate_pos, forward.rs:459-480 ----------------
@@ -2080,11 +2545,12 @@ PHD void pgs_step_end(const MT& M, Env& E) {
 // PGS branch has completed the step. With pgs_stop the PGS branch stops
 // early and returns the row count: PGS_BEFORE_SWEEPS with the warm start
 // applied (velocity in LD(vel); with no rows the step's velocities are final
-// and LD(acc) holds vpos), PGS_BEFORE_WARM with the warm-start forces still in
+// and LD(acc) holds vpos) or, when the env's rows fit pgs_cap doubles, with
+// packed rows whose sweeps apply the warm start (PR_MODE of the first row), PGS_BEFORE_WARM with the warm-start forces still in
 // the row records.
 enum { PGS_FULL = 0, PGS_BEFORE_SWEEPS = 1, PGS_BEFORE_WARM = 2 };
 template <class X, class MT>
-PHD int step_front(const MT& M, const DState& S, Env& E, int pgs_stop = PGS_FULL) {
+PHD int step_front(const MT& M, const DState& S, Env& E, int pgs_stop = PGS_FULL, int64_t pgs_cap = 0) {
   const int nv = M.nv;
   const Real h = M.timestep;
   int* isc = E.si + M.L.i_iscal;
@@ -2115,8 +2581,15 @@ PHD int step_front(const MT& M, const DState& S, Env& E, int pgs_stop = PGS_FULL
     Real* vel = LD(vel);
     Real* vpos = LD(acc);
     X::par(nv, [&](int k) { vel[k] = LD(qvel)[k] + h * a[k]; });
+    if (pgs_stop == PGS_BEFORE_SWEEPS && pgs_cap > 0) {
+      const int nr = pgs_prepare_packed<X>(M, S, E, vel, vpos, pgs_cap);
+      const bool packed = nr != -2;
+      if (nr > 0) X::par(1, [&](int) { (S.grow + E.e * (int64_t)M.nrmax * 10)[PR_MODE] = 1.0; });
+      if (packed) return nr;
+    }
     if (pgs_stop != PGS_FULL) {
       const int nr = pgs_prepare<X>(M, S, E, vel, vpos, pgs_stop == PGS_BEFORE_SWEEPS);
+      if (nr > 0) X::par(1, [&](int) { (S.grow + E.e * (int64_t)M.nrmax * 10)[PR_MODE] = 0.0; });
       return nr < 0 ? STEP_FAILED : nr;
     }
     pgs_solve<X>(M, S, E, vel, vpos);
@@ -2337,7 +2810,7 @@ PHD void run_env(const MT& M, const DState& S, Env& E, int64_t nstep, const Real
 // the three give run_env's results bit for bit.
 template <class X, class MT>
 PHD void run_pgs_front(const MT& M, const DState& S, Env& E, int64_t nstep, int64_t t, const Real* ctrl_seq,
-                       int64_t rel, Real* vel_g, Real* vpos_g) {
+                       int64_t rel, Real* vel_g, Real* vpos_g, int64_t cap) {
   Real* lds = E.s;
   load_state<X>(M, S, E);
   int* isc = E.si + M.L.i_iscal;
@@ -2347,7 +2820,7 @@ PHD void run_pgs_front(const MT& M, const DState& S, Env& E, int64_t nstep, int6
     X::par(M.nu, [&](int k) { lds[M.L.ctrl + k] = ctrl_seq[(rel * nstep + t) * M.nu + k]; });
     X::par(M.nu, [&](int k) { S.ctrl[e * M.nu + k] = lds[M.L.ctrl + k]; });
   }
-  const int nr = step_front<X>(M, S, E, PGS_BEFORE_SWEEPS);
+  const int nr = step_front<X>(M, S, E, PGS_BEFORE_SWEEPS, cap);
   X::par(M.nv, [&](int k) {
     vel_g[k] = LD(vel)[k];
     vpos_g[k] = LD(acc)[k];
@@ -2377,8 +2850,7 @@ PHD void run_pgs_back(const MT& M, const DState& S, Env& E, int64_t nstep, int64
       vpos[k] = vpos_g[k];
     });
     X::par(1, [&](int) { isc[IS_NCON] = S.ncon[e]; });
-    const int nr = S.nrows[e];
-    if (nr > 0) pgs_finish<X>(M, S, E, nr);
+    if (S.nrows[e] > 0) pgs_finish<X>(M, S, E);
     X::par(M.nv, [&](int k) { LD(qacc)[k] = (vel[k] - LD(qvel)[k]) / h; });
     integrate_pos<X>(M, E, vpos, h);
     X::par(M.nv, [&](int k) { LD(qvel)[k] = vel[k]; });
@@ -2649,7 +3121,7 @@ PHD void run_env_mlp(const MT& M, const DState& S, Env& E, int64_t nstep, const 
         if (code > 0) {
           pgs_apply_warm<X>(M, S, E, code, vel);
           sweeps = pgs_sweeps<X>(M, S, E, code, vel, vpos);
-          pgs_finish<X>(M, S, E, code);
+          pgs_finish<X>(M, S, E);
           if (M.mlp.mode & MLP_LOG) mlp_targets_pgs<X>(M, S, E);
         }
         pgs_step_end<X>(M, E);

@@ -21,6 +21,9 @@ struct DevXK : DevLanes {
     __syncthreads();
   }
   __device__ __forceinline__ static void sync() { __syncthreads(); }
+  // 16-lane rows that work on one env, and which of them this lane is in
+  static constexpr int ROWS = G / GL;
+  __device__ __forceinline__ static int row() { return (int)(threadIdx.x % G) / GL; }
 };
 using DevX = DevXK<1>;
 
@@ -126,55 +129,311 @@ __global__ void __launch_bounds__(64) k_step_ws(const DModel* __restrict__ Mp, c
 }
 
 // The PGS step split around its sweeps (run_pgs_front, run_pgs_back in
-// kbody.hpp), one env per workgroup of one wavefront, for physics step t of
-// nstep (K = 1): the front and back keep the step kernel's LDS working set; the sweeps
-// kernel needs no LDS and few registers, so many of its wavefronts share a SIMD
-// and hide each other's dependent chains. vel and vpos hold nv doubles per env
-// (indexed by env id).
+// kbody.hpp), for physics step t of nstep: the front and back keep the step
+// kernel's LDS working set, K envs per workgroup of one wavefront; the sweeps
+// run in kernels of their own. vel and vpos hold nv doubles per env (indexed by
+// env id); cap: the doubles that packed rows of one env may take
+// (k_pgs_sweeps_rows), 0 for a model without packed rows.
 template <int K>
 __global__ void __launch_bounds__(64) k_pgs_front(const DModel* __restrict__ Mp, const DState* __restrict__ Sp,
                                                   int64_t begin, int64_t end, int64_t nstep, int64_t t,
-                                                  const Real* ctrl_seq, Real* vel, Real* vpos) {
+                                                  const Real* ctrl_seq, Real* vel, Real* vpos, int64_t cap,
+                                                  unsigned* counter) {
   const DModel& M = *Mp;
   const DState& S = *Sp;
   extern __shared__ double lds[];
-  const int64_t rel = (int64_t)blockIdx.x;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *counter = 0;  // for the sweeps that follow
+  const int g = (int)threadIdx.x / DevXK<K>::G;
+  const int64_t rel = (int64_t)blockIdx.x * K + g;
   if (begin + rel >= end) return;
   Env E;
-  E.s = lds;
+  E.s = lds + (int64_t)g * (M.L.bytes / 8);
   E.si = reinterpret_cast<int*>(E.s + M.L.ndouble);
   E.e = begin + rel;
   E.var = M.env_var[E.e];
-  static_assert(K == 1, "one env per workgroup");
-  run_pgs_front<DevXK<1>>(M, S, E, nstep, t, ctrl_seq, rel, vel + E.e * M.nv, vpos + E.e * M.nv);
+  run_pgs_front<DevXK<K>>(M, S, E, nstep, t, ctrl_seq, rel, vel + E.e * M.nv, vpos + E.e * M.nv, cap);
 }
 
+// The rest of an env's sweeps in their general form, from its row `at` on:
+// velocities in LDS, rows and forces in HBM (lam: the forces so far). Out of
+// line: hardly any env comes here.
+template <int W>
+__device__ __noinline__ void pgs_sweeps_general(const DModel* Mp, const DState* Sp, int64_t e, int nr, double* v,
+                                                int64_t phase_it, int64_t row_moved, Real* vpos_e) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  using X = DevXK<4>;
+  const DModel& M = *Mp;
+  const DState& S = *Sp;
+  const int nv = M.nv, l = (int)threadIdx.x % GL;
+  const PgsAt at{(int)(phase_it >> 32), (int)(uint32_t)phase_it, (int)(row_moved >> 1), (row_moved & 1) != 0};
+  Real* J = (S.gjac + e * (int64_t)M.nrmax * nv).p;
+  Real* mj = (S.gmj + e * (int64_t)M.nrmax * nv).p;
+  const PgsRecs rec{(S.grow + e * (int64_t)M.nrmax * 10).p};
+  __threadfence_block();
+  pgs_sweeps_rows<X, W>(pgs_consts(M), J, mj, rec, nr, nv, v, at, [&]() {
+    for (int k = l; k < nv; k += GL) vpos_e[k] = v[k];
+  });
+#endif
+}
+
+// The sweeps over packed rows: four envs per wavefront, one per 16-lane row,
+// with the env's rows, forces and velocities in LDS (slice doubles per env), W
+// the widest row's entries. A row update is a chain (read v, W ordered adds,
+// the force, write v) of about 90 instructions that the four envs share; LDS
+// holds 12 envs per CU, so less than one wavefront per SIMD hides nothing of it
+// and every instruction and branch counts: the terms that stay fixed over a
+// phase are formed when the phase begins, normal and friction rows share one
+// expression (a friction row's bias and impulse scale are 0, a normal row's
+// friction coefficient 0 and its upper bound infinite), the next row's entries
+// and the record after it are in flight during an update. The four 16-lane
+// rows advance independently, each from row to row, sweep to sweep and env to
+// env (counter, cleared by k_pgs_front), so none waits for another's longer
+// solve. The expression needs finite velocities and forces; an env that has
+// others goes on in pgs_sweeps_general. EQ: the model has equalities, whose
+// rows are bilateral.
+template <int W, bool EQ>
+__global__ void __launch_bounds__(64) k_pgs_sweeps_rows(const DModel* __restrict__ Mp, const DState* __restrict__ Sp,
+                                                        int64_t begin, int64_t end, Real* vel, Real* vpos, int slice,
+                                                        unsigned* counter) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  using X = DevXK<4>;
+  const DModel& M = *Mp;
+  const DState& S = *Sp;
+  extern __shared__ double lds[];
+  // LDS by byte address (below 64 KiB)
+  typedef __attribute__((address_space(3))) char LC;
+  typedef __attribute__((address_space(3))) double LDd;
+  LC* const lb = (LC*)lds;
+  auto ld = [&](int a) -> double { return *(LDd*)(lb + a); };
+  auto st = [&](int a, double x) { *(LDd*)(lb + a) = x; };
+  const int g = (int)threadIdx.x / GL, l = (int)threadIdx.x % GL, l8 = 8 * l;
+  const int nv = M.nv, vb = 8 * g * slice, spare = vb + 8 * nv, recb = vb + 8 * ((nv + 2) & ~1);
+  constexpr int RB = 8 * PGS_REC;
+  // a row's record: -inv_a times the mass scale, bias, impulse scale, friction
+  // coefficient, force, and where its entries and velocities are
+  enum { C0 = 0, BIAS = 8, IS = 16, MU = 24, LAM = 32, INFO = 40 };
+  const PgsConsts C = pgs_consts(M);
+  const int relax = pgs_relax_sweeps(C);
+  const Real hi0 = pgs_tol_hi(C), lo0 = pgs_tol_lo(C), hi1 = hi0 / C.mass_scale, lo1 = lo0 / C.mass_scale;
+  const int64_t n = end - begin;
+  bool live = true, have = false;
+  int64_t e = 0;
+  int nr = 0, Jb = 0, mo = 0;  // byte address of the J entries, and from there to the M^-1 J^T entries
+  int phase = 0, it = 0, r = 0, limit = 0;
+  bool moved = false;
+  Real c0 = 0.0, bias = 0.0, is = 0.0, mu = 0.0, lam = 0.0, j = 0.0, m = 0.0;  // the current row
+  Real nc0 = 0.0, nbias = 0.0, nis = 0.0, nmu = 0.0;                          // the next one
+  int lo_w = 0, hi_w = 0, nlo = 0, nhi = 0;                                    // their INFO words
+  int va = spare;
+  auto after = [&](int i) { return i + 1 < nr ? i + 1 : 0; };
+  auto count_of = [](int hi) { return (hi >> 21) & 31; };
+  auto v_addr = [&](int lo, int hi) {  // this lane's velocity; a spare slot past the row's entries
+    const int base = l < ((hi >> 16) & 31) ? lo & 0xFFFF : (int)((unsigned)lo >> 16);
+    return l < count_of(hi) ? base + l8 : spare;
+  };
+  auto info = [&](int i, int* lo, int* hi) {
+    const int64_t w = *(__attribute__((address_space(3))) int64_t*)(lb + recb + i * RB + INFO);
+    *lo = (int)w;
+    *hi = (int)(w >> 32);
+  };
+  auto start = [&](int i) {  // fill the pipeline at row i
+    int a = recb + i * RB;
+    c0 = ld(a + C0), bias = ld(a + BIAS), is = ld(a + IS), mu = ld(a + MU), lam = ld(a + LAM);
+    info(i, &lo_w, &hi_w);
+    va = v_addr(lo_w, hi_w);
+    const bool in = l < count_of(hi_w);
+    j = ld(Jb + (hi_w & 0xFFFF) * 8 + l8);
+    m = ld(Jb + mo + (hi_w & 0xFFFF) * 8 + l8);
+    j = in ? j : 0.0;
+    m = in ? m : 0.0;
+    a = recb + after(i) * RB;
+    nc0 = ld(a + C0), nbias = ld(a + BIAS), nis = ld(a + IS), nmu = ld(a + MU);
+    info(after(i), &nlo, &nhi);
+  };
+  auto records = [&](int ph) {  // the rows' terms in phase ph
+    auto rw = S.grow + e * (int64_t)M.nrmax * 10;
+    for (int i = l; i < nr; i += GL) {
+      const PgsRow w = pgs_row(rw[i * 10 + PR_FLAGS]);
+      const Real ia = rw[i * 10 + PR_INVA], b1 = rw[i * 10 + PR_B1];
+      const bool friction = w.kind == PK_FRICTION, soft = ph == 0 && !w.hard && !friction, fixed = ia == 0.0;
+      const int a = recb + i * RB;
+      st(a + C0, soft ? -ia * C.mass_scale : -ia);
+      st(a + BIAS, !friction && (ph == 0 || w.hard) ? b1 : 0.0);
+      st(a + IS, soft && !fixed ? C.impulse_scale : 0.0);
+      st(a + MU, friction && !fixed ? b1 : 0.0);
+      // lo: addresses of entry 0 of the lower block and of entry na of the
+      // upper one less its place; hi: offset 16, na 5, entries 5, sub 2,
+      // bilateral 1, unbounded above 1 (sign)
+      const unsigned alo = (unsigned)(vb + 8 * w.a), blo = (unsigned)(vb + 8 * (w.count > w.na ? w.b - w.na : 0));
+      const unsigned hi = (unsigned)w.off | (unsigned)w.na << 16 | (unsigned)w.count << 21 | (unsigned)w.sub << 26 |
+                          (w.kind == PK_BILATERAL ? 1u << 28 : 0u) | (!friction || fixed ? 1u << 31 : 0u);
+      *(__attribute__((address_space(3))) int64_t*)(lb + a + INFO) = (int64_t)((uint64_t)hi << 32 | blo << 16 | alo);
+    }
+    X::order();
+  };
+  auto store = [&](bool forces) {
+    for (int k = l; k < nv; k += GL) vel[e * nv + k] = ld(vb + 8 * k);
+    auto rw = S.grow + e * (int64_t)M.nrmax * 10;
+    if (forces)
+      for (int i = l; i < nr; i += GL) rw[i * 10 + PR_LAM] = ld(recb + i * RB + LAM);
+    have = false;
+  };
+  auto general = [&](int row) {  // the rest of this env's sweeps
+    auto rw = S.grow + e * (int64_t)M.nrmax * 10;
+    for (int i = l; i < nr; i += GL) rw[i * 10 + PR_LAM] = ld(recb + i * RB + LAM);
+    pgs_sweeps_general<W>(Mp, Sp, e, nr, lds + (int64_t)g * slice, (int64_t)phase << 32 | it,
+                          (int64_t)row << 1 | (moved ? 1 : 0), vpos + e * nv);
+    store(false);
+  };
+  for (;;) {
+    while (live && !have) {
+      unsigned idx = 0;
+      if (l == 0) idx = atomicAdd(counter, 1u);
+      idx = __shfl(idx, g * GL);
+      if ((int64_t)idx >= n) {
+        live = false;
+        break;
+      }
+      e = begin + idx;
+      nr = S.nrows[e];
+      if (S.status[e] != 0 || nr <= 0) continue;
+      auto rw = S.grow + e * (int64_t)M.nrmax * 10;
+      if (rw[PR_MODE] == 0.0) continue;
+      const PgsRow last = pgs_row(rw[(nr - 1) * 10 + PR_FLAGS]);
+      const int entries = (int)last.off + last.count;
+      Jb = recb + nr * RB;
+      mo = 8 * entries;
+      auto gj = S.gjac + e * (int64_t)M.nrmax * nv;
+      auto gm = S.gmj + e * (int64_t)M.nrmax * nv;
+      bool ok = C.iterations > 0;
+      for (int k = l; k < nv; k += GL) st(vb + 8 * k, vel[e * nv + k]);
+      for (int i = l; i < nr; i += GL) {
+        const Real ia = rw[i * 10 + PR_INVA], lm = rw[i * 10 + PR_LAM];
+        st(recb + i * RB + LAM, lm);
+        ok = ok && rfinite(lm) && (ia > 0x1p-900 || (ia == 0.0 && lm == 0.0));
+      }
+      for (int t = l; t < entries; t += GL) {
+        st(Jb + 8 * t, gj[t]);
+        st(Jb + mo + 8 * t, gm[t]);
+      }
+      st(spare, 0.0);
+      st(Jb + 2 * mo + l8, 0.0);
+      X::order();
+      have = true;
+      double* v = lds + (int64_t)g * slice;
+      pgs_warm_rows<X>(v + (Jb + mo - vb) / 8, PgsRecs{rw.p}, nr, nv, v);
+      for (int k = l; k < nv; k += GL) ok = ok && rfinite(ld(vb + 8 * k));
+      phase = it = r = 0;
+      moved = false;
+      limit = C.iterations;
+      if (X::ballot([&](int) { return !ok; })) {
+        general(0);
+        continue;
+      }
+      records(0);
+      start(0);
+    }
+    if (__ballot(live) == 0) break;
+    if (live) {
+      const int rn = after(r), rnn = after(rn);
+      const Real vv = ld(va);
+      const Real lam_n = ld(recb + (r - ((hi_w >> 26) & 3)) * RB + LAM);
+      // the next row's entries, and the record of the one after
+      const int off = (nhi & 0xFFFF) * 8 + l8, a2 = recb + rnn * RB;
+      Real nj = ld(Jb + off), nm = ld(Jb + mo + off);
+      const Real xc0 = ld(a2 + C0), xbias = ld(a2 + BIAS), xis = ld(a2 + IS), xmu = ld(a2 + MU);
+      int xlo, xhi;
+      info(rnn, &xlo, &xhi);
+      const int nva = v_addr(nlo, nhi);
+      const Real jv = X::template rowsum<W>(DLV{j * vv}, rsum0());
+      const Real t = c0 * (jv + bias), il = is * lam, b = mu * lam_n;
+      Real y = lam + (t - il);
+      const Real hi = hi_w < 0 ? INFINITY : b;
+      Real nw = rmin(rmax(y, -b), hi);
+      if constexpr (EQ) {
+        y = (lam + t) - il;
+        nw = (hi_w >> 28) & 1 ? y : nw;
+      }
+      const Real dl = nw - lam, vn = vv + m * dl, size = fabs(dl), ac = fabs(c0);
+      // |dl| against inv_a tol, from c0 = -inv_a or -inv_a mass_scale
+      const bool above = size > ac * (is != 0.0 ? hi1 : hi0), below = size < ac * (is != 0.0 ? lo1 : lo0);
+      const bool odd = !rfinite(vn) || !rfinite(jv);
+      if (__ballot(odd || (!above && !below && dl != 0.0)) == 0) {
+        moved = moved || above;
+        st(va, vn);
+        st(recb + r * RB + LAM, nw);
+      } else if (X::ballot([&](int) { return odd; })) {
+        general(r);  // this row and the rest
+        continue;
+      } else {
+        if (!above && !below && dl != 0.0) {
+          const Real ia = S.grow[e * (int64_t)M.nrmax * 10 + (int64_t)r * 10 + PR_INVA];
+          moved = moved || pgs_reaches_tol(C, size, ia);
+        }
+        moved = moved || above;
+        st(va, vn);
+        st(recb + r * RB + LAM, nw);
+      }
+      X::order();
+      const bool in = l < count_of(nhi);
+      lam = ld(recb + rn * RB + LAM);
+      c0 = nc0, bias = nbias, is = nis, mu = nmu, lo_w = nlo, hi_w = nhi, va = nva;
+      j = in ? nj : 0.0;
+      m = in ? nm : 0.0;
+      nc0 = xc0, nbias = xbias, nis = xis, nmu = xmu, nlo = xlo, nhi = xhi;
+      r = rn;
+      if (rn == 0) {  // the sweep's end
+        it++;
+        if (!moved || it >= limit) {
+          if (phase == 0) {
+            for (int k = l; k < nv; k += GL) vpos[e * nv + k] = ld(vb + 8 * k);
+            phase = 1;
+            it = 0;
+            limit = relax;
+            records(1);
+            start(0);
+          } else {
+            store(true);
+          }
+        }
+        moved = false;
+      }
+    }
+  }
+#endif
+}
+
+// The sweeps over rows that are not packed (a row over 16 dofs, more rows than
+// k_pgs_sweeps_rows holds, a factor that is not finite): one env per wavefront
+// at a time, no LDS and few registers, so that many wavefronts share a SIMD and
+// hide each other's dependent chains.
 template <int K>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) k_pgs_sweeps(const DModel* __restrict__ Mp, const DState* __restrict__ Sp,
                                                    int64_t begin, int64_t end, Real* vel, Real* vpos) {
 #if defined(__HIP_DEVICE_COMPILE__)
   const DModel& M = *Mp;
   const DState& S = *Sp;
-  const int64_t e = begin + (int64_t)blockIdx.x;
-  if (e >= end || S.status[e] != 0) return;
-  const int nr = S.nrows[e];
-  if (nr <= 0) return;
   const int nv = M.nv;
-  Real* J = (S.gjac + e * (int64_t)M.nrmax * nv).p;
-  Real* mj = (S.gmj + e * (int64_t)M.nrmax * nv).p;
-  Real* rw = (S.grow + e * (int64_t)M.nrmax * 10).p;
-  Real* v = vel + e * nv;
-  Real* vp = vpos + e * nv;
   const PgsConsts C = pgs_consts(M);
-  if (nr <= PGS_WAVE_ROWS) {
-    const int lane = (int)threadIdx.x;
-    const LaneVel r = pgs_sweeps_body(C, J, mj, rw, nr, nv, lane < nv ? v[lane] : 0.0);
-    if (lane < nv) {
-      v[lane] = r.v;
-      vp[lane] = r.vpos;
+  for (int64_t e = begin + (int64_t)blockIdx.x; e < end; e += gridDim.x) {
+    const int nr = S.nrows[e];
+    if (S.status[e] != 0 || nr <= 0) continue;
+    Real* rw = (S.grow + e * (int64_t)M.nrmax * 10).p;
+    if ((S.grow + e * (int64_t)M.nrmax * 10)[PR_MODE] != 0.0) continue;
+    Real* J = (S.gjac + e * (int64_t)M.nrmax * nv).p;
+    Real* mj = (S.gmj + e * (int64_t)M.nrmax * nv).p;
+    Real* v = vel + e * nv;
+    Real* vp = vpos + e * nv;
+    if (nr <= PGS_WAVE_ROWS) {
+      const int lane = (int)threadIdx.x;
+      const LaneVel r = pgs_sweeps_body(C, J, mj, rw, nr, nv, lane < nv ? v[lane] : 0.0);
+      if (lane < nv) {
+        v[lane] = r.v;
+        vp[lane] = r.vpos;
+      }
+    } else if (threadIdx.x == 0) {
+      pgs_sweeps_serial(C, J, mj, rw, nr, nv, v, vp);
     }
-  } else if (threadIdx.x == 0) {
-    pgs_sweeps_serial(C, J, mj, rw, nr, nv, v, vp);
   }
 #endif
 }
@@ -186,15 +445,15 @@ __global__ void __launch_bounds__(64) k_pgs_back(const DModel* __restrict__ Mp, 
   const DModel& M = *Mp;
   const DState& S = *Sp;
   extern __shared__ double lds[];
-  const int64_t rel = (int64_t)blockIdx.x;
+  const int g = (int)threadIdx.x / DevXK<K>::G;
+  const int64_t rel = (int64_t)blockIdx.x * K + g;
   if (begin + rel >= end) return;
   Env E;
-  E.s = lds;
+  E.s = lds + (int64_t)g * (M.L.bytes / 8);
   E.si = reinterpret_cast<int*>(E.s + M.L.ndouble);
   E.e = begin + rel;
   E.var = M.env_var[E.e];
-  static_assert(K == 1, "one env per workgroup");
-  run_pgs_back<DevXK<1>>(M, S, E, nstep, t, qpos_out, rel, vel + E.e * M.nv, vpos + E.e * M.nv);
+  run_pgs_back<DevXK<K>>(M, S, E, nstep, t, qpos_out, rel, vel + E.e * M.nv, vpos + E.e * M.nv);
 }
 
 // Contact-count bucketing for k_step_ws, one workgroup: envs [begin, end)

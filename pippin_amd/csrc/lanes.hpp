@@ -79,6 +79,42 @@ struct DevLanes {
     uint64_t m = __ballot(pred(lane()) ? 1 : 0);
     return (uint32_t)((m >> (threadIdx.x & 48u)) & 0xFFFFu);
   }
+  // start + x of lane 0 + x of lane 1 + ... + x of lane N - 1 of this lane's
+  // 16-lane row, added in that order, in every lane. One v_fmac_f64 per term
+  // with the DPP broadcast as its operand: fma(x, 1, s) rounds x + s once, as
+  // the addition does. A broadcast (v_mov_b64_dpp) and an addition per term
+  // would be twice the instructions. The two wait states that a DPP read of a
+  // freshly written register needs are in the block, since the compiler does
+  // not see into it.
+  template <int N>
+  __device__ __forceinline__ static Real rowsum(DLV x, Real start) {
+    Real s = start;
+    const Real one = 1.0;
+#define PH_ROWSUM(k) "v_fmac_f64_dpp %0, %1, %2 row_newbcast:" #k " row_mask:0xf bank_mask:0xf\n\t"
+    if constexpr (N == 6) {
+      asm("s_nop 1\n\t" PH_ROWSUM(0) PH_ROWSUM(1) PH_ROWSUM(2) PH_ROWSUM(3) PH_ROWSUM(4) PH_ROWSUM(5)
+          : "+&v"(s) : "v"(x.v), "v"(one));
+    } else if constexpr (N == 12) {
+      asm("s_nop 1\n\t" PH_ROWSUM(0) PH_ROWSUM(1) PH_ROWSUM(2) PH_ROWSUM(3) PH_ROWSUM(4) PH_ROWSUM(5)
+          PH_ROWSUM(6) PH_ROWSUM(7) PH_ROWSUM(8) PH_ROWSUM(9) PH_ROWSUM(10) PH_ROWSUM(11)
+          : "+&v"(s) : "v"(x.v), "v"(one));
+    } else {
+      static_assert(N == GL, "row sums of 6, 12 or 16 lanes");
+      asm("s_nop 1\n\t" PH_ROWSUM(0) PH_ROWSUM(1) PH_ROWSUM(2) PH_ROWSUM(3) PH_ROWSUM(4) PH_ROWSUM(5)
+          PH_ROWSUM(6) PH_ROWSUM(7) PH_ROWSUM(8) PH_ROWSUM(9) PH_ROWSUM(10) PH_ROWSUM(11)
+          PH_ROWSUM(12) PH_ROWSUM(13) PH_ROWSUM(14) PH_ROWSUM(15)
+          : "+&v"(s) : "v"(x.v), "v"(one));
+    }
+#undef PH_ROWSUM
+    return s;
+  }
+  // LDS writes of this wavefront's lanes before this point are seen by its
+  // reads after it (LDS serves a wavefront's operations in order, so this only
+  // keeps the compiler from moving them)
+  __device__ __forceinline__ static void order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
   // lane J's value in every lane of this lane's 16-lane row: one 64-bit DPP
   // move (v_mov_b64_dpp row_newbcast:J; every source lane is valid)
   template <int J>
@@ -165,6 +201,17 @@ struct HostLanes {
     return r;
   }
   static Real uni(const HLV& a) { return a.v[0]; }
+  template <int N>
+  static Real rowsum(const HLV& x, Real start) {
+    Real s = start;
+    for (int l = 0; l < N; l++) s = s + x.v[l];
+    return s;
+  }
+  static void order() {}
+  // 16-lane rows that work on one env, and this lane's (the device policies
+  // own 4, 2 or 1 by their envs per wavefront)
+  static constexpr int ROWS = 1;
+  static int row() { return 0; }
   template <class P>
   static uint32_t ballot(P&& pred) {
     uint32_t m = 0;

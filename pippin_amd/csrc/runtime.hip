@@ -203,6 +203,13 @@ struct DBuf {
   hipError_t zero() { return hipMemset(p, 0, (n ? n : 1) * sizeof(T)); }
 };
 
+// The packed PGS sweeps for a model's widest row and with or without equalities.
+static const void* pgs_rows_kernel(const DModel& M) {
+  if (M.neq > 0)
+    return M.pgs_w <= 12 ? (const void*)k_pgs_sweeps_rows<12, true> : (const void*)k_pgs_sweeps_rows<16, true>;
+  return M.pgs_w <= 12 ? (const void*)k_pgs_sweeps_rows<12, false> : (const void*)k_pgs_sweeps_rows<16, false>;
+}
+
 struct Variants {
   // host mirrors, [nvar][...]
   std::vector<double> geom_size, geom_aabb, friction, body_mass, body_ipos, body_inertia, dof_damping, act_gain,
@@ -229,6 +236,8 @@ struct ph_sim {
   int spec = 0;         // 1: the model matches SpecAnt (compile-time sizes and layout)
   int sched = PH_SCHED_GRID;  // schedule of the plain step (PH_SCHED_*)
   int cus = 0;                // compute units of the device
+  int pgs_per_cu = 0;         // wavefronts of the packed PGS sweeps that a CU holds
+  int pgs_slice = 0;          // LDS doubles per env of the packed PGS sweeps (0: no packed rows)
   int ws_per_cu[3][2] = {};   // resident work-stealing workgroups per CU, by K = 1, 2, 4 and kernel instance
   std::string arch;           // device architecture name (autotune cache key)
   // work-stealing schedule: env order (offsets from the range start) and slot counter
@@ -461,6 +470,18 @@ extern "C" int pippin_hip_create(const ph_model_desc* desc, int64_t num_envs, co
     }
   HIPCHK(s->d_order.alloc(std::max<int64_t>(num_envs, 1)));
   if (M.solver_kind == 1) {
+    // Packed sweeps: the LDS of an env is what its rows can need, up to a
+    // third of a CU's over the four envs of a wavefront.
+    if (M.pgs_w > 0) {
+      const int64_t rows = 3 * (int64_t)M.ncmax + 2 * hm.nlimited + d.neq;
+      const int64_t most = pgs_packed_doubles(M.nv, rows, rows * M.pgs_w);
+      const int64_t third = (160 * 1024 / 3 - 512) / 4 / 8;  // 512: the allocation's granularity
+      s->pgs_slice = (int)(std::min(most + 1, third) & ~(int64_t)1);
+      const void* k = pgs_rows_kernel(M);
+      const int bytes = 4 * s->pgs_slice * 8;
+      HIPCHK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+      HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&s->pgs_per_cu, k, 64, (size_t)bytes));
+    }
     HIPCHK(s->d_pgs_vel.alloc((size_t)std::max<int64_t>(num_envs * M.nv, 1)));
     HIPCHK(s->d_pgs_vpos.alloc((size_t)std::max<int64_t>(num_envs * M.nv, 1)));
   }
@@ -689,6 +710,28 @@ static unsigned ws_grid(const ph_sim* s, int K, int spec, int64_t nslots) {
   return (unsigned)std::min<int64_t>((int64_t)per_cu * s->cus, nslots);
 }
 
+// Envs per wavefront of the split PGS step's front and back. A round of
+// wavefronts takes about 1 : 1.2 : 1.5 for 1, 2 and 4 envs (the generic Ant
+// kernel: 344, 410 and 520 us per 4-step round), so the fewest rounds win
+// once the device is full, and one env per wavefront while it is not.
+static int split_envs_per_wave(const ph_sim* s, int64_t envs) {
+  const double weight[] = {1.0, 1.2, 1.5};
+  int best = 1;
+  double cost = 0.0;
+  for (int i = 0; i < 3; i++) {
+    const int K = 1 << i;
+    const int64_t lds = (int64_t)K * s->M.L.bytes;
+    if (lds > 64 * 1024) break;
+    const int64_t resident = (int64_t)s->cus * std::min<int64_t>(4, 160 * 1024 / lds), waves = (envs + K - 1) / K;
+    const double c = weight[i] * (double)((waves + resident - 1) / resident);
+    if (i == 0 || c < cost) {
+      best = K;
+      cost = c;
+    }
+  }
+  return best;
+}
+
 // The step without the learned warm start in the given launch shape, with
 // optional per-step controls and qpos outputs (Batch::rollout). Only kernels
 // go on the stream, so the sequence can be captured in a graph.
@@ -698,16 +741,32 @@ static hipError_t launch_plain(ph_sim* s, const ph_launch_shape& sh, int64_t beg
   const size_t lds = (size_t)K * s->M.L.bytes;
   const DModel* mp = s->d_model.p;
   const DState* sp = s->d_state.p;
-  if (sh.schedule == PH_SCHED_PGS_SPLIT) {  // three kernels per physics step, one env per workgroup
-    const unsigned grid = (unsigned)(end - begin);
+  if (sh.schedule == PH_SCHED_PGS_SPLIT) {  // front, sweeps and back of each physics step
+    const int64_t envs = end - begin;
+    const int FK = split_envs_per_wave(s, envs);
+    const unsigned grid = (unsigned)((envs + FK - 1) / FK);
+    const size_t flds = (size_t)FK * s->M.L.bytes;
     double* vel = s->d_pgs_vel.p;
     double* vpos = s->d_pgs_vpos.p;
+    const double *cvel = vel, *cvpos = vpos;
+    const int slice = s->pgs_slice;  // doubles of LDS per env of the packed sweeps
+    int64_t cap = slice;
+    unsigned* counter = s->d_counter.p;
     for (int64_t t = 0; t < nstep; t++) {
-      hipLaunchKernelGGL(k_pgs_front<1>, dim3(grid), dim3(64), lds, s->stream, mp, sp, begin, end, nstep, t, ctrl, vel,
-                         vpos);
-      hipLaunchKernelGGL(k_pgs_sweeps<1>, dim3(grid), dim3(64), 0, s->stream, mp, sp, begin, end, vel, vpos);
-      hipLaunchKernelGGL(k_pgs_back<1>, dim3(grid), dim3(64), lds, s->stream, mp, sp, begin, end, nstep, t, qpos_out,
-                         (const double*)vel, (const double*)vpos);
+      void* fargs[] = {&mp, &sp, &begin, &end, &nstep, &t, &ctrl, &vel, &vpos, &cap, &counter};
+      if (hipError_t e = hipLaunchKernel(pgs_front_kernel(FK), dim3(grid), dim3(64), fargs, flds, s->stream)) return e;
+      unsigned wide = (unsigned)envs;
+      if (slice > 0) {
+        const size_t slds = (size_t)4 * slice * sizeof(double);
+        const int64_t resident = (int64_t)s->cus * std::max(s->pgs_per_cu, 1);
+        const unsigned g4 = (unsigned)std::min<int64_t>((envs + 3) / 4, resident);
+        void* sargs[] = {&mp, &sp, &begin, &end, &vel, &vpos, (void*)&slice, &counter};
+        if (hipError_t e = hipLaunchKernel(pgs_rows_kernel(s->M), dim3(g4), dim3(64), sargs, slds, s->stream)) return e;
+        wide = (unsigned)std::min<int64_t>(envs, 4 * s->cus);  // few envs or none are left to the other kernel
+      }
+      hipLaunchKernelGGL(k_pgs_sweeps<1>, dim3(wide), dim3(64), 0, s->stream, mp, sp, begin, end, vel, vpos);
+      void* bargs[] = {&mp, &sp, &begin, &end, &nstep, &t, &qpos_out, &cvel, &cvpos};
+      if (hipError_t e = hipLaunchKernel(pgs_back_kernel(FK), dim3(grid), dim3(64), bargs, flds, s->stream)) return e;
       if (hipError_t e = hipGetLastError()) return e;
     }
     return hipSuccess;

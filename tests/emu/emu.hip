@@ -312,6 +312,45 @@ int emu_step(emu_sim* s, int64_t begin, int64_t end, int64_t nstep) {
   return 0;
 }
 
+// The PGS step as its front, sweeps and back (run_pgs_front, run_pgs_back), the
+// sweeps over packed rows where they fit cap doubles; returns how many env
+// steps took packed rows.
+int emu_step_split(emu_sim* s, int64_t begin, int64_t end, int64_t nstep, int64_t cap) {
+  const DModel& M = s->M;
+  const DState& S = s->S;
+  const int nv = M.nv;
+  Env E;
+  E.s = s->lds.data();
+  E.si = reinterpret_cast<int*>(E.s + M.L.ndouble);
+  std::vector<double> vel(nv), vpos(nv);
+  int packed = 0;
+  for (int64_t t = 0; t < nstep; t++)
+    for (int64_t e = begin; e < end; e++) {
+      E.e = e;
+      E.var = s->env_var[e];
+      std::fill(s->lds.begin(), s->lds.end(), std::numeric_limits<double>::quiet_NaN());
+      run_pgs_front<HostX>(M, S, E, nstep, t, nullptr, e - begin, vel.data(), vpos.data(), cap);
+      const int nr = S.nrows[e];
+      double* rw = (S.grow + e * (int64_t)M.nrmax * 10).p;
+      double* J = (S.gjac + e * (int64_t)M.nrmax * nv).p;
+      double* mj = (S.gmj + e * (int64_t)M.nrmax * nv).p;
+      if (S.status[e] == 0 && nr > 0 && rw[PR_MODE] != 0.0) {
+        packed++;
+        const PgsRecs rec{rw};
+        auto keep = [&]() { vpos = vel; };
+        const PgsAt start{0, 0, 0, false};
+        pgs_warm_rows<HostX>(mj, rec, nr, nv, vel.data());
+        if (M.pgs_w <= 12) pgs_sweeps_rows<HostX, 12>(pgs_consts(M), J, mj, rec, nr, nv, vel.data(), start, keep);
+        else pgs_sweeps_rows<HostX, 16>(pgs_consts(M), J, mj, rec, nr, nv, vel.data(), start, keep);
+      } else if (S.status[e] == 0 && nr > 0) {
+        pgs_sweeps_serial(pgs_consts(M), J, mj, rw, nr, nv, vel.data(), vpos.data());
+      }
+      std::fill(s->lds.begin(), s->lds.end(), std::numeric_limits<double>::quiet_NaN());
+      run_pgs_back<HostX>(M, S, E, nstep, t, nullptr, e - begin, vel.data(), vpos.data());
+    }
+  return packed;
+}
+
 // Learned warm start: parameters in the device layout (mlp.hpp), hidden width h, mode.
 int emu_mlp_set(emu_sim* s, int h, int mode, const float* P) {
   const int64_t np = mlp_nparam(h), nw = mlp_nweight(h), n = std::max<int64_t>(s->n, 1);

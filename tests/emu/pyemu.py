@@ -27,7 +27,7 @@ def lib():
         L.emu_create.argtypes = [vp, i64]
         L.emu_destroy.argtypes = [vp]
         L.emu_last_error.restype = C.c_char_p
-        for n, a in {"emu_step": [vp, i64, i64, i64], "emu_get": [vp, C.c_int, i64, i64, vp],
+        for n, a in {"emu_step": [vp, i64, i64, i64], "emu_step_split": [vp, i64, i64, i64, i64], "emu_get": [vp, C.c_int, i64, i64, vp],
                      "emu_set": [vp, C.c_int, i64, i64, vp], "emu_ncon": [vp, i64, i64, vp],
                      "emu_iters": [vp, i64, i64, vp], "emu_status": [vp, i64, i64, vp],
                      "emu_contacts": [vp, i64, vp, C.c_int32, vp], "emu_mass_bias": [vp, i64, i64, vp, vp],
@@ -66,6 +66,10 @@ class EmuSim:
 
     def step(self, b, e, nstep=1):
         self.L.emu_step(self.h, b, e, nstep)
+
+    def step_split(self, b, e, nstep=1, cap=1 << 20):
+        """The PGS step as front, sweeps and back; returns the env steps whose rows were packed."""
+        return self.L.emu_step_split(self.h, b, e, nstep, cap)
 
     def get(self, f, b=0, e=None):
         e = self.n if e is None else e
