@@ -100,6 +100,7 @@ struct DModel {
   // bodies of a pair, of a limited joint or of an equality), and the largest such block;
   // 0 when a row can hold more than 16
   int pgs_w, pgs_b;
+  int bmax;  // dofs of the largest dof block
   int hess_mfma;  // 1: Newton's dense Hessian J'DJ on the FP64 matrix cores (one env per wavefront only)
 
   gp<const int> body_parent, body_jntadr, body_jntnum, body_dofadr, body_dofnum, body_lastdof;

@@ -486,6 +486,8 @@ void init_dmodel_scalars(const HostModel& hm, int solver, int max_contacts, phk:
   M.ncmax = std::max(hm.ncmax, 1);
   if (max_contacts > 0) M.ncmax = std::min(M.ncmax, max_contacts);
   M.nrmax = std::max(4 * M.ncmax + 2 * hm.nlimited + d.neq, 1);
+  M.bmax = 0;
+  for (int b = 0; b < M.nblock; b++) M.bmax = std::max(M.bmax, hm.block_adr[b + 1] - hm.block_adr[b]);
   // the widest PGS row: the dof blocks it touches
   {
     auto block_of = [&](int dof) { return dof < 0 ? -1 : hm.dof_block[dof]; };

@@ -627,43 +627,67 @@ PHD void mass_solve(const MT& M, Env& E, Real* x) {
     chol_solve_block<X>(M, E, LD(chol), M.nv, M.block_adr[blk], M.block_adr[blk + 1], x);
 }
 
-// factor_mass then mass_solve for the common case (Euler, one dof block of
-// at most 16 dofs) in registers: M + h diag(damping) one row per lane, the
-// register Cholesky, then the two triangular solves. Other models take the
-// general path. Returns false when the matrix is not positive definite.
+// M + h diag(damping) factored and x solved on the dof blocks of at most NM
+// dofs in registers, the env's 16-lane rows taking a block each at a time
+// (block and row b, b + ROWS, ...): one matrix row per lane, the register
+// Cholesky, then the two triangular solves. The factor is stored in LD(chol).
+template <int NM, class X, class MT>
+PHD bool factor_solve_blocks(const MT& M, Env& E, Real h, Real* x) {
+  using LV = typename X::LV;
+  const int nv = M.nv;
+  const Real* qm = LD(qm);
+  auto damp = M.v_dof_damping + (int64_t)E.var * nv;
+  int* isc = E.si + M.L.i_iscal;
+  const int nblock = M.nblock;
+  for (int b0 = 0; b0 < nblock; b0 += X::ROWS) {
+    const int blk = b0 + X::row();
+    if (blk < nblock) {
+      const int s0 = nblock == 1 ? 0 : M.block_adr[blk], n = nblock == 1 ? nv : M.block_adr[blk + 1] - s0;
+      LV r[NM];
+#pragma unroll
+      for (int k = 0; k < NM; k++)
+        r[k] = X::gen([&](int l) {
+          Real v = qm[(s0 + clampi(l, n)) * nv + s0 + clampi(k, n)];
+          return (l < n && k < n) ? v : 0.0;
+        });
+      // add_implicit_terms (forward.rs:407-431): the diagonal gains h * damping
+      const LV hd = X::gen([&](int l) { return h * damp[s0 + clampi(l, n)]; });
+#pragma unroll
+      for (int k = 0; k < NM; k++) r[k] = X::sel([&](int l) { return l == k; }, r[k] + hd, r[k]);
+      if (!chol_rows<X, NM>(r, n)) {
+        if (nblock == 1 && X::ROWS == 1) return false;
+        X::each([&](int l) {
+          if (l == 0) isc[1] = 1;
+        });
+      } else {
+        store_lower<X, NM>(r, LD(chol), nv, s0, n);
+        X::order();
+        LV lr[NM], lc[NM], lii;
+        load_factor<X, NM>(LD(chol), nv, s0, n, lr, lc, &lii);
+        LV xv = X::gen([&](int l) {
+          Real v = x[s0 + clampi(l, n)];
+          return l < n ? v : 0.0;
+        });
+        xv = solve_rows<X, NM>(r, lc, lii, xv, n);
+        X::each([&](int l) {
+          if (l < n) x[s0 + l] = X::at(xv, l);
+        });
+      }
+    }
+  }
+  X::sync();
+  return (nblock == 1 && X::ROWS == 1) || isc[1] == 0;
+}
+
+// factor_mass then mass_solve. With Euler integration and dof blocks of at
+// most 16 dofs both run in registers, block by block; other models take the
+// general path. Returns false when the matrix is not positive definite
+// (isc[1], which the caller has cleared).
 template <class X, class MT>
 PHD bool factor_solve_mass(const MT& M, Env& E, Real h, Real* x) {
-  if (M.integrator == 0 && M.nblock == 1 && M.nv <= GL) {
-    using LV = typename X::LV;
-    const int nv = M.nv;
-    const Real* qm = LD(qm);
-    auto damp = M.v_dof_damping + (int64_t)E.var * nv;
-    LV r[GL];
-#pragma unroll
-    for (int k = 0; k < GL; k++)
-      r[k] = X::gen([&](int l) {
-        Real v = qm[clampi(l, nv) * nv + clampi(k, nv)];
-        return (l < nv && k < nv) ? v : 0.0;
-      });
-    // add_implicit_terms (forward.rs:407-431): the diagonal gains h * damping
-    const LV hd = X::gen([&](int l) { return h * damp[clampi(l, nv)]; });
-#pragma unroll
-    for (int k = 0; k < GL; k++) r[k] = X::sel([&](int l) { return l == k; }, r[k] + hd, r[k]);
-    if (!chol_rows<X>(r, nv)) return false;
-    store_lower<X>(r, LD(chol), nv, 0, nv);
-    X::sync();
-    LV lr[GL], lc[GL], lii;
-    load_factor<X>(LD(chol), nv, 0, nv, lr, lc, &lii);
-    LV xv = X::gen([&](int l) {
-      Real v = x[clampi(l, nv)];
-      return l < nv ? v : 0.0;
-    });
-    xv = solve_rows<X>(r, lc, lii, xv, nv);
-    X::each([&](int l) {
-      if (l < nv) x[l] = X::at(xv, l);
-    });
-    X::sync();
-    return true;
+  if (M.integrator == 0 && M.bmax <= GL) {
+    if (M.bmax <= 6) return factor_solve_blocks<6, X>(M, E, h, x);
+    return factor_solve_blocks<GL, X>(M, E, h, x);
   }
   if (!factor_mass<X>(M, E, h)) return false;
   mass_solve<X>(M, E, x);
@@ -895,8 +919,8 @@ PHD void mul_m(const NP& P, const Real* x, Real* y) {
 // in LDS and are read with independent loads; the Hessian is assembled one row
 // per lane directly into the register Cholesky. Every sum keeps the
 // reference's order, so the result equals newton_dense's bit for bit.
-template <class X, class MT>
-PHD int newton_lanes(const MT& M, Env& E, const NP& P) {
+template <class X, int NM = GL, class MT>
+PHD int newton_lanes(const MT& M, const NP& P) {
   using LV = typename X::LV;
   const int nv = P.nv, nr = P.nr, n_ineq = P.n_ineq;
   // every array of P is in LDS on this path
@@ -918,27 +942,27 @@ PHD int newton_lanes(const MT& M, Env& E, const NP& P) {
   };
   // M x (damp_h is zero inside Newton: damping is applied after the solve)
   auto mul_m = [&](const LV& x) {
-    LV xb[GL], mr[GL];
-    bcast_all<X>(x, xb);
+    LV xb[NM], mr[NM];
+    bcast_all<X, NM>(x, xb);
 #pragma unroll
-    for (int k = 0; k < GL; k++)
+    for (int k = 0; k < NM; k++)
       mr[k] = X::gen([&](int l) {
         Real v = qm[clampi(l, nv) * nv + clampi(k, nv)];
         return (l < nv && k < nv) ? v : 0.0;
       });
-    return lsdot_rt<X>(mr, xb, nv) + 0.0 * x;
+    return lsdot_rt<X, NM>(mr, xb, nv) + 0.0 * x;
   };
   // J x, one row per lane
   auto jdot = [&](const LV& x) {
-    LV xb[GL], jr[GL];
-    bcast_all<X>(x, xb);
+    LV xb[NM], jr[NM];
+    bcast_all<X, NM>(x, xb);
 #pragma unroll
-    for (int k = 0; k < GL; k++)
+    for (int k = 0; k < NM; k++)
       jr[k] = X::gen([&](int l) {
         Real v = J[clampi(l, nr) * nv + clampi(k, nv)];
         return (l < nr && k < nv) ? v : 0.0;
       });
-    return lsdot_rt<X>(jr, xb, nv);
+    return lsdot_rt<X, NM>(jr, xb, nv);
   };
   // column r of J^T: lane k gets J[r][k]
   auto jrow = [&](int r) {
@@ -965,18 +989,12 @@ PHD int newton_lanes(const MT& M, Env& E, const NP& P) {
   auto cost = [&](const LV& x, const LV& a0v) {
     LV t = x - a0v;
     LV t2 = mul_m(t);
-    Real c = 0.5 * X::uni(lsum_lanes<X>(t * t2, nv, -0.0));
+    Real c = 0.5 * (lsum_lanes<X, NM>(t * t2, nv, -0.0));
     LV jar = jdot(x) - aref;
     uint32_t on = active_mask(jar);
     LV term = ((0.5 * dd) * jar) * jar;
-    LV tb[GL];
-    bcast_all<X>(term, tb);
-#pragma unroll
-    for (int r = 0; r < GL; r++) {
-      Real cr = c + X::uni(tb[r]);
-      c = ((on >> r) & 1u) ? cr : c;
-    }
-    return c;
+    // an inactive row adds -0.0, which leaves the sum as it is
+    return X::template rowsum<GL>(X::sel([&](int l) { return ((on >> l) & 1u) != 0; }, term, X::splat(-0.0)), c);
   };
 
   const LV a0 = X::gen([&](int l) {
@@ -1002,7 +1020,7 @@ PHD int newton_lanes(const MT& M, Env& E, const NP& P) {
     }
   }
   const LV ma0 = mul_m(a0);
-  const Real scale = 1.0 + sqrt_cr(X::uni(lsum_lanes<X>(ma0 * ma0, nv, -0.0)));
+  const Real scale = 1.0 + sqrt_cr((lsum_lanes<X, NM>(ma0 * ma0, nv, -0.0)));
   const Real tol = M.tolerance;
   const int cap = M.iterations > 1 ? M.iterations : 1;
   uint64_t prev = ~(uint64_t)0;
@@ -1020,13 +1038,13 @@ PHD int newton_lanes(const MT& M, Env& E, const NP& P) {
     act_a = act;
     fresh = true;
     const LV grad = add_rows(mul_m(tmp), dd * jar, act);
-    const Real gnorm = sqrt_cr(X::uni(lsum_lanes<X>(grad * grad, nv, -0.0)));
+    const Real gnorm = sqrt_cr((lsum_lanes<X, NM>(grad * grad, nv, -0.0)));
     if (gnorm < tol * scale || ((uint64_t)act == prev && iters > 1)) break;
     prev = act;
     // H = M + sum_active D_r J_r^T J_r, row l in lane l
-    LV h[GL];
+    LV h[NM];
 #pragma unroll
-    for (int j = 0; j < GL; j++) {
+    for (int j = 0; j < NM; j++) {
       h[j] = X::gen([&](int l) {
         Real v = qm[clampi(l, nv) * nv + clampi(j, nv)];
         return (l < nv && j < nv) ? v : 0.0;
@@ -1038,45 +1056,33 @@ PHD int newton_lanes(const MT& M, Env& E, const NP& P) {
       const LV ji = jrow(r);
       const LV di = rdd[r] * ji;
 #pragma unroll
-      for (int j = 0; j < GL; j++) {
+      for (int j = 0; j < NM; j++) {
         Real jrj = J[r * nv + clampi(j, nv)];
         h[j] = X::sel([&](int l) { return on && X::at(ji, l) != 0.0; }, h[j] + di * jrj, h[j]);
       }
     }
-    if (!chol_rows<X>(h, nv)) break;
-    store_lower<X>(h, Lf, nv, 0, nv);
+    if (!chol_rows<X, NM>(h, nv)) break;
+    store_lower<X, NM>(h, Lf, nv, 0, nv);
     X::sync();
-    LV lr[GL], lc[GL], lii;
-    load_factor<X>(Lf, nv, 0, nv, lr, lc, &lii);
-    const LV p = solve_rows<X>(h, lc, lii, -grad, nv);
+    LV lr[NM], lc[NM], lii;
+    load_factor<X, NM>(Lf, nv, 0, nv, lr, lc, &lii);
+    const LV p = solve_rows<X, NM>(h, lc, lii, -grad, nv);
     // exact line search along p (newton.rs:310-351)
     const LV mp = mul_m(p);
-    const Real mpp = X::uni(lsum_lanes<X>(p * mp, nv, -0.0));
-    const Real mpg = X::uni(lsum_lanes<X>(tmp * mp, nv, -0.0));
+    const Real mpp = (lsum_lanes<X, NM>(p * mp, nv, -0.0));
+    const Real mpg = (lsum_lanes<X, NM>(tmp * mp, nv, -0.0));
     const LV jp = jdot(p);
     // Row r's terms, one row per lane: D_r jp_r v_r and D_r jp_r^2 when the
     // row is active at step al, v_r = jar_r + al jp_r; they are then added in
-    // row order. An inactive row (or a lane past nr) adds +0.0, which leaves
-    // the sums equal except for the sign of an exact zero, and no later use
-    // (|d1|, d1 < 0, al - d1 / max(d2, 1e-30)) depends on that sign.
+    // row order. An inactive row (or a lane past nr) adds -0.0, which leaves
+    // the sums as they are.
     const LV dq = dd * jp;
     const LV dq2 = dq * jp;
     auto deriv = [&](Real al, Real* d1o, Real* d2o) {
       const LV v = jar + al * jp;
       auto on = [&](int l) { return l < nr && (l >= n_ineq || X::at(v, l) < 0.0); };
-      const LV t1 = X::sel(on, dq * v, X::splat(0.0));
-      const LV t2 = X::sel(on, dq2, X::splat(0.0));
-      LV b1[GL], b2[GL];
-      bcast_all<X>(t1, b1);
-      bcast_all<X>(t2, b2);
-      Real d1 = al * mpp + mpg, d2 = mpp;
-#pragma unroll
-      for (int r = 0; r < GL; r++) {
-        d1 = d1 + X::uni(b1[r]);
-        d2 = d2 + X::uni(b2[r]);
-      }
-      *d1o = d1;
-      *d2o = d2;
+      *d1o = X::template rowsum<GL>(X::sel(on, dq * v, X::splat(-0.0)), al * mpp + mpg);
+      *d2o = X::template rowsum<GL>(X::sel(on, dq2, X::splat(-0.0)), mpp);
     };
     Real lo = 0.0, hi = INFINITY, al = 1.0, d1, d2;
     deriv(0.0, &d1, &d2);
@@ -1352,14 +1358,14 @@ PHD int newton_solve(const MT& M, const DState& S, Env& E, int nr, const Real* w
   auto whole = [&]() {
     if (nv <= GL && nr <= GL && nr <= M.nrl) {
       NP P{nv, nr, n_ineq, LD(qm), LD(J), LD(aref), LD(dd), LD(qacc), LD(a), LD(qfrc_c), LD(chol), warm2};
-      return newton_lanes<X>(M, E, P);
+      return newton_lanes<X>(M, P);
     }
     NP P{nv, nr, n_ineq, LD(qm), E.J, E.aref, E.dd, LD(qacc), LD(a), LD(qfrc_c), LD(chol), warm2};
     return newton_dense<X>(M, E, P);
   };
   if (M.nblock <= 1) return whole();
-  // per-env island scratch: floats in HBM (gathered into LDS below when an
-  // island fits), the bookkeeping ints in the env's LDS int region
+  // per-env island scratch: floats in HBM (islands of the register solver are
+  // gathered into LDS), the bookkeeping ints in the env's LDS int region
   Real* fs = (S.isl_f + E.e * (int64_t)M.isl_fstride).p;
   int* is = E.si + M.L.i_isl;
   int* rmask = is;                 // nrmax: blocks each row touches
@@ -1367,94 +1373,175 @@ PHD int newton_solve(const MT& M, const DState& S, Env& E, int nr, const Real* w
   int* sridx = sidx + nv;          // nrmax: gathered rows
   int* root = sridx + M.nrmax;     // nblock: island of each block
   int* isl = root + M.nblock;      // nblock + 1: island list, then its length
-  Real* sqm = fs;
-  Real* sJ = sqm + nv * nv;
-  Real* saref = sJ + (int64_t)M.nrmax * nv;
-  Real* sdd = saref + M.nrmax;
-  Real* sa = sdd + M.nrmax;
-  Real* swarm = sa + nv;
-  Real* sqf = swarm + nv;
-  Real* swarm2 = sqf + nv;
-  int* isc = E.si + M.L.i_iscal;
+  const int nb = M.nblock;
+  // per block, in vectors that only newton_dense uses: the blocks its rows
+  // couple it to; per island (at its first block): dofs, rows
+  int* adj = reinterpret_cast<int*>(LD(tmp));
+  int* ik = reinterpret_cast<int*>(LD(tmp2));
+  int* iq = reinterpret_cast<int*>(LD(mp));
+  int* its = reinterpret_cast<int*>(LD(scal) + 8);  // per 16-lane row: iterations
   const Real* J = E.J;
+  X::par(nb, [&](int b) {
+    adj[b] = 0;
+    ik[b] = 0;
+    iq[b] = 0;
+  });
   X::par(nr, [&](int r) {
     uint32_t m = 0;
-    for (int k = 0; k < nv; k++)
-      if (J[r * nv + k] != 0.0) m |= 1u << M.dof_block[k];
-    rmask[r] = (int)m;
-  });
-  X::par(1, [&](int) {
-    const int nb = M.nblock;
-    for (int b = 0; b < nb; b++) root[b] = b;
-    auto find = [&](int x) {
-      while (root[x] != x) x = root[x];
-      return x;
-    };
-    for (int r = 0; r < nr; r++) {
-      uint32_t m = (uint32_t)rmask[r];
-      if (!m) continue;
-      int first = __builtin_ctz(m);
-      for (int b = first + 1; b < nb; b++)
-        if ((m >> b) & 1u) {
-          int x = find(first), y = find(b);
-          if (x != y) root[x > y ? x : y] = x < y ? x : y;
-        }
-    }
-    for (int b = 0; b < nb; b++) root[b] = find(b);
-    // islands holding a row, in increasing order
-    int ni = 0;
     for (int b = 0; b < nb; b++) {
-      bool used = false;
-      for (int r = 0; r < nr && !used; r++) used = rmask[r] && root[__builtin_ctz((uint32_t)rmask[r])] == b;
-      if (used) isl[ni++] = b;
+      bool any = false;
+      for (int k = M.block_adr[b]; k < M.block_adr[b + 1]; k++) any = any || J[r * nv + k] != 0.0;
+      m |= any ? 1u << b : 0u;
     }
-    bool all = ni == 1;
-    for (int b = 0; b < nb && all; b++) all = root[b] == isl[0];
-    isl[nb] = all ? -1 : ni;
+    rmask[r] = (int)m;
+    for (uint32_t u = m; u; u &= u - 1) X::ior(&adj[__builtin_ctz(u)], (int)m);
   });
-  if (isl[M.nblock] < 0) return whole();
-  const int ni = isl[M.nblock];
-  int iters = 0;
-  for (int ii = 0; ii < ni; ii++) {
-    X::par(1, [&](int) {
-      const int id = isl[ii];
-      int k = 0, q = 0, qi = 0;
-      for (int b = 0; b < M.nblock; b++)
-        if (root[b] == id)
-          for (int d = M.block_adr[b]; d < M.block_adr[b + 1]; d++) sidx[k++] = d;
-      for (int r = 0; r < nr; r++)
-        if (rmask[r] && root[__builtin_ctz((uint32_t)rmask[r])] == id) {
-          sridx[q++] = r;
-          if (r < n_ineq) qi++;
-        }
-      isc[10] = k;
-      isc[11] = q;
-      isc[12] = qi;
-    });
-    const int k = isc[10], q = isc[11], qi = isc[12];
-    // An island the register solver takes (k, q <= 16) is gathered into the
-    // LDS of the mass-factor slot, after the k x k Hessian factor that the
-    // solver keeps there, when it fits; otherwise into the HBM island scratch.
-    const bool lds_isl = k <= GL && q <= GL && 2 * k * k + q * k + 2 * q + 4 * k <= nv * nv;
-    if (lds_isl) {
-      sqm = LD(chol) + k * k;
-      sJ = sqm + k * k;
-      saref = sJ + q * k;
-      sdd = saref + q;
-      sa = sdd + q;
-      swarm = sa + k;
-      sqf = swarm + k;
-      swarm2 = sqf + k;
-    } else {
-      sqm = fs;
-      sJ = sqm + nv * nv;
-      saref = sJ + (int64_t)M.nrmax * nv;
-      sdd = saref + M.nrmax;
-      sa = sdd + M.nrmax;
-      swarm = sa + nv;
-      sqf = swarm + nv;
-      swarm2 = sqf + nv;
+  // an island's name is its smallest block: the lowest bit of everything a
+  // block reaches (the reference's union-find links larger roots to smaller
+  // ones)
+  X::par(nb, [&](int b) {
+    uint32_t reach = (uint32_t)adj[b] | 1u << b, seen = 0;
+    while (uint32_t todo = reach & ~seen) {
+      const int c = __builtin_ctz(todo);
+      seen |= 1u << c;
+      reach |= (uint32_t)adj[c];
     }
+    root[b] = __builtin_ctz(reach);
+  });
+  X::par(nb, [&](int b) { X::iadd(&ik[root[b]], M.block_adr[b + 1] - M.block_adr[b]); });
+  X::par(nr, [&](int r) {
+    if (!rmask[r]) return;
+    X::iadd(&iq[root[__builtin_ctz((uint32_t)rmask[r])]], 1);
+  });
+  // islands holding a row, in increasing order; -1 when one spans every block
+  X::par(1, [&](int) {
+    int ni = 0;
+    for (int b = 0; b < nb; b++)
+      if (root[b] == b && iq[b] > 0) isl[ni++] = b;
+    isl[nb] = ni == 1 && ik[isl[0]] == nv ? -1 : ni;
+  });
+  if (isl[nb] < 0) return whole();
+  const int ni = isl[nb];
+  // the dofs and rows of an island, in increasing order, by 16 lanes
+  auto list = [&](int id, int* dofs, int* rows, int* kn, int* qn, int* qin) {
+    int k = 0, q = 0, qi = 0;
+    for (int c = 0; c < nv; c += GL) {
+      const uint32_t m = X::ballot([&](int l) { return c + l < nv && root[M.dof_block[clampi(c + l, nv)]] == id; });
+      X::each([&](int l) {
+        if ((m >> l) & 1u) dofs[k + __builtin_popcount(m & ((1u << l) - 1u))] = c + l;
+      });
+      k += __builtin_popcount(m);
+    }
+    for (int c = 0; c < nr; c += GL) {
+      const uint32_t m = X::ballot([&](int l) {
+        const int r = clampi(c + l, nr);
+        return c + l < nr && rmask[r] && root[__builtin_ctz((uint32_t)rmask[r])] == id;
+      });
+      X::each([&](int l) {
+        if ((m >> l) & 1u) rows[q + __builtin_popcount(m & ((1u << l) - 1u))] = c + l;
+      });
+      q += __builtin_popcount(m);
+      const int left = n_ineq - c;  // inequality rows of this chunk
+      qi += left >= GL ? __builtin_popcount(m) : (left > 0 ? __builtin_popcount(m & ((1u << left) - 1u)) : 0);
+    }
+    *kn = k;
+    *qn = q;
+    *qin = qi;
+  };
+  // Islands that the register solver takes (k, q <= 16): each of the env's
+  // 16-lane rows solves one, as many at a time as fit the LDS of the
+  // mass-factor slot (per island the Hessian factor, then the gathered
+  // problem). One after the other, on 16 of the wavefront's 64 lanes, they
+  // were 139 us of a 363 us step on the six-body pile, and gathering them 59.
+  auto doubles = [](int k, int q) { return 2 * k * k + q * k + 2 * q + 4 * k; };
+  auto in_lanes = [&](int id) { return ik[id] <= GL && iq[id] <= GL && doubles(ik[id], iq[id]) <= nv * nv; };
+  int iters = 0;
+  for (int next = 0; next < ni;) {
+    // this row's island of the batch: the row()-th that fits after the ones
+    // before it
+    int id = -1, o = 0, po = 0, taken = 0, kmax = 0, used = 0, ints = 0;
+    for (; next < ni && taken < X::ROWS; next++) {
+      const int c = isl[next];
+      if (!in_lanes(c)) continue;
+      const int need = doubles(ik[c], iq[c]);
+      if (used + need > nv * nv) break;
+      if (taken == X::row()) {
+        id = c;
+        o = used;
+        po = ints;
+      }
+      kmax = ik[c] > kmax ? ik[c] : kmax;
+      used += need;
+      ints += ik[c] + iq[c];
+      taken++;
+    }
+    int it = 0;
+    if (id >= 0) {
+      int k, q, qi;
+      int* dofs = sidx + po;  // the batch's lists, one after the other
+      int* rows = dofs + ik[id];
+      list(id, dofs, rows, &k, &q, &qi);
+      X::order();
+      Real* fac = LD(chol) + o;
+      Real* sqm = fac + k * k;
+      Real* sJ = sqm + k * k;
+      Real* saref = sJ + q * k;
+      Real* sdd = saref + q;
+      Real* sa = sdd + q;
+      Real* swarm = sa + k;
+      Real* sqf = swarm + k;
+      Real* swarm2 = sqf + k;
+      X::each([&](int l) {
+        if (l < k) {
+          const int d = dofs[l];
+          const Real* qm = LD(qm) + d * nv;
+          for (int i = 0; i < k; i++) sqm[l * k + i] = qm[dofs[i]];
+          for (int t = 0; t < q; t++) sJ[t * k + l] = J[rows[t] * nv + d];
+          sa[l] = LD(a)[d];
+          swarm[l] = LD(qacc)[d];
+          if (warm2) swarm2[l] = warm2[d];
+        }
+        if (l < q) {
+          saref[l] = E.aref[rows[l]];
+          sdd[l] = E.dd[rows[l]];
+        }
+      });
+      X::order();
+      const NP P{k, q, qi, sqm, sJ, saref, sdd, swarm, sa, sqf, fac, warm2 ? swarm2 : nullptr};
+      it = kmax <= 6 ? newton_lanes<X, 6>(M, P) : newton_lanes<X>(M, P);
+      X::each([&](int l) {
+        if (l < k) {
+          LD(a)[dofs[l]] = sa[l];
+          LD(qfrc_c)[dofs[l]] = sqf[l];
+        }
+      });
+    }
+    X::each([&](int l) {
+      if (l == 0) its[X::row()] = it;
+    });
+    X::sync();
+    for (int r = 0; r < X::ROWS; r++) iters = its[r] > iters ? its[r] : iters;
+    X::sync();
+  }
+  // larger islands, gathered into HBM, one after the other (newton_dense takes
+  // the vectors that hold the counts, so the islands done are struck out first)
+  X::par(ni, [&](int i) {
+    if (in_lanes(isl[i])) isl[i] = -1;
+  });
+  for (int ii = 0; ii < ni; ii++) {
+    const int id = isl[ii];
+    if (id < 0) continue;
+    int k, q, qi;
+    list(id, sidx, sridx, &k, &q, &qi);
+    X::sync();
+    Real* sqm = fs;
+    Real* sJ = sqm + nv * nv;
+    Real* saref = sJ + (int64_t)M.nrmax * nv;
+    Real* sdd = saref + M.nrmax;
+    Real* sa = sdd + M.nrmax;
+    Real* swarm = sa + nv;
+    Real* sqf = swarm + nv;
+    Real* swarm2 = sqf + nv;
     X::par(k * k, [&](int t) { sqm[t] = LD(qm)[sidx[t / k] * nv + sidx[t % k]]; });
     X::par(q * k, [&](int t) { sJ[t] = J[sridx[t / k] * nv + sidx[t % k]]; });
     X::par(q, [&](int t) {
@@ -1467,7 +1554,7 @@ PHD int newton_solve(const MT& M, const DState& S, Env& E, int nr, const Real* w
       if (warm2) swarm2[t] = warm2[sidx[t]];
     });
     NP P{k, q, qi, sqm, sJ, saref, sdd, swarm, sa, sqf, LD(chol), warm2 ? swarm2 : nullptr};
-    int it = (k <= GL && q <= GL) ? newton_lanes<X>(M, E, P) : newton_dense<X>(M, E, P);
+    int it = (k <= GL && q <= GL) ? newton_lanes<X>(M, P) : newton_dense<X>(M, E, P);
     iters = it > iters ? it : iters;
     X::par(k, [&](int t) {
       LD(a)[sidx[t]] = sa[t];

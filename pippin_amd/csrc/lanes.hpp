@@ -108,6 +108,9 @@ struct DevLanes {
 #undef PH_ROWSUM
     return s;
   }
+  // p |= v and p += v by several lanes
+  __device__ __forceinline__ static void ior(int* p, int v) { atomicOr(p, v); }
+  __device__ __forceinline__ static void iadd(int* p, int v) { atomicAdd(p, v); }
   // LDS writes of this wavefront's lanes before this point are seen by its
   // reads after it (LDS serves a wavefront's operations in order, so this only
   // keeps the compiler from moving them)
@@ -208,6 +211,8 @@ struct HostLanes {
     return s;
   }
   static void order() {}
+  static void ior(int* p, int v) { *p |= v; }
+  static void iadd(int* p, int v) { *p += v; }
   // 16-lane rows that work on one env, and this lane's (the device policies
   // own 4, 2 or 1 by their envs per wavefront)
   static constexpr int ROWS = 1;
@@ -252,10 +257,13 @@ PHD LV lsdot(const LV* a, const LV* b) {
   }
 }
 
-// out[k] = lane k's x, in every lane
-template <class X, class LV>
+// The functions below hold up to NM rows or entries (their loops are unrolled
+// to that), NM = 16 or, for free bodies' blocks, 6.
+
+// out[k] = lane k's x, in every lane, k < NM
+template <class X, int NM = GL, class LV>
 PHD void bcast_all(LV x, LV* out) {
-  sfor<0, GL>([&](auto KC) {
+  sfor<0, NM>([&](auto KC) {
     constexpr int k = decltype(KC)::value;
     out[k] = X::template bc<k>(x);
     return true;
@@ -264,19 +272,19 @@ PHD void bcast_all(LV x, LV* out) {
 
 // sdot_n (simd.rs:14-64) of a runtime length n <= 16 over register arrays;
 // the structure switches on n (uniform), the unrolled terms stay in order.
-template <class X, class LV>
+template <class X, int NM = GL, class LV>
 PHD LV lsdot_rt(const LV* a, const LV* b, int n) {
-  if (n < 8) {
+  if (NM < 8 || n < 8) {
     LV s = X::splat(0.0);
 #pragma unroll
-    for (int k = 0; k < 7; k++)
+    for (int k = 0; k < (NM < 7 ? NM : 7); k++)
       if (k < n) s = s + a[k] * b[k];
     return s;
   }
   LV s0 = X::splat(0.0), s1 = s0, s2 = s0, s3 = s0;
   const int nb = n / 4 * 4;
 #pragma unroll
-  for (int k = 0; k < GL; k += 4)
+  for (int k = 0; k + 4 <= NM; k += 4)
     if (k + 4 <= nb) {
       s0 = s0 + a[k] * b[k];
       s1 = s1 + a[k + 1] * b[k + 1];
@@ -285,22 +293,17 @@ PHD LV lsdot_rt(const LV* a, const LV* b, int n) {
     }
   LV t = (s0 + s1) + (s2 + s3);
 #pragma unroll
-  for (int k = 8; k < GL; k++)
+  for (int k = 8; k < NM; k++)
     if (k >= nb && k < n) t = t + a[k] * b[k];
   return t;
 }
 
-// Sequential sum of lane values 0..n-1 starting from `start` (Rust's
-// iterator sum folds from -0.0), computed redundantly in every lane.
-template <class X, class LV>
-PHD LV lsum_lanes(LV x, int n, Real start) {
-  LV xb[GL];
-  bcast_all<X>(x, xb);
-  LV s = X::splat(start);
-#pragma unroll
-  for (int k = 0; k < GL; k++)
-    if (k < n) s = s + xb[k];
-  return s;
+// Sequential sum of lane values 0..n-1 (n <= NM) starting from `start` (Rust's
+// iterator sum folds from -0.0), computed redundantly in every lane. The
+// lanes past n add -0.0, which leaves every sum as it is.
+template <class X, int NM = GL, class LV>
+PHD Real lsum_lanes(LV x, int n, Real start) {
+  return X::template rowsum<NM>(X::sel([&](int l) { return l < n; }, x, X::splat(-0.0)), start);
 }
 
 // math.rs:425-447 with one row per lane: in-place lower Cholesky of the
@@ -309,10 +312,10 @@ PHD LV lsum_lanes(LV x, int n, Real start) {
 // dot with row j, lane j's diagonal is broadcast, square-rooted and inverted,
 // and rows below scale their entry j. Only the lower triangle is written, as in
 // the reference. Returns false when a pivot is not positive.
-template <class X, class LV>
+template <class X, int NM = GL, class LV>
 PHD bool chol_rows(LV* r, int n) {
   bool ok = true;
-  sfor<0, GL>([&](auto JC) {
+  sfor<0, NM>([&](auto JC) {
     constexpr int j = decltype(JC)::value;
     if (j >= n) return false;
     LV b[j > 0 ? j : 1];
@@ -334,12 +337,12 @@ PHD bool chol_rows(LV* r, int n) {
 
 // Store the lower triangle (with the diagonal) of register rows into the
 // diagonal block [s0, s0 + n) of A.
-template <class X, class LV>
+template <class X, int NM = GL, class LV>
 PHD void store_lower(const LV* r, Real* A, int nv, int s0, int n) {
   X::each([&](int l) {
     if (l < n) {
 #pragma unroll
-      for (int k = 0; k < GL; k++)
+      for (int k = 0; k < NM; k++)
         if (k <= l) A[(s0 + l) * nv + s0 + k] = X::at(r[k], l);
     }
   });
@@ -364,10 +367,10 @@ PHD bool chol_lanes(Real* A, int nv, int s0, int n) {
 // its dot with the solved prefix, divides, and broadcasts), then backward
 // substitution (lane i divides and broadcasts; lanes above update with
 // column entries they loaded up front). x is overwritten with the solution.
-template <class X, class LV>
+template <class X, int NM = GL, class LV>
 PHD LV solve_rows(const LV* r, const LV* c, LV lii, LV xv, int n) {
-  LV xs[GL];
-  sfor<0, GL>([&](auto IC) {
+  LV xs[NM];
+  sfor<0, NM>([&](auto IC) {
     constexpr int i = decltype(IC)::value;
     if (i >= n) return false;
     LV t = (xv - lsdot<X, i>(r, xs)) / lii;
@@ -375,7 +378,7 @@ PHD LV solve_rows(const LV* r, const LV* c, LV lii, LV xv, int n) {
     xv = X::sel([](int l) { return l == i; }, t, xv);
     return true;
   });
-  sfor_down<0, GL>([&](auto IC) {
+  sfor_down<0, NM>([&](auto IC) {
     constexpr int i = decltype(IC)::value;
     if (i >= n) return;
     LV q = xv / lii;
@@ -387,10 +390,10 @@ PHD LV solve_rows(const LV* r, const LV* c, LV lii, LV xv, int n) {
 
 // Load, for lane l, row l of the strict lower triangle (r), column l below the
 // diagonal (c) and the diagonal entry of the factor in block [s0, s0 + n).
-template <class X, class LV>
+template <class X, int NM = GL, class LV>
 PHD void load_factor(const Real* L, int nv, int s0, int n, LV* r, LV* c, LV* lii) {
 #pragma unroll
-  for (int k = 0; k < GL; k++) {
+  for (int k = 0; k < NM; k++) {
     r[k] = X::gen([&](int l) {
       Real v = L[(s0 + clampi(l, n)) * nv + s0 + clampi(k, n)];
       return (l < n && k < l) ? v : 0.0;
