@@ -21,9 +21,11 @@ namespace phk {
 // On the host both are plain pointers; the layout is one pointer either way.
 #if defined(__HIP_DEVICE_COMPILE__)
 #define PH_AS_GLOBAL __attribute__((address_space(1)))
+#define PH_AS_LDS __attribute__((address_space(3)))
 #define PH_AS_CONST __attribute__((address_space(4)))
 #else
 #define PH_AS_GLOBAL
+#define PH_AS_LDS
 #define PH_AS_CONST
 #endif
 template <class T>
@@ -100,6 +102,7 @@ struct DModel {
   // bodies of a pair, of a limited joint or of an equality), and the largest such block;
   // 0 when a row can hold more than 16
   int pgs_w, pgs_b;
+  int x1;    // doubles of LDS past the layout for constraint rows, with one env per wavefront
   int bmax;  // dofs of the largest dof block
   int hess_mfma;  // 1: Newton's dense Hessian J'DJ on the FP64 matrix cores (one env per wavefront only)
 

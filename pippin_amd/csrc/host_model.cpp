@@ -508,7 +508,7 @@ void init_dmodel_scalars(const HostModel& hm, int solver, int max_contacts, phk:
     M.pgs_b = w <= 16 ? bmax : 0;
   }
   // island scratch (newton.rs:378-473), only when several dof blocks exist
-  M.isl_fstride = M.nblock > 1 ? d.nv * d.nv + M.nrmax * (d.nv + 2) + 4 * d.nv : 0;
+  M.isl_fstride = M.nblock > 1 ? d.nv * d.nv + M.nrmax * (d.nv + 7) + 4 * d.nv : 0;
   M.isl_istride = M.nblock > 1 ? 2 * M.nrmax + d.nv + 2 * M.nblock + 1 : 0;  // ints, in LDS (Layout::i_isl)
   // Rows beyond nrl live in HBM. Keep up to 32 in LDS, fewer if that keeps
   // the per-env working set within 10 KiB (four 4-env workgroups per CU); one
@@ -520,6 +520,9 @@ void init_dmodel_scalars(const HostModel& hm, int solver, int max_contacts, phk:
     M.nrl -= 1;
     M.L = make_layout(hm, M.nrl, M.npair, M.ncmax, M.isl_istride);
   }
+  // with one env per wavefront, rows past nrl stay in LDS as far as four
+  // wavefronts per CU leave room
+  M.x1 = solver == 0 && M.L.bytes < 40 * 1024 ? (40 * 1024 - M.L.bytes) / 8 : 0;
 
 }
 

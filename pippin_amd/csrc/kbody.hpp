@@ -25,12 +25,16 @@ struct Env {
   int var;
   // row storage for the current solve (LDS when it fits, else global)
   Real *J, *aref, *dd, *jar, *jp, *rpos, *rdiag, *ract, *rprev, *rf;
+  bool rows_lds;
 };
 
 #define LD(name) (E.s + M.L.name)
 
+// Row storage: the LDS row block for up to nrl rows, the LDS past the layout
+// when one env owns the wavefront and its rows fit there, else HBM.
 template <class X, class MT>
 PHD void rows_bind(const MT& M, const DState& S, Env& E, int nr) {
+  E.rows_lds = true;
   if (nr <= M.nrl) {
     E.J = LD(J);
     E.aref = LD(aref);
@@ -42,19 +46,28 @@ PHD void rows_bind(const MT& M, const DState& S, Env& E, int nr) {
     E.ract = LD(ract);
     E.rprev = LD(rprev);
     E.rf = LD(rf);
-  } else {
-    E.J = (S.gjac + E.e * (int64_t)M.nrmax * M.nv).p;
-    Real* g = (S.grow + E.e * (int64_t)M.nrmax * 10).p;
-    E.aref = g;
-    E.dd = g + M.nrmax;
-    E.jar = g + 2 * M.nrmax;
-    E.jp = g + 3 * M.nrmax;
-    E.rpos = g + 4 * M.nrmax;
-    E.rdiag = g + 5 * M.nrmax;
-    E.ract = g + 6 * M.nrmax;
-    E.rprev = g + 7 * M.nrmax;
-    E.rf = g + 8 * M.nrmax;
+    return;
   }
+  int64_t stride = nr;
+  Real* g = E.s + M.L.bytes / 8;
+  if (X::ROWS == 4 && (int64_t)nr * (M.nv + 7) <= M.x1) {
+    E.J = g;
+    g += (int64_t)nr * M.nv;
+  } else {
+    E.rows_lds = false;
+    E.J = (S.gjac + E.e * (int64_t)M.nrmax * M.nv).p;
+    g = (S.grow + E.e * (int64_t)M.nrmax * 10).p;
+    stride = M.nrmax;
+  }
+  E.aref = g;
+  E.dd = g + stride;
+  E.jar = g + 2 * stride;
+  E.jp = g + 3 * stride;
+  E.rpos = E.jar;  // row positions and diagonals are read before J a and J p are formed
+  E.rdiag = E.jp;
+  E.ract = g + 4 * stride;
+  E.rprev = g + 5 * stride;
+  E.rf = g + 6 * stride;
 }
 
 // ---------------- kinematics, forward.rs:14-90 ----------------
@@ -709,7 +722,7 @@ PHD int build_rows(const MT& M, const DState& S, Env& E) {
   // from a scan across the lanes; otherwise one lane walks the joints.
   const bool lane_limits = M.njnt <= GL;
   using LV = typename X::LV;
-  auto seps_of = [&](int j, Real* s0, Real* s1) {
+  auto seps_of = [&](int j, Real* s0, Real* s1) __attribute__((always_inline)) {
     int t = M.jnt_type[j];
     if (!M.jnt_limited[j] || !(t == J_HINGE || t == J_SLIDE)) return 0;
     Real q = qpos[M.jnt_qposadr[j]];
@@ -816,7 +829,7 @@ PHD int build_rows(const MT& M, const DState& S, Env& E) {
   });
   // joint limit rows, in joint order (lower then upper), then equalities
   auto iw = M.v_dof_invweight + (int64_t)E.var * nv;
-  auto limit_rows = [&](int j, int f, int r) {
+  auto limit_rows = [&](int j, int f, int r) __attribute__((always_inline)) {
     Real seps[2];
     seps_of(j, &seps[0], &seps[1]);
     int da = M.jnt_dofadr[j];
@@ -895,23 +908,31 @@ PHD int build_rows(const MT& M, const DState& S, Env& E) {
 }
 
 // ---------------- Newton, newton.rs:224-371 ----------------
-// One Newton problem: the whole model (one island) or one island gathered
-// into its own arrays (newton.rs:436-471).
-struct NP {
-  int nv, nr, n_ineq;                  // dofs, rows, rows below n_ineq are inequalities
-  const Real *qm, *J, *aref, *dd;      // qm: nv x nv, J: nr x nv (row stride nv)
-  const Real* warm;                    // previous acceleration (warm start candidate)
-  Real* a;                             // in: unconstrained acceleration; out: solution
-  Real* qf;                            // out: constraint force, nv
-  Real* fac;                           // nv x nv factor storage
-  const Real* warm2;                   // learned warm-start candidate, or null
-};
+// LDS pointers. The solvers below are called out of line in the kernels of
+// run-time sizes (several copies of each inlined into one kernel grow it past
+// what the compiler keeps in order), so what they take is passed by value and
+// typed as LDS; a closure or structure in memory would turn every LDS access
+// of the kernel into a flat one.
+typedef PH_AS_LDS Real* LP;
+typedef PH_AS_GLOBAL Real* GP;
+typedef PH_AS_LDS int* LPI;
 
-template <class X>
-PHD void mul_m(const NP& P, const Real* x, Real* y) {
-  const int nv = P.nv;
-  X::par(nv, [&](int i) { y[i] = sdot_n(P.qm + i * nv, x, nv) + 0.0 * x[i]; });
-}
+// One Newton problem: the whole model (one island) or one island gathered
+// into its own arrays (newton.rs:436-471). QP: where its mass matrix is.
+template <class QP>
+struct NPT {
+  int nv, nr, n_ineq;  // dofs, rows, rows below n_ineq are inequalities
+  int cap;             // iterations at most
+  Real tol;
+  QP qm;               // nv x nv
+  LP warm;             // previous acceleration (warm start candidate)
+  LP a;                // in: unconstrained acceleration; out: solution
+  LP qf;               // out: constraint force, nv
+  LP fac;              // nv x nv factor storage
+  LP warm2;            // learned warm-start candidate, if has_warm2
+  bool has_warm2;
+};
+typedef NPT<LP> NP;
 
 // newton.rs:224-371 for nv <= 16 and nr <= 16 rows held in LDS, with the
 // vectors in registers: a dof vector holds dof k in lane k, a row vector holds
@@ -919,17 +940,14 @@ PHD void mul_m(const NP& P, const Real* x, Real* y) {
 // in LDS and are read with independent loads; the Hessian is assembled one row
 // per lane directly into the register Cholesky. Every sum keeps the
 // reference's order, so the result equals newton_dense's bit for bit.
-template <class X, int NM = GL, class MT>
-PHD int newton_lanes(const MT& M, const NP& P) {
+template <class X, int NM = GL>
+PHD int newton_lanes_body(const NP& P, const LP J, const LP raref, const LP rdd) {
   using LV = typename X::LV;
   const int nv = P.nv, nr = P.nr, n_ineq = P.n_ineq;
-  // every array of P is in LDS on this path
-  const Real* qm = P.qm;
-  const Real* J = P.J;
-  const Real* rdd = P.dd;
-  Real* Lf = P.fac;
+  const LP qm = P.qm;
+  const LP Lf = P.fac;
   const LV aref = X::gen([&](int l) {
-    Real v = P.aref[clampi(l, nr)];
+    Real v = raref[clampi(l, nr)];
     return l < nr ? v : 0.0;
   });
   const LV dd = X::gen([&](int l) {
@@ -986,15 +1004,17 @@ PHD int newton_lanes(const MT& M, const NP& P) {
     }
     return g;
   };
-  auto cost = [&](const LV& x, const LV& a0v) {
-    LV t = x - a0v;
-    LV t2 = mul_m(t);
-    Real c = 0.5 * (lsum_lanes<X, NM>(t * t2, nv, -0.0));
-    LV jar = jdot(x) - aref;
-    uint32_t on = active_mask(jar);
-    LV term = ((0.5 * dd) * jar) * jar;
-    // an inactive row adds -0.0, which leaves the sum as it is
-    return X::template rowsum<GL>(X::sel([&](int l) { return ((on >> l) & 1u) != 0; }, term, X::splat(-0.0)), c);
+  // cost(x) = 1/2 (x-a0)'M(x-a0) + sum_active 1/2 D r^2 with r = J x - aref;
+  // quad is its first part, an inactive row adds -0.0, which changes no sum
+  auto row_terms = [&](const LV& jar) {
+    const uint32_t on = active_mask(jar);
+    return X::sel([&](int l) { return ((on >> l) & 1u) != 0; }, ((0.5 * dd) * jar) * jar, X::splat(-0.0));
+  };
+  auto cost = [&](const LV& x, const LV& a0v, LV* mt, LV* jar) {
+    const LV t = x - a0v;
+    *mt = mul_m(t);
+    *jar = jdot(x) - aref;
+    return X::template rowsum<GL>(row_terms(*jar), 0.5 * lsum_lanes<X, NM>(t * *mt, nv, -0.0));
   };
 
   const LV a0 = X::gen([&](int l) {
@@ -1002,27 +1022,43 @@ PHD int newton_lanes(const MT& M, const NP& P) {
     return l < nv ? v : 0.0;
   });
   LV a = a0;
+  // M (a - a0) and J a - aref of the start, for the first iteration
+  LV mt_a, jar_s;
   {
     const LV warm = X::gen([&](int l) {
       Real v = P.warm[clampi(l, nv)];
       return l < nv ? v : 0.0;
     });
-    Real c0 = cost(a0, a0), c1 = cost(warm, a0);
-    if (c1 < c0) a = warm;
-    if (P.warm2) {
+    // both costs side by side; a0's first part is the sum of 0 = a0 - a0, or
+    // NaN when a0 is not finite
+    const LV t0 = a0 - a0, t1 = warm - a0;
+    const LV mt1 = mul_m(t1), jar0 = jdot(a0) - aref, jar1 = jdot(warm) - aref;
+    Real q0, q1, c0, c1;
+    lsum2_lanes<X, NM>(t0, t1 * mt1, nv, -0.0, &q0, &q1);
+    X::template rowsum2<GL>(row_terms(jar0), row_terms(jar1), 0.5 * q0, 0.5 * q1, &c0, &c1);
+    const bool take = c1 < c0;
+    a = X::sel([&](int) { return take; }, warm, a0);
+    mt_a = X::sel([&](int) { return take; }, mt1, X::splat(q0));  // M 0
+    jar_s = X::sel([&](int) { return take; }, jar1, jar0);
+    if (P.has_warm2) {
       // the learned candidate replaces the reference's choice only when cheaper
       const LV w2 = X::gen([&](int l) {
         Real v = P.warm2[clampi(l, nv)];
         return l < nv ? v : 0.0;
       });
-      Real c2 = cost(w2, a0);
-      if (c2 < (c1 < c0 ? c1 : c0)) a = w2;
+      LV mt2, jar2;
+      const Real c2 = cost(w2, a0, &mt2, &jar2);
+      if (c2 < (take ? c1 : c0)) {
+        a = w2;
+        mt_a = mt2;
+        jar_s = jar2;
+      }
     }
   }
   const LV ma0 = mul_m(a0);
   const Real scale = 1.0 + sqrt_cr((lsum_lanes<X, NM>(ma0 * ma0, nv, -0.0)));
-  const Real tol = M.tolerance;
-  const int cap = M.iterations > 1 ? M.iterations : 1;
+  const Real tol = P.tol;
+  const int cap = P.cap;
   uint64_t prev = ~(uint64_t)0;
   int iters = 0;
   // residuals and active set at the current a, kept for the final force while a is unchanged
@@ -1032,12 +1068,13 @@ PHD int newton_lanes(const MT& M, const NP& P) {
   while (iters < cap) {
     iters++;
     const LV tmp = a - a0;
-    const LV jar = jdot(a) - aref;
+    const bool first = iters == 1;
+    const LV jar = first ? jar_s : jdot(a) - aref;
     const uint32_t act = active_mask(jar);
     jar_a = jar;
     act_a = act;
     fresh = true;
-    const LV grad = add_rows(mul_m(tmp), dd * jar, act);
+    const LV grad = add_rows(first ? mt_a : mul_m(tmp), dd * jar, act);
     const Real gnorm = sqrt_cr((lsum_lanes<X, NM>(grad * grad, nv, -0.0)));
     if (gnorm < tol * scale || ((uint64_t)act == prev && iters > 1)) break;
     prev = act;
@@ -1069,8 +1106,8 @@ PHD int newton_lanes(const MT& M, const NP& P) {
     const LV p = solve_rows<X, NM>(h, lc, lii, -grad, nv);
     // exact line search along p (newton.rs:310-351)
     const LV mp = mul_m(p);
-    const Real mpp = (lsum_lanes<X, NM>(p * mp, nv, -0.0));
-    const Real mpg = (lsum_lanes<X, NM>(tmp * mp, nv, -0.0));
+    Real mpp, mpg;
+    lsum2_lanes<X, NM>(p * mp, tmp * mp, nv, -0.0, &mpp, &mpg);
     const LV jp = jdot(p);
     // Row r's terms, one row per lane: D_r jp_r v_r and D_r jp_r^2 when the
     // row is active at step al, v_r = jar_r + al jp_r; they are then added in
@@ -1081,8 +1118,8 @@ PHD int newton_lanes(const MT& M, const NP& P) {
     auto deriv = [&](Real al, Real* d1o, Real* d2o) {
       const LV v = jar + al * jp;
       auto on = [&](int l) { return l < nr && (l >= n_ineq || X::at(v, l) < 0.0); };
-      *d1o = X::template rowsum<GL>(X::sel(on, dq * v, X::splat(-0.0)), al * mpp + mpg);
-      *d2o = X::template rowsum<GL>(X::sel(on, dq2, X::splat(-0.0)), mpp);
+      X::template rowsum2<GL>(X::sel(on, dq * v, X::splat(-0.0)), X::sel(on, dq2, X::splat(-0.0)), al * mpp + mpg, mpp,
+                              d1o, d2o);
     };
     Real lo = 0.0, hi = INFINITY, al = 1.0, d1, d2;
     deriv(0.0, &d1, &d2);
@@ -1119,6 +1156,17 @@ PHD int newton_lanes(const MT& M, const NP& P) {
   return iters;
 }
 
+template <class X, int NM>
+__host__ __device__ __attribute__((noinline)) int newton_lanes_call(NP P, LP J, LP aref, LP dd) {
+  return newton_lanes_body<X, NM>(P, J, aref, dd);
+}
+// out of line for run-time sizes, in line for a model-specialised kernel
+template <class X, int NM, class MT>
+PHD int newton_lanes(const MT&, const NP& P, LP J, LP aref, LP dd) {
+  if constexpr (std::is_same<MT, DModel>::value) return newton_lanes_call<X, NM>(P, J, aref, dd);
+  return newton_lanes_body<X, NM>(P, J, aref, dd);
+}
+
 // Lanes an env owns in executor X (0 for executors without lane groups).
 template <class X, class = void>
 struct wave_lanes {
@@ -1139,8 +1187,8 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 // l / 16 + 4, l / 16 + 8 and l / 16 + 12 of the tile. The fused multiply-adds and the summation order
 // differ from the reference's (d_r J_ri) J_rj added row by row, so results are
 // not bit-identical with it; used only when the sim asks for it.
-__device__ __noinline__ void hessian_mfma(const Real* qm, const Real* J, const Real* dd, const Real* act, int nr, int nv,
-                                          Real* H) {
+__device__ __noinline__ void hessian_mfma(const Real* qm, const Real* J, const Real* dd, const Real* jar, int n_ineq, int nr,
+                                          int nv, Real* H) {
   const int l = (int)threadIdx.x, c16 = l & 15, q = l >> 4;
   const int nt = (nv + 15) / 16;  // tiles per side (nv <= 64)
   for (int ti = 0; ti < nt; ti++) {
@@ -1149,7 +1197,7 @@ __device__ __noinline__ void hessian_mfma(const Real* qm, const Real* J, const R
     const int i = 16 * ti + c16;
     for (int s = 0; s < nr; s += 4) {
       const int r = s + q;
-      const bool on = r < nr && act[r] != 0.0;
+      const bool on = r < nr && (r >= n_ineq || jar[r] < 0.0);
       const Real a = (on && i < nv) ? dd[r] * J[(int64_t)r * nv + i] : 0.0;
       for (int tj = 0; tj < 4; tj++) {
         if (tj >= nt) break;
@@ -1170,178 +1218,265 @@ __device__ __noinline__ void hessian_mfma(const Real* qm, const Real* J, const R
 }
 #endif
 
-template <class X, class MT>
-PHD int newton_dense(const MT& M, Env& E, const NP& P) {
-  const int nv = P.nv, nr = P.nr;
-  Real* a = P.a;
-  Real* a0 = LD(a0);
-  Real* grad = LD(grad);
-  Real* p = LD(p);
-  Real* tmp = LD(tmp);
-  Real* tmp2 = LD(tmp2);
-  Real* mp = LD(mp);
-  Real* H = P.fac;
-  Real* sc = LD(scal);
-  int* isc = E.si + M.L.i_iscal;
-  const Real* qm = P.qm;
-  const Real* J = P.J;
-  Real* jar = E.jar;
-  Real* jp = E.jp;
-  Real* act = E.ract;
-  Real* prev = E.rprev;
+// start + x[0] + x[st] + ... + x[(n - 1) st], in that order, in every lane: the
+// loads of eight terms are issued before their adds.
+template <class P>
+PHD Real sum_in_order(P x, int st, int n, Real start) {
+  Real s = start;
+  int i = 0;
+  for (; i + 8 <= n; i += 8) {
+    Real v[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[k] = x[(i + k) * st];
+#pragma unroll
+    for (int k = 0; k < 8; k++) s = s + v[k];
+  }
+  for (; i < n; i++) s = s + x[i * st];
+  return s;
+}
+
+// Rows of a dense problem: J (nr x nv), targets, 1/R, J a - aref, J p, two
+// numbers per row of scratch, and the list of active rows (one double each).
+template <class P>
+struct RowsP {
+  P J, aref, dd, jar, jp, t, lst;
+};
+
+// newton_dense's dof vectors and a flag, in LDS.
+struct DenseVecs {
+  LP a0, grad, p, tmp, tmp2, mp;
+  LPI flag;
+  int mfma;  // the Hessian on the FP64 matrix cores
+};
+
+// math.rs:425-463 for an n x n matrix in LDS: n <= 16 one row per lane in
+// registers, else a lane per entry below the diagonal (chol_block's order).
+template <class X>
+PHD bool dense_chol(LP A, int n, LPI flag) {
+  if (n <= GL) {
+    const bool ok = chol_lanes<X>(A, n, 0, n);
+    X::sync();
+    return ok;
+  }
+  X::par(1, [&](int) { *flag = 0; });
+  for (int j = 0; j < n; j++) {
+    const LP rj = A + j * n;
+    // every entry of the column less its dot, then the root and the scaling
+    X::par(n - j, [&](int t) {
+      const int i = j + t;
+      const LP ri = A + i * n;
+      const Real d = ri[j] - sdot_n(ri, rj, j);
+      ri[j] = t == 0 ? (d <= 0.0 ? 0.0 : sqrt(d)) : d;
+      if (t == 0 && d <= 0.0) *flag = 1;
+    });
+    if (*flag) return false;
+    const Real inv = 1.0 / rj[j];
+    X::par(n - j - 1, [&](int t) { A[(j + 1 + t) * n + j] = A[(j + 1 + t) * n + j] * inv; });
+  }
+  return true;
+}
+template <class X>
+PHD void dense_solve(LP L, int n, LP x) {
+  if (n <= GL) {
+    solve_lanes<X>(L, n, 0, n, x);
+    X::sync();
+    return;
+  }
+  // forward: each lane's dot with the solved prefix would be in the same
+  // order on any lane, so the prefix is one lane's; the substitution upwards
+  // updates all entries above at once
+  X::par(1, [&](int) {
+    for (int i = 0; i < n; i++) x[i] = (x[i] - sdot_n(L + i * n, x, i)) / L[i * n + i];
+  });
+  for (int i = n - 1; i >= 0; i--) {
+    const Real xi = x[i] / L[i * n + i];
+    X::par(i + 1, [&](int k) { x[k] = k == i ? xi : x[k] + -xi * L[i * n + k]; });
+  }
+}
+
+// newton.rs:224-371 on the env's lanes, for any size. Sums over rows run in the
+// reference's order but never branch on a row: the terms of inactive rows are
+// -0.0 (which changes no sum), and products with J go over the list of active
+// rows, several rows' loads ahead of their adds. (With a branch per row, on
+// rows in HBM, the 92 rows of the arm's step took 300 us of its 523.) P: where
+// the rows are, LDS or anywhere.
+template <class X, class P, class QP>
+__host__ __device__ __attribute__((noinline)) int newton_dense(NPT<QP> Q, RowsP<P> R, DenseVecs D) {
+  const int nv = Q.nv, nr = Q.nr, n_ineq = Q.n_ineq;
+  const LP a = Q.a, a0 = D.a0, grad = D.grad, p = D.p, tmp = D.tmp, tmp2 = D.tmp2, mp = D.mp, H = Q.fac;
+  const QP qm = Q.qm;
+  const P J = R.J, aref = R.aref, dd = R.dd, jar = R.jar, jp = R.jp, t = R.t, lst = R.lst;
+  auto mul_m = [&](LP x, LP y) {
+    X::par(nv, [&](int i) { y[i] = sdot_n(qm + i * nv, x, nv) + 0.0 * x[i]; });
+  };
+  auto row_dots = [&](LP x, P out, bool minus_aref) {
+    X::par(nr, [&](int r) {
+      const Real v = sdot_n(J + r * nv, x, nv);
+      out[r] = minus_aref ? v - aref[r] : v;
+    });
+  };
+  auto sum_k = [&](LP x, LP y) {  // sum over dofs of x y
+    X::par(nv, [&](int k) { mp[k] = x[k] * y[k]; });
+    return sum_in_order(mp, 1, nv, rsum0());
+  };
   X::par(nv, [&](int k) { a0[k] = a[k]; });
-  const int nb = (nr + 63) / 64;
   // cost(x) = 1/2 (x-a0)'M(x-a0) + sum_active 1/2 D r^2 with r = J x - aref
-  auto cost_into = [&](const Real* x, int slot) {
+  auto cost = [&](LP x) {
     X::par(nv, [&](int k) { tmp[k] = x[k] - a0[k]; });
-    mul_m<X>(P, tmp, tmp2);
-    X::par(nr, [&](int r) { jar[r] = sdot_n(J + r * nv, x, nv) - P.aref[r]; });
-    X::par(1, [&](int) {
-      Real s = rsum0();
-      for (int k = 0; k < nv; k++) s += tmp[k] * tmp2[k];
-      Real c = 0.5 * s;
-      for (int r = 0; r < nr; r++) {
-        bool on = r >= P.n_ineq || jar[r] < 0.0;
-        if (on) c += 0.5 * P.dd[r] * jar[r] * jar[r];
+    mul_m(tmp, tmp2);
+    X::par(nr, [&](int r) {
+      const Real v = sdot_n(J + r * nv, x, nv) - aref[r];
+      t[r] = r >= n_ineq || v < 0.0 ? 0.5 * dd[r] * v * v : -0.0;
+    });
+    const Real c = 0.5 * sum_k(tmp, tmp2);
+    return sum_in_order(t, 1, nr, c);
+  };
+  // the active rows at jar, in order, into the list (their number returned),
+  // 16 per entry at the end of t; *same: as they were before
+  auto active_rows = [&](bool* same) {
+    int n = 0;
+    for (int c = 0; c < nr; c += GL) {
+      const uint32_t m = X::ballot([&](int l) {
+        const int r = clampi(c + l, nr);
+        return c + l < nr && (r >= n_ineq || jar[r] < 0.0);
+      });
+      const int at = 2 * nr - 1 - c / GL;
+      *same = *same && t[at] == (Real)m;
+      X::order();
+      X::each([&](int l) {
+        if ((m >> l) & 1u) lst[n + __builtin_popcount(m & ((1u << l) - 1u))] = (Real)(c + l);
+        if (l == 0) t[at] = (Real)m;
+      });
+      n += __builtin_popcount(m);
+    }
+    X::sync();
+    return n;
+  };
+  // g[k] + sum over the active rows, in order, of f_r J_rk, f_r = sign dd_r jar_r
+  auto add_rows = [&](bool from_g, LP g, Real sign, int na, LP out) {
+    X::par(na, [&](int i) {
+      const int r = (int)lst[i];
+      t[i] = sign * dd[r] * jar[r];
+    });
+    X::par(nv, [&](int k) {
+      Real s = from_g ? g[k] : 0.0;
+      int i = 0;
+      for (; i + 4 <= na; i += 4) {
+        Real v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = t[i + u] * J[(int)lst[i + u] * nv + k];
+#pragma unroll
+        for (int u = 0; u < 4; u++) s += v[u];
       }
-      sc[slot] = c;
+      for (; i < na; i++) s += t[i] * J[(int)lst[i] * nv + k];
+      out[k] = s;
     });
   };
   // warm start from the previous acceleration when cheaper (newton.rs:238-245)
-  const Real* warm = P.warm;
-  cost_into(a0, 0);
-  cost_into(warm, 1);
-  if (sc[1] < sc[0]) X::par(nv, [&](int k) { a[k] = warm[k]; });
-  if (P.warm2) {
+  const Real c0 = cost(a0), c1 = cost(Q.warm);
+  if (c1 < c0) X::par(nv, [&](int k) { a[k] = Q.warm[k]; });
+  if (Q.has_warm2) {
     // the learned candidate replaces the reference's choice only when cheaper
-    cost_into(P.warm2, 4);
-    if (sc[4] < (sc[1] < sc[0] ? sc[1] : sc[0])) X::par(nv, [&](int k) { a[k] = P.warm2[k]; });
+    const Real c2 = cost(Q.warm2);
+    if (c2 < (c1 < c0 ? c1 : c0)) X::par(nv, [&](int k) { a[k] = Q.warm2[k]; });
   }
-  mul_m<X>(P, a0, tmp);
-  X::par(1, [&](int) {
-    Real s = rsum0();
-    for (int k = 0; k < nv; k++) s += tmp[k] * tmp[k];
-    sc[2] = 1.0 + sqrt(s);  // scale
-  });
-  const Real scale = sc[2];
-  const Real tol = M.tolerance;
-  const int cap = M.iterations > 1 ? M.iterations : 1;
-  const int n_ineq = P.n_ineq;
-  X::par(nr, [&](int r) { prev[r] = -1.0; });  // u128::MAX sentinel
-  int iters = 0;
+  mul_m(a0, tmp);
+  const Real scale = 1.0 + sqrt(sum_k(tmp, tmp));
+  const Real tol = Q.tol;
+  const int cap = Q.cap;
+  int iters = 0, na = 0;
+  bool at_a = false;  // jar and the list belong to a
   while (iters < cap) {
     iters++;
     X::par(nv, [&](int k) { tmp[k] = a[k] - a0[k]; });
-    mul_m<X>(P, tmp, grad);
-    X::par(nr, [&](int r) {
-      Real v = sdot_n(J + r * nv, a, nv) - P.aref[r];
-      jar[r] = v;
-      bool on = r >= n_ineq || v < 0.0;
-      act[r] = on ? 1.0 : 0.0;
-      E.rf[r] = P.dd[r] * v;
-    });
-    X::par(nv, [&](int k) {
-      Real g = grad[k];
-      for (int r = 0; r < nr; r++)
-        if (act[r] != 0.0) g += E.rf[r] * J[r * nv + k];
-      grad[k] = g;
-    });
-    X::par(1, [&](int) {
-      Real s = rsum0();
-      for (int k = 0; k < nv; k++) s += grad[k] * grad[k];
-      Real gnorm = sqrt(s);
-      bool same = nr <= 128 && iters > 1;
-      if (same)
-        for (int r = 0; r < nr && r < 128; r++)
-          if (act[r] != prev[r]) {
-            same = false;
-            break;
-          }
-      isc[6] = (gnorm < tol * scale || same) ? 1 : 0;
-    });
-    if (isc[6]) break;
-    X::par(nr, [&](int r) { prev[r] = act[r]; });
+    mul_m(tmp, grad);
+    row_dots(a, jar, true);
+    bool same = nr <= 128 && iters > 1;
+    na = active_rows(&same);
+    at_a = true;
+    add_rows(true, grad, 1.0, na, grad);
+    const Real gnorm = sqrt(sum_k(grad, grad));
+    if (gnorm < tol * scale || same) break;
     bool on_mfma = false;
 #if defined(__HIP_DEVICE_COMPILE__)
     if constexpr (wave_lanes<X>::value == 64) {
-      if (M.hess_mfma && nv <= 64) {  // four 16-column tiles per row of tiles
-        hessian_mfma(qm, J, P.dd, act, nr, nv, H);
+      if (D.mfma && nv <= 64) {  // four 16-column tiles per row of tiles
+        hessian_mfma((const Real*)qm, (const Real*)J, (const Real*)dd, (const Real*)jar, n_ineq, nr, nv, (Real*)H);
         __syncthreads();
         on_mfma = true;
       }
     }
 #endif
-    // H = M + J_A' D J_A, entry-parallel, rows in order
-    if (!on_mfma) X::par(nv * nv, [&](int t) {
-      int i = t / nv, j = t % nv;
-      Real h = qm[t];
+    // H = M + J_A' D J_A, entry-parallel, rows in order; only the lower
+    // triangle, which is all that the factorisation reads
+    if (!on_mfma) X::par(nv * (nv + 1) / 2, [&](int e) {
+      int i = (int)((sqrtf(8.0f * (float)e + 1.0f) - 1.0f) * 0.5f);
+      while (i * (i + 1) / 2 > e) i--;
+      while ((i + 1) * (i + 2) / 2 <= e) i++;
+      const int j = e - i * (i + 1) / 2;
+      Real h = qm[i * nv + j];
       if (i == j) h += 0.0;
-      for (int r = 0; r < nr; r++) {
-        if (act[r] == 0.0) continue;
-        Real ji = J[r * nv + i];
-        if (ji == 0.0) continue;
-        h += (P.dd[r] * ji) * J[r * nv + j];
+      int n = 0;
+      for (; n + 4 <= na; n += 4) {
+        Real v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const int r = (int)lst[n + u];
+          v[u] = (dd[r] * J[r * nv + i]) * J[r * nv + j];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) h += v[u];
       }
-      H[t] = h;
+      for (; n < na; n++) {
+        const int r = (int)lst[n];
+        h += (dd[r] * J[r * nv + i]) * J[r * nv + j];
+      }
+      H[i * nv + j] = h;
     });
-    X::par(1, [&](int) { isc[1] = 0; });
-    if (!chol_block<X>(M, E, H, nv, 0, nv)) break;
+    if (!dense_chol<X>(H, nv, D.flag)) break;
     X::par(nv, [&](int k) { p[k] = -grad[k]; });
-    chol_solve_block<X>(M, E, H, nv, 0, nv, p);
+    dense_solve<X>(H, nv, p);
     // exact line search along p (newton.rs:310-351)
-    mul_m<X>(P, p, mp);
-    X::par(nr, [&](int r) { jp[r] = sdot_n(J + r * nv, p, nv); });
-    X::par(1, [&](int) {
-      Real mpp = rsum0(), mpg = rsum0();
-      for (int k = 0; k < nv; k++) mpp += p[k] * mp[k];
-      for (int k = 0; k < nv; k++) mpg += tmp[k] * mp[k];
-      auto deriv = [&](Real al, Real* d1o, Real* d2o) {
-        Real d1 = al * mpp + mpg, d2 = mpp;
-        for (int r = 0; r < nr; r++) {
-          Real v = jar[r] + al * jp[r];
-          if (r >= n_ineq || v < 0.0) {
-            Real dq = P.dd[r] * jp[r];
-            d1 += dq * v;
-            d2 += dq * jp[r];
-          }
-        }
-        *d1o = d1;
-        *d2o = d2;
-      };
-      Real lo = 0.0, hi = INFINITY, al = 1.0, d1, d2;
-      deriv(0.0, &d1, &d2);
-      Real ltol = 1e-12 * rmax(fabs(d1), 1e-30);
-      for (int it = 0; it < 50; it++) {
-        deriv(al, &d1, &d2);
-        if (fabs(d1) <= ltol) break;
-        if (d1 < 0.0) lo = al;
-        else hi = al;
-        Real next = al - d1 / rmax(d2, 1e-30);
-        if (next <= lo || next >= hi) next = rfinite(hi) ? 0.5 * (lo + hi) : 2.0 * rmax(al, lo);
-        if (fabs(next - al) <= 1e-14 * rmax(fabs(al), 1.0)) {
-          al = next;
-          break;
-        }
+    mul_m(p, tmp2);
+    row_dots(p, jp, false);
+    const Real mpp = sum_k(p, tmp2), mpg = sum_k(tmp, tmp2);
+    auto deriv = [&](Real al, Real* d1o, Real* d2o) {
+      X::par(nr, [&](int r) {
+        const Real v = jar[r] + al * jp[r], dq = dd[r] * jp[r];
+        const bool on = r >= n_ineq || v < 0.0;
+        t[r] = on ? dq * v : -0.0;
+        lst[r] = on ? dq * jp[r] : -0.0;
+      });
+      *d1o = sum_in_order(t, 1, nr, al * mpp + mpg);
+      *d2o = sum_in_order(lst, 1, nr, mpp);
+      X::sync();
+    };
+    Real lo = 0.0, hi = INFINITY, al = 1.0, d1, d2;
+    deriv(0.0, &d1, &d2);
+    const Real ltol = 1e-12 * rmax(fabs(d1), 1e-30);
+    for (int it = 0; it < 50; it++) {
+      deriv(al, &d1, &d2);
+      if (fabs(d1) <= ltol) break;
+      if (d1 < 0.0) lo = al;
+      else hi = al;
+      Real next = al - d1 / rmax(d2, 1e-30);
+      if (next <= lo || next >= hi) next = rfinite(hi) ? 0.5 * (lo + hi) : 2.0 * rmax(al, lo);
+      if (fabs(next - al) <= 1e-14 * rmax(fabs(al), 1.0)) {
         al = next;
+        break;
       }
-      sc[3] = al;
-    });
-    const Real al = sc[3];
+      al = next;
+    }
     X::par(nv, [&](int k) { a[k] += al * p[k]; });
+    at_a = false;
   }
-  (void)nb;
-  // add_constraint_force (newton.rs:361-371)
-  X::par(nr, [&](int r) {
-    Real v = sdot_n(J + r * nv, a, nv) - P.aref[r];
-    act[r] = (r >= n_ineq || v < 0.0) ? 1.0 : 0.0;
-    E.rf[r] = -P.dd[r] * v;
-  });
-  X::par(nv, [&](int k) {
-    Real f = 0.0;
-    for (int r = 0; r < nr; r++)
-      if (act[r] != 0.0) f += E.rf[r] * J[r * nv + k];
-    P.qf[k] = f;
-  });
+  // add_constraint_force (newton.rs:361-371), from zero, at the final a
+  if (!at_a) {
+    bool same = false;
+    row_dots(a, jar, true);
+    na = active_rows(&same);
+  }
+  add_rows(false, grad, -1.0, na, Q.qf);
   return iters;
 }
 
@@ -1355,13 +1490,19 @@ template <class X, class MT>
 PHD int newton_solve(const MT& M, const DState& S, Env& E, int nr, const Real* warm2) {
   const int nv = M.nv;
   const int n_ineq = nr - M.neq;
-  auto whole = [&]() {
-    if (nv <= GL && nr <= GL && nr <= M.nrl) {
-      NP P{nv, nr, n_ineq, LD(qm), LD(J), LD(aref), LD(dd), LD(qacc), LD(a), LD(qfrc_c), LD(chol), warm2};
-      return newton_lanes<X>(M, P);
-    }
-    NP P{nv, nr, n_ineq, LD(qm), E.J, E.aref, E.dd, LD(qacc), LD(a), LD(qfrc_c), LD(chol), warm2};
-    return newton_dense<X>(M, E, P);
+  const int cap = M.iterations > 1 ? M.iterations : 1;
+  const bool w2 = warm2 != nullptr;
+  const DenseVecs D{(LP)LD(a0), (LP)LD(grad), (LP)LD(p), (LP)LD(tmp), (LP)LD(tmp2), (LP)LD(mp),
+                    (LPI)(E.si + M.L.i_iscal + 1), M.hess_mfma};
+  // the model as one problem, in place
+  auto whole = [&]() __attribute__((always_inline)) {
+    const NP P{nv, nr, n_ineq, cap, M.tolerance, (LP)LD(qm), (LP)LD(qacc), (LP)LD(a), (LP)LD(qfrc_c), (LP)LD(chol),
+               (LP)LD(vel), w2};
+    if (nv <= GL && nr <= GL && nr <= M.nrl)
+      return newton_lanes<X, GL>(M, P, (LP)LD(J), (LP)LD(aref), (LP)LD(dd));
+    if (E.rows_lds)
+      return newton_dense<X>(P, RowsP<LP>{(LP)E.J, (LP)E.aref, (LP)E.dd, (LP)E.jar, (LP)E.jp, (LP)E.ract, (LP)E.rf}, D);
+    return newton_dense<X>(P, RowsP<GP>{(GP)E.J, (GP)E.aref, (GP)E.dd, (GP)E.jar, (GP)E.jp, (GP)E.ract, (GP)E.rf}, D);
   };
   if (M.nblock <= 1) return whole();
   // per-env island scratch: floats in HBM (islands of the register solver are
@@ -1423,7 +1564,7 @@ PHD int newton_solve(const MT& M, const DState& S, Env& E, int nr, const Real* w
   if (isl[nb] < 0) return whole();
   const int ni = isl[nb];
   // the dofs and rows of an island, in increasing order, by 16 lanes
-  auto list = [&](int id, int* dofs, int* rows, int* kn, int* qn, int* qin) {
+  auto list = [&](int id, int* dofs, int* rows, int* kn, int* qn, int* qin) __attribute__((always_inline)) {
     int k = 0, q = 0, qi = 0;
     for (int c = 0; c < nv; c += GL) {
       const uint32_t m = X::ballot([&](int l) { return c + l < nv && root[M.dof_block[clampi(c + l, nv)]] == id; });
@@ -1454,7 +1595,7 @@ PHD int newton_solve(const MT& M, const DState& S, Env& E, int nr, const Real* w
   // problem). One after the other, on 16 of the wavefront's 64 lanes, they
   // were 139 us of a 363 us step on the six-body pile, and gathering them 59.
   auto doubles = [](int k, int q) { return 2 * k * k + q * k + 2 * q + 4 * k; };
-  auto in_lanes = [&](int id) { return ik[id] <= GL && iq[id] <= GL && doubles(ik[id], iq[id]) <= nv * nv; };
+  auto in_lanes = [&](int id) __attribute__((always_inline)) { return ik[id] <= GL && iq[id] <= GL && doubles(ik[id], iq[id]) <= nv * nv; };
   int iters = 0;
   for (int next = 0; next < ni;) {
     // this row's island of the batch: the row()-th that fits after the ones
@@ -1482,24 +1623,17 @@ PHD int newton_solve(const MT& M, const DState& S, Env& E, int nr, const Real* w
       int* rows = dofs + ik[id];
       list(id, dofs, rows, &k, &q, &qi);
       X::order();
-      Real* fac = LD(chol) + o;
-      Real* sqm = fac + k * k;
-      Real* sJ = sqm + k * k;
-      Real* saref = sJ + q * k;
-      Real* sdd = saref + q;
-      Real* sa = sdd + q;
-      Real* swarm = sa + k;
-      Real* sqf = swarm + k;
-      Real* swarm2 = sqf + k;
+      const LP fac = (LP)LD(chol) + o, sqm = fac + k * k, sJ = sqm + k * k, saref = sJ + q * k, sdd = saref + q,
+               sa = sdd + q, swarm = sa + k, sqf = swarm + k, swarm2 = sqf + k;
       X::each([&](int l) {
         if (l < k) {
           const int d = dofs[l];
-          const Real* qm = LD(qm) + d * nv;
+          const LP qm = (LP)LD(qm) + d * nv;
           for (int i = 0; i < k; i++) sqm[l * k + i] = qm[dofs[i]];
           for (int t = 0; t < q; t++) sJ[t * k + l] = J[rows[t] * nv + d];
           sa[l] = LD(a)[d];
           swarm[l] = LD(qacc)[d];
-          if (warm2) swarm2[l] = warm2[d];
+          if (w2) swarm2[l] = warm2[d];
         }
         if (l < q) {
           saref[l] = E.aref[rows[l]];
@@ -1507,8 +1641,8 @@ PHD int newton_solve(const MT& M, const DState& S, Env& E, int nr, const Real* w
         }
       });
       X::order();
-      const NP P{k, q, qi, sqm, sJ, saref, sdd, swarm, sa, sqf, fac, warm2 ? swarm2 : nullptr};
-      it = kmax <= 6 ? newton_lanes<X, 6>(M, P) : newton_lanes<X>(M, P);
+      const NP P{k, q, qi, cap, M.tolerance, sqm, swarm, sa, sqf, fac, swarm2, w2};
+      it = kmax <= 6 ? newton_lanes<X, 6>(M, P, sJ, saref, sdd) : newton_lanes<X, GL>(M, P, sJ, saref, sdd);
       X::each([&](int l) {
         if (l < k) {
           LD(a)[dofs[l]] = sa[l];
@@ -1523,38 +1657,49 @@ PHD int newton_solve(const MT& M, const DState& S, Env& E, int nr, const Real* w
     for (int r = 0; r < X::ROWS; r++) iters = its[r] > iters ? its[r] : iters;
     X::sync();
   }
-  // larger islands, gathered into HBM, one after the other (newton_dense takes
-  // the vectors that hold the counts, so the islands done are struck out first)
+  // larger islands one after the other (newton_dense takes the vectors that
+  // hold the counts, so the islands done are struck out first), gathered into
+  // LDS when they fit: the mass-factor slot and, when this step's rows are
+  // elsewhere, the row block after it; else into HBM
   X::par(ni, [&](int i) {
     if (in_lanes(isl[i])) isl[i] = -1;
   });
+  const int64_t room = E.J == LD(J) ? (int64_t)nv * nv : (int64_t)M.L.rf + M.nrl - M.L.chol;
   for (int ii = 0; ii < ni; ii++) {
     const int id = isl[ii];
     if (id < 0) continue;
     int k, q, qi;
     list(id, sidx, sridx, &k, &q, &qi);
     X::sync();
-    Real* sqm = fs;
-    Real* sJ = sqm + nv * nv;
-    Real* saref = sJ + (int64_t)M.nrmax * nv;
-    Real* sdd = saref + M.nrmax;
-    Real* sa = sdd + M.nrmax;
-    Real* swarm = sa + nv;
-    Real* sqf = swarm + nv;
-    Real* swarm2 = sqf + nv;
-    X::par(k * k, [&](int t) { sqm[t] = LD(qm)[sidx[t / k] * nv + sidx[t % k]]; });
-    X::par(q * k, [&](int t) { sJ[t] = J[sridx[t / k] * nv + sidx[t % k]]; });
-    X::par(q, [&](int t) {
-      saref[t] = E.aref[sridx[t]];
-      sdd[t] = E.dd[sridx[t]];
-    });
+    // the dof vectors take slots that the step has used up (the forces summed in LD(smooth))
+    const LP sa = (LP)LD(acc), swarm = (LP)LD(bias), sqf = (LP)LD(passive), swarm2 = (LP)LD(qfrc_act), fac = (LP)LD(chol);
     X::par(k, [&](int t) {
-      sa[t] = LD(a)[sidx[t]];
-      swarm[t] = LD(qacc)[sidx[t]];
-      if (warm2) swarm2[t] = warm2[sidx[t]];
+      const int d = sidx[t];
+      sa[t] = LD(a)[d];
+      swarm[t] = LD(qacc)[d];
+      if (w2) swarm2[t] = warm2[d];
     });
-    NP P{k, q, qi, sqm, sJ, saref, sdd, swarm, sa, sqf, LD(chol), warm2 ? swarm2 : nullptr};
-    int it = (k <= GL && q <= GL) ? newton_lanes<X>(M, P) : newton_dense<X>(M, E, P);
+    auto solve = [&](auto sqm, auto sJ) __attribute__((always_inline)) {
+      typedef decltype(sJ) BP;
+      typedef decltype(sqm) MP;
+      const BP saref = sJ + (int64_t)q * k, sdd = saref + q;
+      X::par(k, [&](int t) {
+        const int d = sidx[t];
+        for (int i = 0; i < k; i++) sqm[t * k + i] = LD(qm)[d * nv + sidx[i]];
+      });
+      X::par(q, [&](int t) {
+        const int r = sridx[t];
+        for (int i = 0; i < k; i++) sJ[t * k + i] = J[r * nv + sidx[i]];
+        saref[t] = E.aref[r];
+        sdd[t] = E.dd[r];
+      });
+      const NPT<MP> P{k, q, qi, cap, M.tolerance, sqm, swarm, sa, sqf, fac, swarm2, w2};
+      return newton_dense<X>(P, RowsP<BP>{sJ, saref, sdd, sdd + q, sdd + 2 * q, sdd + 3 * q, sdd + 5 * q}, D);
+    };
+    const int64_t rows_at = 2 * (int64_t)k * k;
+    int it;
+    if (rows_at + (int64_t)q * (k + 7) <= room) it = solve(fac + k * k, fac + rows_at);
+    else it = solve((GP)fs, (GP)(fs + nv * nv));
     iters = it > iters ? it : iters;
     X::par(k, [&](int t) {
       LD(a)[sidx[t]] = sa[t];
@@ -2284,7 +2429,7 @@ PHD int pgs_prepare_packed(const MT& M, const DState& S, Env& E, Real* v, Real* 
   const int ncon = isc[0];
   const PgsConsts C = pgs_consts(M);
   int* coff = reinterpret_cast<int*>(LD(cact));  // per contact: entries of its J rows, then their offset
-  auto span_of = [&](int c, PgsRow* r) {
+  auto span_of = [&](int c, PgsRow* r) __attribute__((always_inline)) {
     const int d1 = M.body_lastdof[M.geom_body[cg[3 * c]]], d2 = M.body_lastdof[M.geom_body[cg[3 * c + 1]]];
     pgs_span(M, d1 < 0 ? -1 : M.dof_block[d1], d2 < 0 ? -1 : M.dof_block[d2], r);
   };

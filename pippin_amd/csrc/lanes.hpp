@@ -108,6 +108,29 @@ struct DevLanes {
 #undef PH_ROWSUM
     return s;
   }
+  // two row sums side by side: their chains fill each other's latency (a
+  // dependent v_fmac_f64 issues every 7.3 cycles, independent ones every 5.2)
+  template <int N>
+  __device__ __forceinline__ static void rowsum2(DLV x, DLV y, Real sx, Real sy, Real* ox, Real* oy) {
+    Real s = sx, t = sy;
+    const Real one = 1.0;
+#define PH_ROWSUM2(k)                                                               \
+  "v_fmac_f64_dpp %0, %2, %4 row_newbcast:" #k " row_mask:0xf bank_mask:0xf\n\t"    \
+  "v_fmac_f64_dpp %1, %3, %4 row_newbcast:" #k " row_mask:0xf bank_mask:0xf\n\t"
+    if constexpr (N == 6) {
+      asm("s_nop 1\n\t" PH_ROWSUM2(0) PH_ROWSUM2(1) PH_ROWSUM2(2) PH_ROWSUM2(3) PH_ROWSUM2(4) PH_ROWSUM2(5)
+          : "+&v"(s), "+&v"(t) : "v"(x.v), "v"(y.v), "v"(one));
+    } else {
+      static_assert(N == GL, "row sums of 6 or 16 lanes");
+      asm("s_nop 1\n\t" PH_ROWSUM2(0) PH_ROWSUM2(1) PH_ROWSUM2(2) PH_ROWSUM2(3) PH_ROWSUM2(4) PH_ROWSUM2(5)
+          PH_ROWSUM2(6) PH_ROWSUM2(7) PH_ROWSUM2(8) PH_ROWSUM2(9) PH_ROWSUM2(10) PH_ROWSUM2(11)
+          PH_ROWSUM2(12) PH_ROWSUM2(13) PH_ROWSUM2(14) PH_ROWSUM2(15)
+          : "+&v"(s), "+&v"(t) : "v"(x.v), "v"(y.v), "v"(one));
+    }
+#undef PH_ROWSUM2
+    *ox = s;
+    *oy = t;
+  }
   // p |= v and p += v by several lanes
   __device__ __forceinline__ static void ior(int* p, int v) { atomicOr(p, v); }
   __device__ __forceinline__ static void iadd(int* p, int v) { atomicAdd(p, v); }
@@ -210,6 +233,11 @@ struct HostLanes {
     for (int l = 0; l < N; l++) s = s + x.v[l];
     return s;
   }
+  template <int N>
+  static void rowsum2(const HLV& x, const HLV& y, Real sx, Real sy, Real* ox, Real* oy) {
+    *ox = rowsum<N>(x, sx);
+    *oy = rowsum<N>(y, sy);
+  }
   static void order() {}
   static void ior(int* p, int v) { *p |= v; }
   static void iadd(int* p, int v) { *p += v; }
@@ -306,6 +334,12 @@ PHD Real lsum_lanes(LV x, int n, Real start) {
   return X::template rowsum<NM>(X::sel([&](int l) { return l < n; }, x, X::splat(-0.0)), start);
 }
 
+template <class X, int NM = GL, class LV>
+PHD void lsum2_lanes(LV x, LV y, int n, Real start, Real* ox, Real* oy) {
+  X::template rowsum2<NM>(X::sel([&](int l) { return l < n; }, x, X::splat(-0.0)),
+                          X::sel([&](int l) { return l < n; }, y, X::splat(-0.0)), start, start, ox, oy);
+}
+
 // math.rs:425-447 with one row per lane: in-place lower Cholesky of the
 // diagonal block [s0, s0 + n) (n <= 16) of the row-major stride-nv matrix A.
 // Column j: lanes receive row j (entries < j) by broadcast, each lane forms its
@@ -337,8 +371,8 @@ PHD bool chol_rows(LV* r, int n) {
 
 // Store the lower triangle (with the diagonal) of register rows into the
 // diagonal block [s0, s0 + n) of A.
-template <class X, int NM = GL, class LV>
-PHD void store_lower(const LV* r, Real* A, int nv, int s0, int n) {
+template <class X, int NM = GL, class LV, class AP>
+PHD void store_lower(const LV* r, AP A, int nv, int s0, int n) {
   X::each([&](int l) {
     if (l < n) {
 #pragma unroll
@@ -348,8 +382,8 @@ PHD void store_lower(const LV* r, Real* A, int nv, int s0, int n) {
   });
 }
 
-template <class X>
-PHD bool chol_lanes(Real* A, int nv, int s0, int n) {
+template <class X, class AP>
+PHD bool chol_lanes(AP A, int nv, int s0, int n) {
   using LV = typename X::LV;
   LV r[GL];
 #pragma unroll
@@ -390,8 +424,8 @@ PHD LV solve_rows(const LV* r, const LV* c, LV lii, LV xv, int n) {
 
 // Load, for lane l, row l of the strict lower triangle (r), column l below the
 // diagonal (c) and the diagonal entry of the factor in block [s0, s0 + n).
-template <class X, int NM = GL, class LV>
-PHD void load_factor(const Real* L, int nv, int s0, int n, LV* r, LV* c, LV* lii) {
+template <class X, int NM = GL, class LV, class AP>
+PHD void load_factor(AP L, int nv, int s0, int n, LV* r, LV* c, LV* lii) {
 #pragma unroll
   for (int k = 0; k < NM; k++) {
     r[k] = X::gen([&](int l) {
@@ -410,8 +444,8 @@ PHD void load_factor(const Real* L, int nv, int s0, int n, LV* r, LV* c, LV* lii
   });
 }
 
-template <class X>
-PHD void solve_lanes(const Real* L, int nv, int s0, int n, Real* x) {
+template <class X, class AP, class XP>
+PHD void solve_lanes(AP L, int nv, int s0, int n, XP x) {
   using LV = typename X::LV;
   LV r[GL], c[GL], lii;
   load_factor<X>(L, nv, s0, n, r, c, &lii);

@@ -34,12 +34,12 @@ static void emit(const char* name, const phk::DModel& M) {
   printf("struct %s : DModel {\n", name);
 #define SZ(f) printf("  static constexpr int " #f " = %d;\n", M.f);
   SZ(nq) SZ(nv) SZ(nu) SZ(nbody) SZ(njnt) SZ(ngeom) SZ(ncam) SZ(neq) SZ(npair) SZ(nlevel) SZ(nblock) SZ(nacc)
-  SZ(integrator) SZ(solver_kind) SZ(iterations) SZ(ncmax) SZ(nrmax) SZ(nrl) SZ(ngeneral)
+  SZ(integrator) SZ(solver_kind) SZ(iterations) SZ(ncmax) SZ(nrmax) SZ(nrl) SZ(ngeneral) SZ(bmax)
 #undef SZ
   printf("  static constexpr Layout L = %s_layout;\n", name);
   printf("  static bool matches(const DModel& m) {\n    return ");
   const char* f[] = {"nq", "nv", "nu", "nbody", "njnt", "ngeom", "ncam", "neq", "npair", "nlevel", "nblock", "nacc",
-                     "integrator", "solver_kind", "iterations", "ncmax", "nrmax", "nrl", "ngeneral"};
+                     "integrator", "solver_kind", "iterations", "ncmax", "nrmax", "nrl", "ngeneral", "bmax"};
   for (const char* x : f) printf("m.%s == %s && ", x, x);
   printf("layout_equal(m.L, %s_layout);\n  }\n};\n\n", name);
 }
