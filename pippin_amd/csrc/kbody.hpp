@@ -3022,6 +3022,12 @@ PHD void set_const_env(const MT& M, Env& E, Real* dof_iw, Real* body_iw) {
 // ---------------- per-env driver (shared by the kernels and the serial policy) ----------------
 enum { IS_NCON = 0, IS_STATUS = 7, IS_ITERS = 8, IS_NROWS = 9 };
 
+// Tells the host that an env of the launch cannot be stepped; the envs' own
+// status words say which.
+PHD void report_failure(const DState& S, int status) {
+  if (status != 0 && S.failed.p) S.failed[0] = 1;
+}
+
 template <class X, class MT>
 PHD void load_state(const MT& M, const DState& S, Env& E) {
   Real* s = E.s;
@@ -3080,6 +3086,7 @@ PHD void run_env(const MT& M, const DState& S, Env& E, int64_t nstep, const Real
   X::par(1, [&](int) {
     S.ncon[e] = isc[IS_NCON];
     S.status[e] = isc[IS_STATUS];
+    report_failure(S, isc[IS_STATUS]);
     S.iters[e] = isc[IS_ITERS];
     S.nrows[e] = isc[IS_NROWS];
     S.cost[e] = cost;
@@ -3153,6 +3160,7 @@ PHD void run_pgs_back(const MT& M, const DState& S, Env& E, int64_t nstep, int64
     X::par(1, [&](int) {
       S.cost[e] = 0;
       S.time[e] += (Real)nstep * M.timestep;
+      report_failure(S, status);
     });
 }
 
@@ -3436,6 +3444,7 @@ PHD void run_env_mlp(const MT& M, const DState& S, Env& E, int64_t nstep, const 
   X::par(1, [&](int) {
     S.ncon[e] = isc[IS_NCON];
     S.status[e] = isc[IS_STATUS];
+    report_failure(S, isc[IS_STATUS]);
     S.iters[e] = isc[IS_ITERS];
     S.nrows[e] = isc[IS_NROWS];
     S.time[e] += (Real)nstep * M.timestep;

@@ -4,6 +4,7 @@
 // LDS; per-env state, contacts and large row buffers in HBM. The C entry points
 // follow the `Physics` trait (crates/pippin-env/src/lib.rs:110-155) and the CPU
 // backend's conventions (crates/pippin-env/src/pippin_cpu.rs).
+#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -120,6 +121,12 @@ __global__ void __launch_bounds__(64) k_mass_bias(const DModel* __restrict__ Mp,
   DevX::par(M.nv, [&](int k) { bias[rel * M.nv + k] = lds[M.L.bias + k]; });
 }
 
+// n doubles from src to dst, where one of them is pinned host memory.
+__global__ void __launch_bounds__(256) k_copy(const Real* src, Real* dst, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) dst[i] = src[i];
+}
+
 // set_const for listed variants.
 __global__ void __launch_bounds__(64) k_setconst(const DModel* __restrict__ Mp, const int* vars, Real* dof_iw,
                                                  Real* body_iw) {
@@ -210,6 +217,27 @@ static const void* pgs_rows_kernel(const DModel& M) {
   return M.pgs_w <= 12 ? (const void*)k_pgs_sweeps_rows<12, false> : (const void*)k_pgs_sweeps_rows<16, false>;
 }
 
+// Pinned host memory of a sim: the failure flag the step kernels write, and
+// staging for small get and set calls, whose copies are kernels on the sim's
+// stream. (A blocking copy to or from pageable memory took 12 to 20 us of the
+// 125 us of a host-driven step of one env.)
+struct Pinned {
+  static constexpr size_t STAGE = 256 * 1024;  // bytes; larger calls copy directly
+  char* p = nullptr;
+  size_t used = 0;  // staging bytes whose copies may still be in flight
+  std::mutex mu;    // held while the staging is in use: get may be called from several threads
+  ~Pinned() {
+    if (p) (void)hipHostFree(p);
+  }
+  hipError_t alloc() {
+    hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&p), 256 + STAGE, hipHostMallocDefault);
+    if (e == hipSuccess) *failed() = 0;
+    return e;
+  }
+  volatile int* failed() const { return reinterpret_cast<volatile int*>(p); }
+  double* stage() const { return reinterpret_cast<double*>(p + 256); }
+};
+
 struct Variants {
   // host mirrors, [nvar][...]
   std::vector<double> geom_size, geom_aabb, friction, body_mass, body_ipos, body_inertia, dof_damping, act_gain,
@@ -262,6 +290,8 @@ struct ph_sim {
   DBuf<double> d_pgs_vel, d_pgs_vpos;
   DBuf<int> d_cam_body;
   DBuf<double> d_cam_pos, d_cam_quat;
+  mutable Pinned pin;
+  bool state_shared = false;  // a device pointer to state was handed out: set() returns with its copy done
   bool qpos_shared = false;  // a device qpos pointer was handed out (pippin_hip_state_device)
   hipStream_t stream = nullptr;
   DModel M;
@@ -425,6 +455,7 @@ extern "C" int pippin_hip_create(const ph_model_desc* desc, int64_t num_envs, co
   HIPCHK(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking));
   HIPCHK(hipEventCreate(&s->ev0));
   HIPCHK(hipEventCreate(&s->ev1));
+  HIPCHK(s->pin.alloc());
 
   DModel& M = s->M;
   phh::init_dmodel_scalars(hm, solver, opt ? opt->max_contacts : 0, M);
@@ -622,6 +653,7 @@ extern "C" int pippin_hip_create(const ph_model_desc* desc, int64_t num_envs, co
   S.nrows = s->s_nrows.p;
   S.status = s->s_status.p;
   S.cost = s->s_cost.p;
+  S.failed = reinterpret_cast<int*>(s->pin.p);
   S.con = s->s_con.p;
   S.cgeom = s->s_cgeom.p;
   S.pcon = s->s_pcon.p;
@@ -742,7 +774,8 @@ static int split_envs_per_wave(const ph_sim* s, int64_t envs) {
 // optional per-step controls and qpos outputs (Batch::rollout). Only kernels
 // go on the stream, so the sequence can be captured in a graph.
 static hipError_t launch_plain(ph_sim* s, const ph_launch_shape& sh, int64_t begin, int64_t end, int64_t nstep,
-                               const Real* ctrl = nullptr, Real* qpos_out = nullptr) {
+                               const Real* ctrl = nullptr, Real* qpos_out = nullptr, hipEvent_t start = nullptr,
+                               hipEvent_t stop = nullptr) {
   const int K = sh.envs_per_wave, spec = sh.specialised;
   const size_t lds = step_lds(s, K);
   const DModel* mp = s->d_model.p;
@@ -780,6 +813,8 @@ static hipError_t launch_plain(ph_sim* s, const ph_launch_shape& sh, int64_t beg
   if (sh.schedule == PH_SCHED_GRID) {
     const unsigned grid = (unsigned)((end - begin + K - 1) / K);
     void* args[] = {&mp, &sp, &begin, &end, &nstep, &ctrl, &qpos_out};
+    if (start)  // timed by the dispatch itself
+      return hipExtLaunchKernel(step_kernel(K, spec), dim3(grid), dim3(64), args, lds, s->stream, start, stop, 0);
     return hipLaunchKernel(step_kernel(K, spec), dim3(grid), dim3(64), args, lds, s->stream);
   }
   int* order = nullptr;
@@ -1001,16 +1036,25 @@ static int timed_launch(ph_sim* s, int64_t begin, int64_t end, int64_t nstep, co
   const bool plain = !s->M.mlp.mode;
   const bool trial = plain && s->tune_rounds > 0 && nstep > 0;
   const ph_launch_shape sh = trial ? s->tune_cand[s->tune_next] : current_shape(s);
-  HIPCHK(hipEventRecord(s->ev0, s->stream));
-  if (!plain) HIPCHK(launch_step(s, begin, end, nstep, ctrl, qpos_out));
-  else if (s->use_graphs && !trial && !ctrl && !qpos_out) {
-    if (int rc = launch_plain_graph(s, sh, begin, end, nstep)) return rc;
-  } else
-    HIPCHK(launch_plain(s, sh, begin, end, nstep, ctrl, qpos_out));
+  *s->pin.failed() = 0;
+  // the grid schedule is one launch, which carries its own time stamps; a
+  // sequence is replayed from a graph between two event records
+  const bool one = plain && sh.schedule == PH_SCHED_GRID;
+  if (one) {
+    HIPCHK(launch_plain(s, sh, begin, end, nstep, ctrl, qpos_out, s->ev0, s->ev1));
+  } else {
+    HIPCHK(hipEventRecord(s->ev0, s->stream));
+    if (!plain) HIPCHK(launch_step(s, begin, end, nstep, ctrl, qpos_out));
+    else if (s->use_graphs && !trial && !ctrl && !qpos_out) {
+      if (int rc = launch_plain_graph(s, sh, begin, end, nstep)) return rc;
+    } else
+      HIPCHK(launch_plain(s, sh, begin, end, nstep, ctrl, qpos_out));
+  }
   s->poses_stale = true;
   HIPCHK(hipGetLastError());
-  HIPCHK(hipEventRecord(s->ev1, s->stream));
+  if (!one) HIPCHK(hipEventRecord(s->ev1, s->stream));
   HIPCHK(hipStreamSynchronize(s->stream));
+  s->pin.used = 0;
   float ms = 0.0f;
   HIPCHK(hipEventElapsedTime(&ms, s->ev0, s->ev1));
   s->kernel_ms += ms;
@@ -1022,7 +1066,7 @@ static int timed_launch(ph_sim* s, int64_t begin, int64_t end, int64_t nstep, co
       if (++s->tune_round == s->tune_rounds) tune_finish(s);
     }
   }
-  return status_of(s, begin, end);
+  return nstep == 0 || *s->pin.failed() ? status_of(s, begin, end) : PH_OK;
 }
 
 extern "C" int pippin_hip_step(ph_sim* s, int64_t begin, int64_t end, int64_t nstep) {
@@ -1067,6 +1111,13 @@ extern "C" int pippin_hip_state_device(ph_sim* s, int32_t field, double** ptr) {
   // the caller may write qpos through the pointer at any time from now on,
   // so poses are recomputed on every poses() call
   if (field == PH_FIELD_QPOS) s->qpos_shared = true;
+  if (*ptr) {
+    s->state_shared = true;
+    if (s->pin.used) {  // copies staged before are done when the pointer is out
+      HIPCHK(hipStreamSynchronize(s->stream));
+      s->pin.used = 0;
+    }
+  }
   return *ptr ? PH_OK : fail(PH_ERR_ARG, "unknown field");
 }
 
@@ -1080,6 +1131,19 @@ extern "C" int pippin_hip_get(const ph_sim* s, int32_t field, int64_t begin, int
   if (w < 0) return fail(PH_ERR_ARG, "unknown field");
   if (int rc = check_len("get", len, end - begin, w)) return rc;
   if (w == 0 || end == begin) return PH_OK;
+  const int64_t count = (end - begin) * w;
+  if ((size_t)count * sizeof(double) <= Pinned::STAGE) {
+    HIPCHK(hipSetDevice(s->device));
+    std::lock_guard<std::mutex> lock(s->pin.mu);
+    if (s->pin.used) HIPCHK(hipStreamSynchronize(s->stream));  // the staging of set calls
+    hipLaunchKernelGGL(k_copy, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s->stream, d + begin * w,
+                       s->pin.stage(), count);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(s->stream));
+    s->pin.used = 0;
+    memcpy(out, s->pin.stage(), count * sizeof(double));
+    return PH_OK;
+  }
   // copies queued by set_device run on the library stream, which the null
   // stream does not wait for
   HIPCHK(hipStreamSynchronize(s->stream));
@@ -1094,7 +1158,28 @@ extern "C" int pippin_hip_set(ph_sim* s, int32_t field, int64_t begin, int64_t e
   if (w < 0) return fail(PH_ERR_ARG, "unknown field");
   if (int rc = check_len("set", len, end - begin, w)) return rc;
   if (w == 0 || end == begin) return PH_OK;
+  const size_t bytes = (size_t)(end - begin) * w * sizeof(double);
+  if (bytes <= Pinned::STAGE && !s->state_shared) {
+    // staged, and copied in order with the stream's other work: only pointers
+    // that the sim handed out could see the state before that
+    HIPCHK(hipSetDevice(s->device));
+    std::lock_guard<std::mutex> lock(s->pin.mu);
+    if (s->pin.used + bytes > Pinned::STAGE) {
+      HIPCHK(hipStreamSynchronize(s->stream));
+      s->pin.used = 0;
+    }
+    double* stage = s->pin.stage() + s->pin.used / sizeof(double);
+    memcpy(stage, src, bytes);
+    s->pin.used += bytes;
+    const int64_t count = (end - begin) * w;
+    hipLaunchKernelGGL(k_copy, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s->stream, stage, d + begin * w,
+                       count);
+    HIPCHK(hipGetLastError());
+    if (field == PH_FIELD_QPOS) s->poses_stale = true;
+    return PH_OK;
+  }
   HIPCHK(hipStreamSynchronize(s->stream));  // a pending set_device copy must not overwrite this one
+  s->pin.used = 0;
   HIPCHK(hipMemcpy(d + begin * w, src, (end - begin) * w * sizeof(double), hipMemcpyHostToDevice));
   if (field == PH_FIELD_QPOS) s->poses_stale = true;
   return PH_OK;

@@ -261,6 +261,7 @@ emu_sim* emu_create(const ph_model_desc* desc, int64_t n) {
   S.nrows = s->nrows.data();
   S.status = s->status.data();
   S.cost = s->cost.data();
+  S.failed = nullptr;
   S.con = s->con.data();
   S.cgeom = s->cgeom.data();
   S.pcon = s->pcon.data();
