@@ -184,8 +184,8 @@ __device__ __noinline__ void pgs_sweeps_general(const DModel* Mp, const DState* 
 // and every instruction and branch counts: the terms that stay fixed over a
 // phase are formed when the phase begins, normal and friction rows share one
 // expression (a friction row's bias and impulse scale are 0, a normal row's
-// friction coefficient 0 and its upper bound infinite), the next row's entries
-// and the record after it are in flight during an update. The four 16-lane
+// friction coefficient 0 and its upper bound infinite), the row's record and
+// the next row's entries are in flight during the sum. The four 16-lane
 // rows advance independently, each from row to row, sweep to sweep and env to
 // env (counter, cleared by k_pgs_front), so none waits for another's longer
 // solve. The expression needs finite velocities and forces; an env that has
@@ -221,34 +221,28 @@ __global__ void __launch_bounds__(64) k_pgs_sweeps_rows(const DModel* __restrict
   int nr = 0, Jb = 0, mo = 0;  // byte address of the J entries, and from there to the M^-1 J^T entries
   int phase = 0, it = 0, r = 0, limit = 0;
   bool moved = false;
-  Real c0 = 0.0, bias = 0.0, is = 0.0, mu = 0.0, lam = 0.0, j = 0.0, m = 0.0;  // the current row
-  Real nc0 = 0.0, nbias = 0.0, nis = 0.0, nmu = 0.0;                          // the next one
-  int lo_w = 0, hi_w = 0, nlo = 0, nhi = 0;                                    // their INFO words
-  int va = spare;
-  auto after = [&](int i) { return i + 1 < nr ? i + 1 : 0; };
+  // the current row: its record, its J entry here and that entry's address, the
+  // velocity it meets, the INFO word
+  int ra = recb, ja = 0, va = spare, hi_w = 0;
+  Real j = 0.0;
   auto count_of = [](int hi) { return (hi >> 21) & 31; };
-  auto v_addr = [&](int lo, int hi) {  // this lane's velocity; a spare slot past the row's entries
+  auto v_addr = [&](int lo, int hi) {  // a spare slot past the row's entries
     const int base = l < ((hi >> 16) & 31) ? lo & 0xFFFF : (int)((unsigned)lo >> 16);
     return l < count_of(hi) ? base + l8 : spare;
   };
-  auto info = [&](int i, int* lo, int* hi) {
-    const int64_t w = *(__attribute__((address_space(3))) int64_t*)(lb + recb + i * RB + INFO);
+  auto info = [&](int a, int* lo, int* hi) {
+    const int64_t w = *(__attribute__((address_space(3))) int64_t*)(lb + a + INFO);
     *lo = (int)w;
     *hi = (int)(w >> 32);
   };
-  auto start = [&](int i) {  // fill the pipeline at row i
-    int a = recb + i * RB;
-    c0 = ld(a + C0), bias = ld(a + BIAS), is = ld(a + IS), mu = ld(a + MU), lam = ld(a + LAM);
-    info(i, &lo_w, &hi_w);
-    va = v_addr(lo_w, hi_w);
-    const bool in = l < count_of(hi_w);
-    j = ld(Jb + (hi_w & 0xFFFF) * 8 + l8);
-    m = ld(Jb + mo + (hi_w & 0xFFFF) * 8 + l8);
-    j = in ? j : 0.0;
-    m = in ? m : 0.0;
-    a = recb + after(i) * RB;
-    nc0 = ld(a + C0), nbias = ld(a + BIAS), nis = ld(a + IS), nmu = ld(a + MU);
-    info(after(i), &nlo, &nhi);
+  auto start = [&]() {  // the first row
+    int lo;
+    ra = recb;
+    info(ra, &lo, &hi_w);
+    va = v_addr(lo, hi_w);
+    ja = Jb + (hi_w & 0xFFFF) * 8 + l8;
+    j = ld(ja);
+    j = l < count_of(hi_w) ? j : 0.0;
   };
   auto records = [&](int ph) {  // the rows' terms in phase ph
     auto rw = S.grow + e * (int64_t)M.nrmax * 10;
@@ -262,11 +256,13 @@ __global__ void __launch_bounds__(64) k_pgs_sweeps_rows(const DModel* __restrict
       st(a + IS, soft && !fixed ? C.impulse_scale : 0.0);
       st(a + MU, friction && !fixed ? b1 : 0.0);
       // lo: addresses of entry 0 of the lower block and of entry na of the
-      // upper one less its place; hi: offset 16, na 5, entries 5, sub 2,
-      // bilateral 1, unbounded above 1 (sign)
+      // upper one less its place; hi: offset 16 bits, na 5, entries 5,
+      // bilateral, unbounded above, and in 16 bytes the way back to the
+      // contact's normal row's record 4
       const unsigned alo = (unsigned)(vb + 8 * w.a), blo = (unsigned)(vb + 8 * (w.count > w.na ? w.b - w.na : 0));
-      const unsigned hi = (unsigned)w.off | (unsigned)w.na << 16 | (unsigned)w.count << 21 | (unsigned)w.sub << 26 |
-                          (w.kind == PK_BILATERAL ? 1u << 28 : 0u) | (!friction || fixed ? 1u << 31 : 0u);
+      const unsigned hi = (unsigned)w.off | (unsigned)w.na << 16 | (unsigned)w.count << 21 |
+                          (w.kind == PK_BILATERAL ? 1u << 26 : 0u) | (!friction || fixed ? 1u << 27 : 0u) |
+                          (unsigned)(w.sub * (RB / 16)) << 28;
       *(__attribute__((address_space(3))) int64_t*)(lb + a + INFO) = (int64_t)((uint64_t)hi << 32 | blo << 16 | alo);
     }
     X::order();
@@ -331,58 +327,55 @@ __global__ void __launch_bounds__(64) k_pgs_sweeps_rows(const DModel* __restrict
         continue;
       }
       records(0);
-      start(0);
+      start();
     }
     if (__ballot(live) == 0) break;
     if (live) {
-      const int rn = after(r), rnn = after(rn);
-      const Real vv = ld(va);
-      const Real lam_n = ld(recb + (r - ((hi_w >> 26) & 3)) * RB + LAM);
-      // the next row's entries, and the record of the one after
-      const int off = (nhi & 0xFFFF) * 8 + l8, a2 = recb + rnn * RB;
-      Real nj = ld(Jb + off), nm = ld(Jb + mo + off);
-      const Real xc0 = ld(a2 + C0), xbias = ld(a2 + BIAS), xis = ld(a2 + IS), xmu = ld(a2 + MU);
-      int xlo, xhi;
-      info(rnn, &xlo, &xhi);
-      const int nva = v_addr(nlo, nhi);
+      // what the update needs, on its way during the sum; then the next row
+      const Real vv = ld(va), c0 = ld(ra + C0), bias = ld(ra + BIAS), is = ld(ra + IS), mu = ld(ra + MU);
+      const Real lam = ld(ra + LAM), lam_n = ld(ra - (int)(((unsigned)hi_w >> 28) << 4) + LAM), mr = ld(ja + mo);
+      const bool last = r + 1 == nr;
+      const int rb = last ? recb : ra + RB;
+      int nlo, nhi;
+      info(rb, &nlo, &nhi);
       const Real jv = X::template rowsum<W>(DLV{j * vv}, rsum0());
+      const int nja = Jb + (nhi & 0xFFFF) * 8 + l8, nva = v_addr(nlo, nhi);
+      const Real nj = ld(nja);
+      const Real m = l < count_of(hi_w) ? mr : 0.0;
       const Real t = c0 * (jv + bias), il = is * lam, b = mu * lam_n;
       Real y = lam + (t - il);
-      const Real hi = hi_w < 0 ? INFINITY : b;
+      const Real hi = (hi_w >> 27) & 1 ? INFINITY : b;
       Real nw = rmin(rmax(y, -b), hi);
       if constexpr (EQ) {
         y = (lam + t) - il;
-        nw = (hi_w >> 28) & 1 ? y : nw;
+        nw = (hi_w >> 26) & 1 ? y : nw;
       }
-      const Real dl = nw - lam, vn = vv + m * dl, size = fabs(dl), ac = fabs(c0);
-      // |dl| against inv_a tol, from c0 = -inv_a or -inv_a mass_scale
-      const bool above = size > ac * (is != 0.0 ? hi1 : hi0), below = size < ac * (is != 0.0 ? lo1 : lo0);
-      const bool odd = !rfinite(vn) || !rfinite(jv);
-      if (__ballot(odd || (!above && !below && dl != 0.0)) == 0) {
-        moved = moved || above;
-        st(va, vn);
-        st(recb + r * RB + LAM, nw);
-      } else if (X::ballot([&](int) { return odd; })) {
-        general(r);  // this row and the rest
-        continue;
-      } else {
-        if (!above && !below && dl != 0.0) {
-          const Real ia = S.grow[e * (int64_t)M.nrmax * 10 + (int64_t)r * 10 + PR_INVA];
-          moved = moved || pgs_reaches_tol(C, size, ia);
+      const Real dl = nw - lam, vn = vv + m * dl;
+      const bool odd = __builtin_isnan(jv) || !__builtin_isfinite(vn);
+      if (__ballot(odd)) {
+        if (X::ballot([&](int) { return odd; })) {
+          general(r);  // this row and the rest
+          continue;
+        }
+      }
+      if (__ballot(!moved && dl != 0.0)) {
+        // |dl| against inv_a tol, from c0 = -inv_a or -inv_a mass_scale
+        const Real size = fabs(dl), ac = fabs(c0);
+        const bool soft = is != 0.0;
+        const bool above = size > ac * (soft ? hi1 : hi0), below = size < ac * (soft ? lo1 : lo0);
+        if (__ballot(!above && !below && dl != 0.0)) {
+          if (!above && !below && dl != 0.0)
+            moved = moved || pgs_reaches_tol(C, size, S.grow[e * (int64_t)M.nrmax * 10 + (int64_t)r * 10 + PR_INVA]);
         }
         moved = moved || above;
-        st(va, vn);
-        st(recb + r * RB + LAM, nw);
       }
+      st(va, vn);
+      st(ra + LAM, nw);
       X::order();
-      const bool in = l < count_of(nhi);
-      lam = ld(recb + rn * RB + LAM);
-      c0 = nc0, bias = nbias, is = nis, mu = nmu, lo_w = nlo, hi_w = nhi, va = nva;
-      j = in ? nj : 0.0;
-      m = in ? nm : 0.0;
-      nc0 = xc0, nbias = xbias, nis = xis, nmu = xmu, nlo = xlo, nhi = xhi;
-      r = rn;
-      if (rn == 0) {  // the sweep's end
+      j = l < count_of(nhi) ? nj : 0.0;
+      va = nva, ja = nja, hi_w = nhi, ra = rb;
+      r = last ? 0 : r + 1;
+      if (last) {  // the sweep's end
         it++;
         if (!moved || it >= limit) {
           if (phase == 0) {
@@ -391,7 +384,7 @@ __global__ void __launch_bounds__(64) k_pgs_sweeps_rows(const DModel* __restrict
             it = 0;
             limit = relax;
             records(1);
-            start(0);
+            start();
           } else {
             store(true);
           }
