@@ -477,13 +477,21 @@ extern "C" int pippin_hip_create(const ph_model_desc* desc, int64_t num_envs, co
       s->envs_per_wg = k;
       break;
     }
+  // PGS models with packed rows start with the split step: fused, the sweeps of
+  // several envs wait for each other at every row (Ant, 4096 envs, 4 steps: 9.9
+  // ms fused, 2.1 ms split; six-body pile, 8192 envs: 125 and 11.4 ms)
+  if (M.solver_kind == 1 && M.pgs_w > 0) {
+    s->envs_per_wg = 1;
+    s->sched = PH_SCHED_PGS_SPLIT;
+  }
   if (const char* ev = std::getenv("PIPPIN_HIP_ENVS_PER_WG")) {
+    s->sched = PH_SCHED_GRID;
     int k = std::atoi(ev);
     if ((k == 1 || k == 2 || k == 4) && (int64_t)k * M.L.bytes <= lds_max) s->envs_per_wg = k;
   }
   // model-specialised kernel when the model's sizes and layout match one built
   // in (PIPPIN_HIP_SPEC=0 forces the generic kernel)
-  s->spec = SpecAnt::matches(M) ? 1 : 0;
+  s->spec = SpecAnt::matches(M) && M.solver_kind == 0 ? 1 : 0;
   if (const char* ev = std::getenv("PIPPIN_HIP_SPEC"))
     if (std::atoi(ev) == 0) s->spec = 0;
   for (int k : {1, 2, 4}) {
