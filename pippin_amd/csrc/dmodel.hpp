@@ -109,7 +109,7 @@ struct DModel {
   gp<const int> body_parent, body_jntadr, body_jntnum, body_dofadr, body_dofnum, body_lastdof;
   gp<const uint64_t> body_chain;  // dofs on the path world..body (bit k = dof k)
   gp<const Real> body_pos, body_quat;
-  gp<const int> level_adr, level_body;  // bodies grouped by depth (parents first)
+  gp<const int> level_adr, level_body, body_level;  // bodies grouped by depth (parents first), and their depths
   gp<const int> acc_level_adr, acc_parent, acc_child_adr, acc_child;  // leaf-to-root sum schedule
   gp<const int> jnt_type, jnt_qposadr, jnt_dofadr, jnt_limited;
   gp<const Real> jnt_pos, jnt_axis, jnt_range, jnt_stiffness, jnt_springref;

@@ -362,8 +362,11 @@ bool build_host_model(const ph_model_desc& s, HostModel& m, std::string* err) {
   }
   m.level_adr.clear();
   m.level_body.clear();
+  m.body_level.assign(nb, -1);
   for (int l = 1; l <= maxd; l++) {
     m.level_adr.push_back((int)m.level_body.size());
+    for (int b = 1; b < nb; b++)
+      if (depth[b] == l) m.body_level[b] = (int)m.level_adr.size() - 1;
     for (int b = 1; b < nb; b++)
       if (depth[b] == l) m.level_body.push_back(b);
   }

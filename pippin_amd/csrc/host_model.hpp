@@ -37,7 +37,7 @@ struct HostModel {
   // derived (model.rs:279-316)
   std::vector<int32_t> body_lastdof, dof_parent, body_weldid, block_adr, dof_block;
   std::vector<uint64_t> body_chain, dof_anc;
-  std::vector<int32_t> level_adr, level_body;
+  std::vector<int32_t> level_adr, level_body, body_level;
   // leaf-to-root accumulation schedule (crba / rne): levels deepest first;
   // each level lists (parent, children in descending index order) groups
   std::vector<int32_t> acc_level_adr, acc_parent, acc_child_adr, acc_child;

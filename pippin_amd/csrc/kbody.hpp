@@ -71,20 +71,71 @@ PHD void rows_bind(const MT& M, const DState& S, Env& E, int nr) {
 }
 
 // ---------------- kinematics, forward.rs:14-90 ----------------
+// What the level loops need of a body. Each lane keeps its own body's record
+// in registers over a step's level loops: read in the loops, the indices were
+// three dependent loads a level.
+struct BodyRec {
+  int level, parent, j0, nj, type, qa, da;  // type, qa, da: the first joint's
+  V3 pos, jpos, jaxis;
+  Q4 quat;
+};
+template <class MT>
+PHD BodyRec body_rec(const MT& M, int b) {
+  BodyRec r{};
+  r.level = M.body_level[b];
+  r.parent = M.body_parent[b];
+  r.j0 = M.body_jntadr[b];
+  r.nj = M.body_jntnum[b];
+  r.pos = ld3(M.body_pos + 3 * b);
+  r.quat = ldq(M.body_quat + 4 * b);
+  if (r.nj > 0) {
+    r.type = M.jnt_type[r.j0];
+    r.qa = M.jnt_qposadr[r.j0];
+    r.da = M.jnt_dofadr[r.j0];
+    r.jpos = ld3(M.jnt_pos + 3 * r.j0);
+    r.jaxis = ld3(M.jnt_axis + 3 * r.j0);
+  }
+  return r;
+}
+// The records of an env's bodies, one per lane (models of more bodies than the
+// env has lanes read them as they go).
+template <class X>
+using BodyRecs = typename X::template Own<BodyRec>;
 template <class X, class MT>
-PHD void fk_body(const MT& M, Env& E, int b) {
+PHD void load_body_recs(const MT& M, BodyRecs<X>& recs) {
+  if (M.nbody - 1 <= X::WIDTH) X::par(M.nbody - 1, [&](int i) { recs.at(i) = body_rec(M, i + 1); });
+}
+// f(b, record) for the bodies of level l, then a sync.
+template <class X, class MT, class F>
+PHD void each_of_level(const MT& M, BodyRecs<X>& recs, int l, F&& f) {
+  if (M.nbody - 1 <= X::WIDTH) {
+    X::par(M.nbody - 1, [&](int i) {
+      if (recs.at(i).level == l) f(i + 1, recs.at(i));
+    });
+  } else {
+    const int b0 = M.level_adr[l], nb = M.level_adr[l + 1] - b0;
+    X::par(nb, [&](int i) {
+      const int b = M.level_body[b0 + i];
+      f(b, body_rec(M, b));
+    });
+  }
+}
+
+template <class X, class MT>
+PHD void fk_body(const MT& M, Env& E, int b, const BodyRec& R) {
   Real* xpos = LD(xpos);
   Real* xquat = LD(xquat);
   Real* xmat = LD(xmat);
   const Real* q = LD(qpos);
   Real* cdof = LD(cdof);
-  int p = M.body_parent[b];
-  V3 pos = ld3(xpos + 3 * p) + mul_vec(ldm(xmat + 9 * p), ld3(M.body_pos + 3 * b));
-  Q4 quat = qmul(ldq(xquat + 4 * p), ldq(M.body_quat + 4 * b));
-  int j0 = M.body_jntadr[b], j1 = j0 + M.body_jntnum[b];
-  for (int j = j0; j < j1; j++) {
-    int qa = M.jnt_qposadr[j], da = M.jnt_dofadr[j];
-    int t = M.jnt_type[j];
+  const int p = R.parent;
+  V3 pos = ld3(xpos + 3 * p) + mul_vec(ldm(xmat + 9 * p), R.pos);
+  Q4 quat = qmul(ldq(xquat + 4 * p), R.quat);
+  for (int j = R.j0; j < R.j0 + R.nj; j++) {
+    const bool first = j == R.j0;
+    const int qa = first ? R.qa : M.jnt_qposadr[j], da = first ? R.da : M.jnt_dofadr[j];
+    const int t = first ? R.type : M.jnt_type[j];
+    const V3 jp = first ? R.jpos : ld3(M.jnt_pos + 3 * j), jax = first ? R.jaxis : ld3(M.jnt_axis + 3 * j);
     if (t == J_FREE) {
       pos = v3(q[qa], q[qa + 1], q[qa + 2]);
       quat = qnormalized(q4(q[qa + 3], q[qa + 4], q[qa + 5], q[qa + 6]));
@@ -96,7 +147,6 @@ PHD void fk_body(const MT& M, Env& E, int b) {
         stsp(cdof + 6 * (da + 3 + k), sp(a, cross(pos, a)));
       }
     } else if (t == J_BALL) {
-      V3 jp = ld3(M.jnt_pos + 3 * j);
       V3 anchor = pos + qrotate(quat, jp);
       Q4 ql = qnormalized(q4(q[qa], q[qa + 1], q[qa + 2], q[qa + 3]));
       quat = qmul(quat, ql);
@@ -107,14 +157,12 @@ PHD void fk_body(const MT& M, Env& E, int b) {
         stsp(cdof + 6 * (da + k), sp(a, cross(anchor, a)));
       }
     } else if (t == J_HINGE) {
-      V3 jp = ld3(M.jnt_pos + 3 * j), jax = ld3(M.jnt_axis + 3 * j);
       V3 anchor = pos + qrotate(quat, jp);
       V3 axis = qrotate(quat, jax);
       quat = qmul(quat, ldq(LD(jq) + 4 * j));  // from_axis_angle(axis, q - qpos0), precomputed
       pos = anchor - qrotate(quat, jp);
       stsp(cdof + 6 * da, sp(axis, cross(anchor, axis)));
     } else {
-      V3 jp = ld3(M.jnt_pos + 3 * j), jax = ld3(M.jnt_axis + 3 * j);
       V3 anchor = pos + qrotate(quat, jp);
       (void)anchor;
       V3 axis = qrotate(quat, jax);
@@ -150,7 +198,8 @@ PHD void body_inertia(const MT& M, Env& E, int b) {
 }
 
 template <class X, class MT>
-PHD void kinematics(const MT& M, Env& E) {
+PHD void kinematics(const MT& M, Env& E, BodyRecs<X>& recs) {
+  load_body_recs<X>(M, recs);
   // hinge rotations do not depend on the parent's pose: evaluate their
   // sin/cos for all joints at once, off the tree's serial path
   X::par(M.njnt, [&](int j) {
@@ -167,11 +216,14 @@ PHD void kinematics(const MT& M, Env& E) {
     Real* ci = LD(cinert);
     for (int k = 0; k < 13; k++) ci[k] = 0.0;
   });
-  for (int l = 0; l < M.nlevel; l++) {
-    int b0 = M.level_adr[l], nb = M.level_adr[l + 1] - b0;
-    X::par(nb, [&](int i) { fk_body<X>(M, E, M.level_body[b0 + i]); });
-  }
+  for (int l = 0; l < M.nlevel; l++)
+    each_of_level<X>(M, recs, l, [&](int b, const BodyRec& r) { fk_body<X>(M, E, b, r); });
   X::par(M.nbody - 1, [&](int i) { body_inertia<X>(M, E, i + 1); });
+}
+template <class X, class MT>
+PHD void kinematics(const MT& M, Env& E) {
+  BodyRecs<X> recs;
+  kinematics<X>(M, E, recs);
 }
 
 // Geom world poses, the last loop of forward.rs:14-90. Evaluated where they
@@ -263,7 +315,7 @@ PHD void crba(const MT& M, Env& E) {
 // would read it, so it never needs storage. Then the backward force sum and
 // qfrc_bias (forward.rs:166-171).
 template <class X, class MT>
-PHD void velocity_rne(const MT& M, Env& E) {
+PHD void velocity_rne(const MT& M, Env& E, BodyRecs<X>& recs) {
   Real* cvel = LD(cvel);
   Real* cacc = LD(cacc);
   Real* cfrc = LD(cfrc);
@@ -276,15 +328,12 @@ PHD void velocity_rne(const MT& M, Env& E) {
     stsp(cfrc, sp(v3z(), v3z()));
   });
   for (int l = 0; l < M.nlevel; l++) {
-    int b0 = M.level_adr[l], nb = M.level_adr[l + 1] - b0;
-    X::par(nb, [&](int i) {
-      int b = M.level_body[b0 + i];
-      int par = M.body_parent[b];
+    each_of_level<X>(M, recs, l, [&](int b, const BodyRec& R) {
+      const int par = R.parent;
       SP v = ldsp(cvel + 6 * par);
       SP a = ldsp(cacc + 6 * par);
-      int j0 = M.body_jntadr[b], j1 = j0 + M.body_jntnum[b];
-      for (int j = j0; j < j1; j++) {
-        int da = M.jnt_dofadr[j], t = M.jnt_type[j];
+      for (int j = R.j0; j < R.j0 + R.nj; j++) {
+        const int da = j == R.j0 ? R.da : M.jnt_dofadr[j], t = j == R.j0 ? R.type : M.jnt_type[j];
         if (t == J_FREE || t == J_BALL) {
           int lin = t == J_FREE ? 3 : 0, rot = t == J_FREE ? da + 3 : da;
           for (int k = 0; k < lin; k++) {
@@ -308,6 +357,13 @@ PHD void velocity_rne(const MT& M, Env& E) {
   X::par(M.nv, [&](int k) {
     LD(bias)[k] = sdot(ldsp(LD(cdof) + 6 * k), ldsp(cfrc + 6 * M.dof_body[k]));
   });
+}
+
+template <class X, class MT>
+PHD void velocity_rne(const MT& M, Env& E) {
+  BodyRecs<X> recs;
+  load_body_recs<X>(M, recs);
+  velocity_rne<X>(M, E, recs);
 }
 
 // ---------------- passive + actuation, forward.rs:173-211 ----------------
@@ -2841,9 +2897,12 @@ PHD int step_front(const MT& M, const DState& S, Env& E, int pgs_stop = PGS_FULL
   const int nv = M.nv;
   const Real h = M.timestep;
   int* isc = E.si + M.L.i_iscal;
-  kinematics<X>(M, E);
-  crba<X>(M, E);
-  velocity_rne<X>(M, E);
+  {
+    BodyRecs<X> recs;
+    kinematics<X>(M, E, recs);
+    crba<X>(M, E);
+    velocity_rne<X>(M, E, recs);
+  }
   passive_actuation<X>(M, E);
   collide<X>(M, S, E);
   if (isc[7] & ST_CONTACT_OVERFLOW) return STEP_FAILED;

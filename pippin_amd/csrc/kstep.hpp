@@ -15,6 +15,7 @@ namespace phk {
 template <int K>
 struct DevXK : DevLanes {
   static constexpr int G = 64 / K;
+  static constexpr int WIDTH = G;  // lanes of an env
   template <class F>
   __device__ __forceinline__ static void par(int n, F&& f) {
     for (int i = (int)(threadIdx.x % G); i < n; i += G) f(i);

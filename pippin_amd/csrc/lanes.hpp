@@ -53,6 +53,12 @@ __device__ __forceinline__ DLV operator+(DLV a, Real b) { return {a.v + b}; }
 
 struct DevLanes {
   using LV = DLV;
+  // one T per lane
+  template <class T>
+  struct Own {
+    T v;
+    __device__ __forceinline__ T& at(int) { return v; }
+  };
   __device__ __forceinline__ static int lane() { return (int)(threadIdx.x & (GL - 1)); }
   __device__ __forceinline__ static DLV splat(Real c) { return {c}; }
   template <class F>
@@ -194,6 +200,12 @@ inline HLV operator+(const HLV& a, Real b) {
 
 struct HostLanes {
   using LV = HLV;
+  static constexpr int WIDTH = 64;
+  template <class T>
+  struct Own {
+    T v[WIDTH];
+    T& at(int i) { return v[i]; }
+  };
   static HLV splat(Real c) {
     HLV r;
     for (int l = 0; l < GL; l++) r.v[l] = c;

@@ -549,6 +549,7 @@ extern "C" int pippin_hip_create(const ph_model_desc* desc, int64_t num_envs, co
   HIPCHK(ui(hm.body_lastdof, &M.body_lastdof));
   HIPCHK(ui(hm.level_adr, &M.level_adr));
   HIPCHK(ui(hm.level_body, &M.level_body));
+  HIPCHK(ui(hm.body_level, &M.body_level));
   HIPCHK(ui(hm.acc_level_adr, &M.acc_level_adr));
   HIPCHK(ui(hm.acc_parent, &M.acc_parent));
   HIPCHK(ui(hm.acc_child_adr, &M.acc_child_adr));

@@ -112,6 +112,7 @@ emu_sim* emu_create(const ph_model_desc* desc, int64_t n) {
   M.body_quat = hm.body_quat.data();
   M.level_adr = hm.level_adr.data();
   M.level_body = hm.level_body.data();
+  M.body_level = hm.body_level.data();
   M.acc_level_adr = hm.acc_level_adr.data();
   M.acc_parent = hm.acc_parent.data();
   M.acc_child_adr = hm.acc_child_adr.data();
