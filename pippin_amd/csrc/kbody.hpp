@@ -662,31 +662,39 @@ PHD void chol_solve_block(const MT& M, Env& E, const Real* L, int nv, int s0, in
   });
 }
 
+// M + h diag(damping) and the implicit actuator terms into LD(chol)
 template <class X, class MT>
-PHD bool factor_mass(const MT& M, Env& E, Real h) {
+PHD void assemble_mass(const MT& M, Env& E, Real h) {
   const int nv = M.nv;
   Real* chol = LD(chol);
   const Real* qm = LD(qm);
   X::par(nv * nv, [&](int k) { chol[k] = qm[k]; });
   // add_implicit_terms, forward.rs:407-431
   X::par(nv, [&](int k) { chol[k * nv + k] += h * M.v_dof_damping[(int64_t)E.var * nv + k]; });
-  if (M.integrator == 1) {
-    X::par(1, [&](int) {
-      for (int u = 0; u < M.nu; u++) {
-        Real kv = -M.v_act_bias[((int64_t)E.var * M.nu + u) * 3 + 2] * M.act_gear[u] * M.act_gear[u];
+  // each dof's row by one lane, its actuators in order; the terms of an entry
+  // keep the reference's (actuator, joint, joint) order
+  if (M.integrator == 1)
+    X::par(nv, [&](int a) {
+      const int i0 = M.dofact_adr[a], i1 = i0 + M.dofact_num[a];
+      for (int i = i0; i < i1; i++) {
+        const int u = M.dofact_u[i];
+        const Real kv = -M.v_act_bias[((int64_t)E.var * M.nu + u) * 3 + 2] * M.act_gear[u] * M.act_gear[u];
         if (kv == 0.0 || LD(actclamp)[u] != 0.0) continue;
-        int a0 = M.act_madr[u], a1 = a0 + M.act_mnum[u];
-        for (int ia = a0; ia < a1; ia++)
-          for (int ib = a0; ib < a1; ib++) {
-            int a = M.jnt_dofadr[M.mom_jnt[ia]], b = M.jnt_dofadr[M.mom_jnt[ib]];
-            bool anc = ((M.dof_anc[b] >> a) & 1) || ((M.dof_anc[a] >> b) & 1);
-            if (a == b || anc) chol[a * nv + b] += h * kv * M.mom_coef[ia] * M.mom_coef[ib];
-          }
+        const int m0 = M.act_madr[u], m1 = m0 + M.act_mnum[u];
+        for (int ib = m0; ib < m1; ib++) {
+          const int b = M.jnt_dofadr[M.mom_jnt[ib]];
+          const bool anc = ((M.dof_anc[b] >> a) & 1) || ((M.dof_anc[a] >> b) & 1);
+          if (a == b || anc) chol[a * nv + b] += h * kv * M.dofact_coef[i] * M.mom_coef[ib];
+        }
       }
     });
-  }
+}
+
+template <class X, class MT>
+PHD bool factor_mass(const MT& M, Env& E, Real h) {
+  assemble_mass<X>(M, E, h);
   for (int blk = 0; blk < M.nblock; blk++)
-    if (!chol_block<X>(M, E, chol, nv, M.block_adr[blk], M.block_adr[blk + 1])) return false;
+    if (!chol_block<X>(M, E, LD(chol), M.nv, M.block_adr[blk], M.block_adr[blk + 1])) return false;
   return true;
 }
 
@@ -701,10 +709,9 @@ PHD void mass_solve(const MT& M, Env& E, Real* x) {
 // (block and row b, b + ROWS, ...): one matrix row per lane, the register
 // Cholesky, then the two triangular solves. The factor is stored in LD(chol).
 template <int NM, class X, class MT>
-PHD bool factor_solve_blocks(const MT& M, Env& E, Real h, Real* x) {
+PHD bool factor_solve_blocks(const MT& M, Env& E, const Real* qm, Real h, Real* x) {
   using LV = typename X::LV;
   const int nv = M.nv;
-  const Real* qm = LD(qm);
   auto damp = M.v_dof_damping + (int64_t)E.var * nv;
   int* isc = E.si + M.L.i_iscal;
   const int nblock = M.nblock;
@@ -748,15 +755,20 @@ PHD bool factor_solve_blocks(const MT& M, Env& E, Real h, Real* x) {
   return (nblock == 1 && X::ROWS == 1) || isc[1] == 0;
 }
 
-// factor_mass then mass_solve. With Euler integration and dof blocks of at
-// most 16 dofs both run in registers, block by block; other models take the
-// general path. Returns false when the matrix is not positive definite
-// (isc[1], which the caller has cleared).
+// factor_mass then mass_solve. Dof blocks of at most 16 dofs are factored and
+// solved in registers, block by block (from M itself when there are no implicit
+// actuator terms to add: Euler integration, or h = 0); larger ones take the
+// general path. Returns false when the matrix is not positive definite (isc[1],
+// which the caller has cleared).
 template <class X, class MT>
 PHD bool factor_solve_mass(const MT& M, Env& E, Real h, Real* x) {
-  if (M.integrator == 0 && M.bmax <= GL) {
-    if (M.bmax <= 6) return factor_solve_blocks<6, X>(M, E, h, x);
-    return factor_solve_blocks<GL, X>(M, E, h, x);
+  if (M.bmax <= GL) {
+    const bool own = M.integrator == 0 || h == 0.0;
+    if (!own) assemble_mass<X>(M, E, h);
+    const Real* A = own ? LD(qm) : LD(chol);
+    const Real hd = own ? h : 0.0;
+    if (M.bmax <= 6) return factor_solve_blocks<6, X>(M, E, A, hd, x);
+    return factor_solve_blocks<GL, X>(M, E, A, hd, x);
   }
   if (!factor_mass<X>(M, E, h)) return false;
   mass_solve<X>(M, E, x);
@@ -1335,21 +1347,46 @@ __device__ __noinline__ void hessian_mfma(const Real* qm, const Real* J, const R
 }
 #endif
 
-// start + x[0] + x[st] + ... + x[(n - 1) st], in that order, in every lane: the
+// start + x[0] + x[1] + ... + x[n - 1], in that order, in every lane: the
 // loads of eight terms are issued before their adds.
 template <class P>
-PHD Real sum_in_order(P x, int st, int n, Real start) {
+PHD Real sum_in_order(P x, int n, Real start) {
   Real s = start;
   int i = 0;
   for (; i + 8 <= n; i += 8) {
     Real v[8];
 #pragma unroll
-    for (int k = 0; k < 8; k++) v[k] = x[(i + k) * st];
+    for (int k = 0; k < 8; k++) v[k] = x[i + k];
 #pragma unroll
     for (int k = 0; k < 8; k++) s = s + v[k];
   }
-  for (; i < n; i++) s = s + x[i * st];
+  for (; i < n; i++) s = s + x[i];
   return s;
+}
+
+// The same for x and y side by side.
+template <class P>
+PHD void sum2_in_order(P x, P y, int n, Real sx, Real sy, Real* ox, Real* oy) {
+  int i = 0;
+  for (; i + 4 <= n; i += 4) {
+    Real u[4], v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      u[k] = x[i + k];
+      v[k] = y[i + k];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      sx = sx + u[k];
+      sy = sy + v[k];
+    }
+  }
+  for (; i < n; i++) {
+    sx = sx + x[i];
+    sy = sy + y[i];
+  }
+  *ox = sx;
+  *oy = sy;
 }
 
 // Rows of a dense problem: J (nr x nv), targets, 1/R, J a - aref, J p, two
@@ -1434,7 +1471,7 @@ __host__ __device__ __attribute__((noinline)) int newton_dense(NPT<QP> Q, RowsP<
   };
   auto sum_k = [&](LP x, LP y) {  // sum over dofs of x y
     X::par(nv, [&](int k) { mp[k] = x[k] * y[k]; });
-    return sum_in_order(mp, 1, nv, rsum0());
+    return sum_in_order(mp, nv, rsum0());
   };
   X::par(nv, [&](int k) { a0[k] = a[k]; });
   // cost(x) = 1/2 (x-a0)'M(x-a0) + sum_active 1/2 D r^2 with r = J x - aref
@@ -1446,7 +1483,7 @@ __host__ __device__ __attribute__((noinline)) int newton_dense(NPT<QP> Q, RowsP<
       t[r] = r >= n_ineq || v < 0.0 ? 0.5 * dd[r] * v * v : -0.0;
     });
     const Real c = 0.5 * sum_k(tmp, tmp2);
-    return sum_in_order(t, 1, nr, c);
+    return sum_in_order(t, nr, c);
   };
   // the active rows at jar, in order, into the list (their number returned),
   // 16 per entry at the end of t; *same: as they were before
@@ -1564,8 +1601,7 @@ __host__ __device__ __attribute__((noinline)) int newton_dense(NPT<QP> Q, RowsP<
         t[r] = on ? dq * v : -0.0;
         lst[r] = on ? dq * jp[r] : -0.0;
       });
-      *d1o = sum_in_order(t, 1, nr, al * mpp + mpg);
-      *d2o = sum_in_order(lst, 1, nr, mpp);
+      sum2_in_order(t, lst, nr, al * mpp + mpg, mpp, d1o, d2o);
       X::sync();
     };
     Real lo = 0.0, hi = INFINITY, al = 1.0, d1, d2;
