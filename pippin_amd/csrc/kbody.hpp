@@ -559,6 +559,26 @@ PHD void collide(const MT& M, const DState& S, Env& E) {
   }
   auto con = S.con + E.e * (int64_t)M.ncmax * CW;
   auto cg = S.cgeom + E.e * (int64_t)M.ncmax * 3;
+  // With the contacts' places in the staging area listed (over the geom
+  // rotations, used up by now), all lanes copy them side by side; with a lane
+  // per pair the copies of the six-body pile's contacts took 8 us of the step.
+  const int ncon = isc[0];
+  if (ncon <= 18 * ng) {
+    int* src = reinterpret_cast<int*>(LD(gxmat));
+    X::par(M.npair, [&](int p) {
+      const int n = cnt[p], o = off[p];
+      for (int h = 0; h < n && o + h < M.ncmax; h++) src[o + h] = MAXHIT * p + h;
+    });
+    X::par(ncon * CW, [&](int t) { con[t] = stage[(int64_t)src[t / CW] * CW + t % CW]; });
+    X::par(ncon, [&](int c) {
+      const int p = src[c] / MAXHIT;
+      auto gd = cg + 3 * c;
+      gd[0] = M.pair_g1[p];
+      gd[1] = M.pair_g2[p];
+      gd[2] = src[c] % MAXHIT;
+    });
+    return;
+  }
   X::par(M.npair, [&](int p) {
     int n = cnt[p];
     for (int h = 0; h < n && off[p] + h < M.ncmax; h++) {
