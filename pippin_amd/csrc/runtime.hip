@@ -516,12 +516,16 @@ extern "C" int pippin_hip_create(const ph_model_desc* desc, int64_t num_envs, co
   HIPCHK(s->d_order.alloc(std::max<int64_t>(num_envs, 1)));
   if (M.solver_kind == 1) {
     // Packed sweeps: the LDS of an env is what its rows can need, up to a
-    // third of a CU's over the four envs of a wavefront.
+    // third or a quarter of a CU's over the four envs of a wavefront.
     if (M.pgs_w > 0) {
       const int64_t rows = 3 * (int64_t)M.ncmax + 2 * hm.nlimited + d.neq;
       const int64_t most = pgs_packed_doubles(M.nv, rows, rows * M.pgs_w);
-      const int64_t third = (160 * 1024 / 3 - 512) / 4 / 8;  // 512: the allocation's granularity
-      s->pgs_slice = (int)(std::min(most + 1, third) & ~(int64_t)1);
+      // A single tree of at most 16 dofs meets few contacts: a quarter of the
+      // LDS holds 37 rows of an Ant, and four wavefronts per CU fill its SIMDs
+      // (4096 envs in flight instead of 3072). Piles of bodies need a third
+      // (62 rows of two free bodies).
+      const int64_t part = (160 * 1024 / (M.nv <= 16 ? 4 : 3) - 512) / 4 / 8;  // 512: the allocation's granularity
+      s->pgs_slice = (int)(std::min(most + 1, part) & ~(int64_t)1);
       const void* k = pgs_rows_kernel(M);
       const int bytes = 4 * s->pgs_slice * 8;
       HIPCHK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
