@@ -479,7 +479,7 @@ extern "C" int pippin_hip_create(const ph_model_desc* desc, int64_t num_envs, co
     }
   // PGS models with packed rows start with the split step: fused, the sweeps of
   // several envs wait for each other at every row (Ant, 4096 envs, 4 steps: 9.9
-  // ms fused, 2.1 ms split; six-body pile, 8192 envs: 125 and 11.4 ms)
+  // ms fused, 1.84 ms split; six-body pile, 8192 envs: 125 and 11.0 ms)
   if (M.solver_kind == 1 && M.pgs_w > 0) {
     s->envs_per_wg = 1;
     s->sched = PH_SCHED_PGS_SPLIT;

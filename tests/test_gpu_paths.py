@@ -1,0 +1,88 @@
+"""Host paths of get and set, and the split PGS step's launches (needs a GPU)."""
+import sys
+
+import numpy as np
+import pytest
+
+from oracle import mjcf
+from oracle.pyoracle import OracleSim
+from pippin_amd.physics import HipPhysics
+from pippin_amd.workloads import arm_gripper_xml, random_pile_xml
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+@pytest.mark.parametrize("shared", [False, True])
+def test_get_and_set_on_both_sides_of_the_staging(assets, shared):
+    """Up to 256 KiB (2184 Ants' qpos) go through pinned staging, which several
+    calls in a row fill; more is copied directly, as is every set call after a
+    device pointer to state was handed out."""
+    n = 2300
+    say("staging, shared", shared)
+    arr = mjcf.load_file(assets / "ant.xml")
+    g = HipPhysics(arr, n)
+    if shared:
+        assert g.state_ptr("qpos")
+    rng = np.random.default_rng(3)
+    want = g.get("qpos").copy()
+    # one env, a block and a ragged end, the largest staged, the smallest direct,
+    # and staged calls that do not fit beside each other
+    for b, e in [(0, 1), (17, 120), (2299, 2300), (0, 2184), (5, 2190), (0, 1500), (300, 1800), (100, 101), (0, 2300),
+                 (900, 2300)]:
+        x = rng.normal(size=(e - b, 15))
+        g.set("qpos", b, e, x)
+        want[b:e] = x
+        x[:] = np.nan  # the caller's array is free again when the call returns
+    assert np.array_equal(g.get("qpos"), want)
+    for b, e in [(0, 1), (2299, 2300), (0, 2184), (0, 2185), (116, 2300)]:
+        assert np.array_equal(g.get("qpos", b, e), want[b:e]), (b, e)
+    g.close()
+
+
+@pytest.mark.parametrize("n", [1, 5, 130])
+@pytest.mark.parametrize("name", ["ant", "pressed", "arm", "pile"])
+def test_split_pgs_step_equals_the_oracle(assets, name, n):
+    """The shape that PGS models start with: one dof block with limits; Ants
+    pressed into the floor, some with more rows than the packed sweeps hold;
+    two blocks with an equality and a tendon; blocks of six dofs."""
+    if name == "arm":
+        arr = mjcf.load_string(arm_gripper_xml(3))
+    elif name == "pile":
+        arr = mjcf.load_string(random_pile_xml(29))
+    else:
+        arr = mjcf.load_file(assets / "ant.xml")
+    arr = {**arr, "solver_kind": 1}
+    o, g = OracleSim(arr, n), HipPhysics(arr, n)
+    say("split PGS", name, n, g.launch_shape())
+    assert g.launch_shape()[2] == "pgs_split"
+    rng = np.random.default_rng(1)
+    q = o.get("qpos")
+    if name == "pressed":
+        q[:, 2] = rng.uniform(0.05, 0.35, n)
+        q[:, 7:] += rng.uniform(-0.8, 0.8, (n, 8))
+    elif name == "ant":
+        q += 0.01 * rng.normal(size=q.shape)
+    for s in (o, g):
+        s.set("qpos", 0, n, q)
+    nu = int(arr["nu"])
+    rows = 0
+    for t in range(20):
+        if nu:
+            c = rng.uniform(-0.3, 0.3, (n, nu))
+            for s in (o, g):
+                s.set("ctrl", 0, n, c)
+        # uneven ranges, one and several steps a call
+        for s in (o, g):
+            s.step(0, (n + 1) // 2, 1)
+            s.step(0, n, 3)
+        rows = max(rows, int(o.step_stats()[1].max()))
+        assert np.array_equal(o.ncon(), g.ncon()), t
+        assert np.array_equal(o.get("qpos"), g.get("qpos")), t
+        assert np.array_equal(o.get("qvel"), g.get("qvel")), t
+    say("  rows up to", rows)
+    g.close()
