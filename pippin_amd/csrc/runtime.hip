@@ -230,6 +230,7 @@ struct Pinned {
   static constexpr size_t STAGE = 256 * 1024;  // bytes; larger calls copy directly
   char* p = nullptr;
   size_t used = 0;  // staging bytes whose copies may still be in flight
+  bool device = false;  // copies of set_device may still be in flight
   std::mutex mu;    // held while the staging is in use: get may be called from several threads
   ~Pinned() {
     if (p) (void)hipHostFree(p);
@@ -723,6 +724,14 @@ static size_t step_lds(const ph_sim* s, int K) {
   return (size_t)K * s->M.L.bytes + (K == 1 ? (size_t)s->M.x1 * sizeof(double) : 0);
 }
 
+// Waits for the sim's stream: no copy of the staging or of set_device is in flight after it.
+static hipError_t drain(const ph_sim* s) {
+  if (hipError_t e = hipStreamSynchronize(s->stream)) return e;
+  s->pin.used = 0;
+  s->pin.device = false;
+  return hipSuccess;
+}
+
 static int check_range(const ph_sim* s, int64_t b, int64_t e) {
   if (!s) return fail(PH_ERR_ARG, "null sim");
   if (b < 0 || e < b || e > s->n) return fail(PH_ERR_ARG, "env range out of bounds");
@@ -1071,8 +1080,7 @@ static int timed_launch(ph_sim* s, int64_t begin, int64_t end, int64_t nstep, co
   s->poses_stale = true;
   HIPCHK(hipGetLastError());
   if (!one) HIPCHK(hipEventRecord(s->ev1, s->stream));
-  HIPCHK(hipStreamSynchronize(s->stream));
-  s->pin.used = 0;
+  HIPCHK(drain(s));
   float ms = 0.0f;
   HIPCHK(hipEventElapsedTime(&ms, s->ev0, s->ev1));
   s->kernel_ms += ms;
@@ -1111,6 +1119,7 @@ extern "C" int pippin_hip_set_device(ph_sim* s, int32_t field, int64_t begin, in
   int w = field_width(s, field, &d);
   if (field != PH_FIELD_QVEL && field != PH_FIELD_CTRL) return fail(PH_ERR_ARG, "set_device takes qvel or ctrl");
   if (w == 0 || end == begin) return PH_OK;
+  s->pin.device = true;
   HIPCHK(hipMemcpyAsync(d + begin * w, src, (end - begin) * w * sizeof(double), hipMemcpyDeviceToDevice, s->stream));
   return PH_OK;
 }
@@ -1131,10 +1140,7 @@ extern "C" int pippin_hip_state_device(ph_sim* s, int32_t field, double** ptr) {
   if (field == PH_FIELD_QPOS) s->qpos_shared = true;
   if (*ptr) {
     s->state_shared = true;
-    if (s->pin.used) {  // copies staged before are done when the pointer is out
-      HIPCHK(hipStreamSynchronize(s->stream));
-      s->pin.used = 0;
-    }
+    if (s->pin.used) HIPCHK(drain(s));  // copies staged before are done when the pointer is out
   }
   return *ptr ? PH_OK : fail(PH_ERR_ARG, "unknown field");
 }
@@ -1157,8 +1163,7 @@ extern "C" int pippin_hip_get(const ph_sim* s, int32_t field, int64_t begin, int
     hipLaunchKernelGGL(k_copy, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s->stream, d + begin * w,
                        s->pin.stage(), count);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(s->stream));
-    s->pin.used = 0;
+    HIPCHK(drain(s));
     memcpy(out, s->pin.stage(), count * sizeof(double));
     return PH_OK;
   }
@@ -1177,15 +1182,13 @@ extern "C" int pippin_hip_set(ph_sim* s, int32_t field, int64_t begin, int64_t e
   if (int rc = check_len("set", len, end - begin, w)) return rc;
   if (w == 0 || end == begin) return PH_OK;
   const size_t bytes = (size_t)(end - begin) * w * sizeof(double);
-  if (bytes <= Pinned::STAGE && !s->state_shared) {
+  if (bytes <= Pinned::STAGE && !s->state_shared && !s->pin.device) {
     // staged, and copied in order with the stream's other work: only pointers
-    // that the sim handed out could see the state before that
+    // that the sim handed out could see the state before that, and only
+    // set_device's sources are read by copies that this call has to wait for
     HIPCHK(hipSetDevice(s->device));
     std::lock_guard<std::mutex> lock(s->pin.mu);
-    if (s->pin.used + bytes > Pinned::STAGE) {
-      HIPCHK(hipStreamSynchronize(s->stream));
-      s->pin.used = 0;
-    }
+    if (s->pin.used + bytes > Pinned::STAGE) HIPCHK(drain(s));
     double* stage = s->pin.stage() + s->pin.used / sizeof(double);
     memcpy(stage, src, bytes);
     s->pin.used += bytes;
@@ -1196,8 +1199,7 @@ extern "C" int pippin_hip_set(ph_sim* s, int32_t field, int64_t begin, int64_t e
     if (field == PH_FIELD_QPOS) s->poses_stale = true;
     return PH_OK;
   }
-  HIPCHK(hipStreamSynchronize(s->stream));  // a pending set_device copy must not overwrite this one
-  s->pin.used = 0;
+  HIPCHK(drain(s));  // a pending set_device copy must not overwrite this one, and its source is free after it
   HIPCHK(hipMemcpy(d + begin * w, src, (end - begin) * w * sizeof(double), hipMemcpyHostToDevice));
   if (field == PH_FIELD_QPOS) s->poses_stale = true;
   return PH_OK;

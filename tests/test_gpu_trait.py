@@ -294,6 +294,29 @@ def test_set_device_is_ordered_before_get_set_and_step(assets):
     assert np.array_equal(g.get("qpos"), ref.get("qpos"))
 
 
+@pytest.mark.parametrize("field", ["ctrl", "qvel"])
+def test_set_waits_for_the_copies_of_set_device(assets, field):
+    """Once set has returned, a caller may refill or free set_device's source:
+    no copy is left on the library stream, however small the set call."""
+    import torch
+
+    arr = mjcf.load_file(assets / "ant.xml")
+    n = 16384
+    g = HipPhysics(arr, n)
+    stream = torch.cuda.ExternalStream(g.L.pippin_hip_stream(g.h))
+    w = g.width(field)
+    buf = torch.zeros((n, w), dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    one = np.full((1, g.nq), 0.5)
+    for _ in range(3):
+        g.set("qpos", 0, 1, one)  # staged
+        for _ in range(300):  # about 1 ms of copies
+            g.set_device(field, 0, n, buf.data_ptr())
+        g.set("qpos", 1, 2, one)
+        assert stream.query()
+    assert np.array_equal(g.get("qpos", 0, 2), np.repeat(one, 2, axis=0))
+
+
 def test_device_poses_equal_host_poses(assets):
     """pippin_hip_poses_device: the f32 Pose records of every env in device
     memory, for a renderer on the GPU; equal to the host copy of poses() bit
