@@ -1155,6 +1155,7 @@ extern "C" int pippin_hip_get(const ph_sim* s, int32_t field, int64_t begin, int
   if (w < 0) return fail(PH_ERR_ARG, "unknown field");
   if (int rc = check_len("get", len, end - begin, w)) return rc;
   if (w == 0 || end == begin) return PH_OK;
+  if (!out) return fail(PH_ERR_ARG, "null argument");
   const int64_t count = (end - begin) * w;
   if ((size_t)count * sizeof(double) <= Pinned::STAGE) {
     HIPCHK(hipSetDevice(s->device));
@@ -1181,6 +1182,7 @@ extern "C" int pippin_hip_set(ph_sim* s, int32_t field, int64_t begin, int64_t e
   if (w < 0) return fail(PH_ERR_ARG, "unknown field");
   if (int rc = check_len("set", len, end - begin, w)) return rc;
   if (w == 0 || end == begin) return PH_OK;
+  if (!src) return fail(PH_ERR_ARG, "null argument");
   const size_t bytes = (size_t)(end - begin) * w * sizeof(double);
   if (bytes <= Pinned::STAGE && !s->state_shared && !s->pin.device) {
     // staged, and copied in order with the stream's other work: only pointers

@@ -44,6 +44,17 @@ def test_get_and_set_on_both_sides_of_the_staging(assets, shared):
     g.close()
 
 
+@pytest.mark.parametrize("n", [1, 2300])
+def test_get_and_set_refuse_a_null_buffer(assets, n):
+    """Through the staging as on the direct path: an error code, and nothing is changed."""
+    g = HipPhysics(mjcf.load_file(assets / "ant.xml"), n)
+    before = g.get("qpos")
+    for fn in (g.L.pippin_hip_get, g.L.pippin_hip_set):
+        assert fn(g.h, 0, 0, n, None, n * g.nq) != 0
+        assert fn(g.h, 0, 0, 0, None, 0) == 0  # no envs: nothing to copy
+    assert np.array_equal(g.get("qpos"), before)
+
+
 @pytest.mark.parametrize("n", [1, 5, 130])
 @pytest.mark.parametrize("name", ["ant", "pressed", "arm", "pile"])
 def test_split_pgs_step_equals_the_oracle(assets, name, n):
