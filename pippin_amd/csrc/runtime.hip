@@ -21,6 +21,7 @@
 #include "../../include/pippin_hip.h"
 #include "host_model.hpp"
 #include "kstep.hpp"
+#include "launch_rules.hpp"
 #include "mlp_host.hpp"
 #include "spec_models.hpp"
 #include "step_kernels.hpp"
@@ -271,6 +272,7 @@ struct ph_sim {
   int sched = PH_SCHED_GRID;  // schedule of the plain step (PH_SCHED_*)
   int cus = 0;                // compute units of the device
   int pgs_per_cu = 0;         // wavefronts of the packed PGS sweeps that a CU holds
+  int pgs_wide_per_cu = 0;    // and of the sweeps over rows that are not packed
   int pgs_slice = 0;          // LDS doubles per env of the packed PGS sweeps (0: no packed rows)
   int ws_per_cu[3][2] = {};   // resident work-stealing workgroups per CU, by K = 1, 2, 4 and kernel instance
   std::string arch;           // device architecture name (autotune cache key)
@@ -531,6 +533,7 @@ extern "C" int pippin_hip_create(const ph_model_desc* desc, int64_t num_envs, co
       const int bytes = 4 * s->pgs_slice * 8;
       HIPCHK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
       HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&s->pgs_per_cu, k, 64, (size_t)bytes));
+      HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&s->pgs_wide_per_cu, (const void*)k_pgs_sweeps<1>, 64, 0));
     }
     HIPCHK(s->d_pgs_vel.alloc((size_t)std::max<int64_t>(num_envs * M.nv, 1)));
     HIPCHK(s->d_pgs_vpos.alloc((size_t)std::max<int64_t>(num_envs * M.nv, 1)));
@@ -828,7 +831,7 @@ static hipError_t launch_plain(ph_sim* s, const ph_launch_shape& sh, int64_t beg
         const unsigned g4 = (unsigned)std::min<int64_t>((envs + 3) / 4, resident);
         void* sargs[] = {&mp, &sp, &begin, &end, &vel, &vpos, (void*)&slice, &counter};
         if (hipError_t e = hipLaunchKernel(pgs_rows_kernel(s->M), dim3(g4), dim3(64), sargs, slds, s->stream)) return e;
-        wide = (unsigned)std::min<int64_t>(envs, 4 * s->cus);  // few envs or none are left to the other kernel
+        wide = general_sweep_blocks(envs, s->pgs_wide_per_cu, s->cus);
       }
       hipLaunchKernelGGL(k_pgs_sweeps<1>, dim3(wide), dim3(64), 0, s->stream, mp, sp, begin, end, vel, vpos);
       void* bargs[] = {&mp, &sp, &begin, &end, &nstep, &t, &qpos_out, &cvel, &cvpos};

@@ -18,6 +18,7 @@
 #include "../../include/pippin_hip.h"
 #include "../../pippin_amd/csrc/host_model.hpp"
 #include "../../pippin_amd/csrc/kbody.hpp"
+#include "../../pippin_amd/csrc/launch_rules.hpp"
 
 using namespace phk;
 
@@ -88,6 +89,9 @@ static thread_local std::string g_err;
 extern "C" {
 
 const char* emu_last_error(void) { return g_err.c_str(); }
+
+// launch rules (launch_rules.hpp)
+unsigned emu_general_sweep_blocks(int64_t envs, int per_cu, int cus) { return general_sweep_blocks(envs, per_cu, cus); }
 
 emu_sim* emu_create(const ph_model_desc* desc, int64_t n) {
   emu_sim* s = new emu_sim();
