@@ -343,7 +343,8 @@ int pippin_hip_set_launch_shape(ph_sim* s, const ph_launch_shape* shape);
  * calls (without the learned warm start) cycle through every valid shape for
  * 1 + `rounds` rounds, timing each
  * launch per env-step (the first round is not timed), then keep the shape with
- * the lowest median. With `cache_path` (or NULL), a shape stored there for this
+ * the lowest median, or PH_SCHED_WS_BUCKET of the same kernel where one of its
+ * launches was no slower than that median. With `cache_path` (or NULL), a shape stored there for this
  * model's sizes, env count and device is taken at once, and a tuned one is
  * appended as a line "key : K specialised schedule". */
 int pippin_hip_autotune(ph_sim* s, int32_t rounds, const char* cache_path);

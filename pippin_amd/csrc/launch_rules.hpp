@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <vector>
 
 namespace phk {
 
@@ -17,6 +18,29 @@ namespace phk {
 // packed, 4096 Ants walking, 1.80 ms either way).
 inline unsigned general_sweep_blocks(int64_t envs, int per_cu, int cus) {
   return (unsigned)std::min<int64_t>(envs, (int64_t)std::max(per_cu, 4) * std::max(cus, 1));
+}
+
+// Which of an autotuning's candidates to keep, by the times of their timed
+// launches (one entry per round; none: not timed): the lowest median. prefer
+// names a candidate to take instead of another, -1 for none: it is taken where
+// the trials do not tell the two apart, that is where its fastest launch was no
+// slower than the median of the lowest. Returns -1 when nothing was timed.
+inline int tune_choice(const std::vector<std::vector<double>>& ms, const std::vector<int>& prefer) {
+  int best = -1;
+  double least = 0.0;
+  for (size_t c = 0; c < ms.size(); c++) {
+    if (ms[c].empty()) continue;
+    std::vector<double> v = ms[c];
+    std::sort(v.begin(), v.end());
+    const double med = v[v.size() / 2];
+    if (best < 0 || med < least) {
+      least = med;
+      best = (int)c;
+    }
+  }
+  if (best < 0 || prefer[best] < 0) return best;
+  const std::vector<double>& v = ms[prefer[best]];
+  return !v.empty() && *std::min_element(v.begin(), v.end()) <= least ? prefer[best] : best;
 }
 
 }  // namespace phk

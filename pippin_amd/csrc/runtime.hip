@@ -915,35 +915,22 @@ static std::string tune_key(const ph_sim* s) {
   return k;
 }
 
-// The candidate with the lowest median; the bucketed order of the same kernel
-// where it lies within 5 % of that. What buckets gain depends on how well an
-// env's last launch predicts its next one: on steps that move on, as the trials
-// do, grid and buckets of the Ant kernel are within 3 % of each other, and on
-// launches from the same states (planning, line searches over controls) the
-// buckets are 16 % faster (1.53 against 1.28 ms at 16384 envs, 4 steps).
+// Keeps the candidate with the lowest median, or the bucketed order of the same
+// kernel where the trials do not tell the two apart (tune_choice): what buckets
+// gain depends on how well an env's last launch predicts its next one. On steps
+// that move on, as the trials do, grid and buckets of the Ant kernel are within 3 %
+// of each other; on launches from the same states (planning, line searches over
+// controls) the buckets are 16 % faster (1.53 against 1.28 ms at 16384 envs, 4 steps).
 static void tune_finish(ph_sim* s) {
-  double best = 0.0;
-  int bi = -1;
-  std::vector<double> med(s->tune_cand.size(), -1.0);
-  for (size_t c = 0; c < s->tune_cand.size(); c++) {
-    std::vector<double> v = s->tune_ms[c];
-    if (v.empty()) continue;
-    std::sort(v.begin(), v.end());
-    med[c] = v[v.size() / 2];
-    if (bi < 0 || med[c] < best) {
-      best = med[c];
-      bi = (int)c;
-    }
-  }
-  if (bi >= 0)
-    for (size_t c = 0; c < s->tune_cand.size(); c++) {
-      const ph_launch_shape &x = s->tune_cand[c], &y = s->tune_cand[bi];
+  std::vector<int> bucket(s->tune_cand.size(), -1);
+  for (size_t c = 0; c < s->tune_cand.size(); c++)
+    for (size_t b = 0; b < s->tune_cand.size(); b++) {
+      const ph_launch_shape &x = s->tune_cand[b], &y = s->tune_cand[c];
       if (x.schedule == PH_SCHED_WS_BUCKET && y.schedule != PH_SCHED_PGS_SPLIT && x.envs_per_wave == y.envs_per_wave &&
-          x.specialised == y.specialised && med[c] >= 0.0 && med[c] <= 1.05 * best) {
-        bi = (int)c;
-        break;
-      }
+          x.specialised == y.specialised)
+        bucket[c] = (int)b;
     }
+  const int bi = tune_choice(s->tune_ms, bucket);
   if (bi >= 0) {
     const ph_launch_shape& sh = s->tune_cand[bi];
     s->envs_per_wg = sh.envs_per_wave;

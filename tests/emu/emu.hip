@@ -92,6 +92,14 @@ const char* emu_last_error(void) { return g_err.c_str(); }
 
 // launch rules (launch_rules.hpp)
 unsigned emu_general_sweep_blocks(int64_t envs, int per_cu, int cus) { return general_sweep_blocks(envs, per_cu, cus); }
+// ms: ncand x rounds, a negative time for a launch that was not timed
+int emu_tune_choice(const double* ms, const int* prefer, int ncand, int rounds) {
+  std::vector<std::vector<double>> v(ncand);
+  for (int c = 0; c < ncand; c++)
+    for (int r = 0; r < rounds; r++)
+      if (ms[c * rounds + r] >= 0.0) v[c].push_back(ms[c * rounds + r]);
+  return tune_choice(v, std::vector<int>(prefer, prefer + ncand));
+}
 
 emu_sim* emu_create(const ph_model_desc* desc, int64_t n) {
   emu_sim* s = new emu_sim();

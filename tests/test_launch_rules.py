@@ -1,7 +1,8 @@
 """The host's launch rules (pippin_amd/csrc/launch_rules.hpp), without a device."""
+import numpy as np
 import pytest
 
-from tests.emu.pyemu import lib
+from tests.emu.pyemu import _p, lib
 
 
 @pytest.mark.parametrize("envs", [1, 7, 1023, 1024, 1025, 5120, 8192, 16384])
@@ -9,3 +10,27 @@ from tests.emu.pyemu import lib
 def test_the_general_sweeps_fill_the_device(envs, per_cu, cus):
     """Every env of a batch may be left to them: a wavefront each, as far as the device holds them."""
     assert lib().emu_general_sweep_blocks(envs, per_cu, cus) == min(envs, per_cu * cus)
+
+
+# candidates: grid, stealing and buckets of one kernel, the same of another, the split step
+@pytest.mark.parametrize("times,want", [
+    # the lowest median, wherever it is
+    ([[9, 9, 9], [8, 8, 8], [9, 9, 9], [7, 7, 7], [6, 6, 6], [7, 7, 7], [8, 8, 8]], 4),
+    ([[9, 9, 9], [8, 8, 8], [9, 9, 9], [7, 7, 7], [7, 7, 7], [7, 7, 7], [1, 1, 1]], 6),
+    # buckets 3 % slower in every launch: told apart, so not taken
+    ([[1.00, 1.01, 0.99], [2, 2, 2], [1.03, 1.04, 1.02], [2, 2, 2], [2, 2, 2], [2, 2, 2], [2, 2, 2]], 0),
+    # buckets with a launch as fast: not told apart
+    ([[1.00, 1.03, 0.99], [2, 2, 2], [1.02, 1.00, 1.04], [2, 2, 2], [2, 2, 2], [2, 2, 2], [2, 2, 2]], 2),
+    # one slow launch of the other does not make buckets that are slower in every launch its equal
+    ([[1.00, 5.00, 1.01], [2, 2, 2], [1.20, 1.21, 1.20], [2, 2, 2], [2, 2, 2], [2, 2, 2], [2, 2, 2]], 0),
+    # only of the same kernel, and not instead of the split step
+    ([[1.00, 1.00, 1.00], [2, 2, 2], [3, 3, 3], [2, 2, 2], [2, 2, 2], [0.9, 1.1, 1.1], [2, 2, 2]], 0),
+    ([[2, 2, 2], [2, 2, 2], [0.9, 1.1, 1.1], [2, 2, 2], [2, 2, 2], [2, 2, 2], [1.00, 1.00, 1.00]], 6),
+    # not timed
+    ([[-1, -1, -1], [-1, -1, -1], [-1, -1, -1], [2, 2, 2], [-1] * 3, [-1] * 3, [-1] * 3], 3),
+    ([[-1] * 3] * 7, -1),
+])
+def test_autotuning_keeps_what_its_trials_show(times, want):
+    ms = np.array(times, dtype=np.float64)
+    prefer = np.array([2, 2, 2, 5, 5, 5, -1], dtype=np.int32)
+    assert lib().emu_tune_choice(_p(ms), _p(prefer), *ms.shape) == want
