@@ -311,8 +311,11 @@ int pippin_hip_state_device(ph_sim* s, int32_t field, double** ptr);
  * buffer, ordered on the library stream before the next step (no host sync);
  * pippin_hip_get and pippin_hip_set wait for it. */
 int pippin_hip_set_device(ph_sim* s, int32_t field, int64_t begin, int64_t end, const double* src);
-/* Accumulated device time of the step kernel (hipEvents around each launch on the
- * library stream) and the number of launches since the last reset. */
+/* Accumulated device time of the step launches and their number since the last
+ * reset. A PH_SCHED_GRID launch counts its kernel alone (the dispatch's own time
+ * stamps); the other schedules, the learned warm start and autotuning trials
+ * count the time between hipEvents recorded around their launches on the library
+ * stream, which is some microseconds more. */
 int pippin_hip_kernel_timing(ph_sim* s, int32_t reset, double* total_ms, int64_t* launches);
 /* Stream the library launches on (a hipStream_t). */
 void* pippin_hip_stream(ph_sim* s);
@@ -341,8 +344,8 @@ int pippin_hip_get_launch_shape(const ph_sim* s, ph_launch_shape* out);
 int pippin_hip_set_launch_shape(ph_sim* s, const ph_launch_shape* shape);
 /* Online autotuning: the following pippin_hip_step and pippin_hip_rollout_device
  * calls (without the learned warm start) cycle through every valid shape for
- * 1 + `rounds` rounds, timing each
- * launch per env-step (the first round is not timed), then keep the shape with
+ * 1 + `rounds` rounds, timing each launch per env-step between hipEvents, the
+ * same for every shape (the first round is not timed), then keep the shape with
  * the lowest median, or PH_SCHED_WS_BUCKET of the same kernel where one of its
  * launches was no slower than that median. With `cache_path` (or NULL), a shape stored there for this
  * model's sizes, env count and device is taken at once, and a tuned one is

@@ -20,6 +20,14 @@ inline unsigned general_sweep_blocks(int64_t envs, int per_cu, int cus) {
   return (unsigned)std::min<int64_t>(envs, (int64_t)std::max(per_cu, 4) * std::max(cus, 1));
 }
 
+// Whether a launch carries its own time stamps. A grid launch of the plain step
+// is a single dispatch and can, which saves two event records (cartpole, one
+// env: 30 us by the dispatch, 33 to 39 us between records). An autotuning's trials
+// do not: other schedules are sequences that are timed between records, and on
+// launches of some tens of microseconds the two clocks differ by more than the
+// candidates.
+inline bool timed_by_dispatch(bool plain, bool trial, bool grid) { return plain && !trial && grid; }
+
 // Which of an autotuning's candidates to keep, by the times of their timed
 // launches (one entry per round; none: not timed): the lowest median. prefer
 // names a candidate to take instead of another, -1 for none: it is taken where

@@ -1054,9 +1054,9 @@ static int timed_launch(ph_sim* s, int64_t begin, int64_t end, int64_t nstep, co
   const bool trial = plain && s->tune_rounds > 0 && nstep > 0;
   const ph_launch_shape sh = trial ? s->tune_cand[s->tune_next] : current_shape(s);
   *s->pin.failed() = 0;
-  // the grid schedule is one launch, which carries its own time stamps; a
-  // sequence is replayed from a graph between two event records
-  const bool one = plain && sh.schedule == PH_SCHED_GRID;
+  // one launch can carry its own time stamps; a sequence is replayed from a
+  // graph between two event records
+  const bool one = timed_by_dispatch(plain, trial, sh.schedule == PH_SCHED_GRID);
   if (one) {
     HIPCHK(launch_plain(s, sh, begin, end, nstep, ctrl, qpos_out, s->ev0, s->ev1));
   } else {

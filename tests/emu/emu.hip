@@ -92,6 +92,7 @@ const char* emu_last_error(void) { return g_err.c_str(); }
 
 // launch rules (launch_rules.hpp)
 unsigned emu_general_sweep_blocks(int64_t envs, int per_cu, int cus) { return general_sweep_blocks(envs, per_cu, cus); }
+int emu_timed_by_dispatch(int plain, int trial, int grid) { return timed_by_dispatch(plain, trial, grid); }
 // ms: ncand x rounds, a negative time for a launch that was not timed
 int emu_tune_choice(const double* ms, const int* prefer, int ncand, int rounds) {
   std::vector<std::vector<double>> v(ncand);

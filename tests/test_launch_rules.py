@@ -34,3 +34,12 @@ def test_autotuning_keeps_what_its_trials_show(times, want):
     ms = np.array(times, dtype=np.float64)
     prefer = np.array([2, 2, 2, 5, 5, 5, -1], dtype=np.int32)
     assert lib().emu_tune_choice(_p(ms), _p(prefer), *ms.shape) == want
+
+
+def test_trials_are_timed_alike():
+    """One clock for every candidate of an autotuning; a grid launch outside of it stamps itself."""
+    by_dispatch = lib().emu_timed_by_dispatch
+    assert {by_dispatch(1, 1, grid) for grid in (0, 1)} == {0}
+    assert by_dispatch(1, 0, 1) == 1
+    assert {by_dispatch(0, trial, grid) for trial in (0, 1) for grid in (0, 1)} == {0}
+    assert by_dispatch(1, 0, 0) == 0
