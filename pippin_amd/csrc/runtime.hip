@@ -903,10 +903,12 @@ static bool shape_valid(const ph_sim* s, const ph_launch_shape& sh) {
 }
 
 // Key of an autotuned shape: the model's sizes and layout, env count, device.
+// The version goes up when the step kernels or the schedules change so much that
+// shapes measured before say nothing (v2: packed PGS rows, islands side by side).
 static std::string tune_key(const ph_sim* s) {
   const DModel& M = s->M;
   char buf[256];
-  snprintf(buf, sizeof buf, "v1 nq%d nv%d nu%d nb%d ng%d np%d nc%d nr%d sk%d it%d L%d n%lld %s cu%d", M.nq, M.nv, M.nu,
+  snprintf(buf, sizeof buf, "v2 nq%d nv%d nu%d nb%d ng%d np%d nc%d nr%d sk%d it%d L%d n%lld %s cu%d", M.nq, M.nv, M.nu,
            M.nbody, M.ngeom, M.npair, M.ncmax, M.nrmax, M.solver_kind, M.iterations, M.L.bytes, (long long)s->n,
            s->arch.c_str(), s->cus);
   std::string k = buf;

@@ -218,3 +218,24 @@ def test_autotune_cache_is_keyed_by_env_count(assets, tmp_path):
     assert not k.autotune_pending() and k.launch_shape() == g.launch_shape()
     for s in (g, h, k):
         s.close()
+
+
+def test_shapes_tuned_for_earlier_kernels_are_not_taken(tmp_path):
+    """A line of an earlier version names a shape that was measured on other
+    kernels (fused PGS, before its rows were packed): the shapes are tried again."""
+    arr = {**mjcf.load_string(random_pile_xml(29)), "solver_kind": 1}
+    cache = tmp_path / "shapes.txt"
+    g = HipPhysics(arr, 3)
+    g.autotune(rounds=1, cache_path=cache)
+    while g.autotune_pending():
+        g.step(0, 3, 1)
+    g.close()
+    key = cache.read_text().split(" : ")[0]
+    cache.write_text(f"v1{key[2:]} : 1 0 0\n")
+    h = HipPhysics(arr, 3)
+    h.autotune(rounds=1, cache_path=cache)
+    assert h.autotune_pending() and h.launch_shape()[2] == "pgs_split"
+    cache.write_text(f"{key} : 1 0 0\n")
+    h.autotune(rounds=1, cache_path=cache)
+    assert not h.autotune_pending() and h.launch_shape() == (1, 0, "grid")
+    h.close()
