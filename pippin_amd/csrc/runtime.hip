@@ -469,29 +469,13 @@ extern "C" int pippin_hip_create(const ph_model_desc* desc, int64_t num_envs, co
   phh::init_dmodel_scalars(hm, solver, opt ? opt->max_contacts : 0, M);
   M.hess_mfma = opt && opt->hessian_mfma ? 1 : 0;
   if (M.L.bytes > 64 * 1024) return fail(PH_ERR_MODEL, "model too large for the per-env LDS working set");
-  // Pack as many envs per workgroup as fit 64 KiB of LDS (PIPPIN_HIP_ENVS_PER_WG overrides: 1, 2 or 4,
-  // up to the device's per-workgroup LDS).
   hipDeviceProp_t prop;
   HIPCHK(hipGetDeviceProperties(&prop, s->device));
   const int64_t lds_max = (int64_t)prop.sharedMemPerBlock;
-  s->envs_per_wg = 1;
-  for (int k : {4, 2})
-    if (k * M.L.bytes <= 64 * 1024) {
-      s->envs_per_wg = k;
-      break;
-    }
-  // PGS models with packed rows start with the split step: fused, the sweeps of
-  // several envs wait for each other at every row (Ant, 4096 envs, 4 steps: 9.9
-  // ms fused, 1.84 ms split; six-body pile, 8192 envs: 125 and 11.0 ms)
-  if (M.solver_kind == 1 && M.pgs_w > 0) {
-    s->envs_per_wg = 1;
-    s->sched = PH_SCHED_PGS_SPLIT;
-  }
-  if (const char* ev = std::getenv("PIPPIN_HIP_ENVS_PER_WG")) {
-    s->sched = PH_SCHED_GRID;
-    int k = std::atoi(ev);
-    if ((k == 1 || k == 2 || k == 4) && (int64_t)k * M.L.bytes <= lds_max) s->envs_per_wg = k;
-  }
+  const StartShape first = start_shape(M.L.bytes, M.solver_kind == 1 && M.pgs_w > 0, lds_max,
+                                       std::getenv("PIPPIN_HIP_ENVS_PER_WG"));
+  s->envs_per_wg = first.envs_per_wave;
+  s->sched = first.schedule;
   // model-specialised kernel when the model's sizes and layout match one built
   // in (PIPPIN_HIP_SPEC=0 forces the generic kernel)
   s->spec = SpecAnt::matches(M) && M.solver_kind == 0 ? 1 : 0;

@@ -92,6 +92,12 @@ const char* emu_last_error(void) { return g_err.c_str(); }
 
 // launch rules (launch_rules.hpp)
 unsigned emu_general_sweep_blocks(int64_t envs, int per_cu, int cus) { return general_sweep_blocks(envs, per_cu, cus); }
+int emu_start_shape(int64_t lds_bytes, int packed_pgs, int64_t lds_max, const char* asked, int* k, int* sched) {
+  const StartShape sh = start_shape(lds_bytes, packed_pgs, lds_max, asked);
+  *k = sh.envs_per_wave;
+  *sched = sh.schedule;
+  return 0;
+}
 int emu_timed_by_dispatch(int plain, int trial, int grid) { return timed_by_dispatch(plain, trial, grid); }
 // ms: ncand x rounds, a negative time for a launch that was not timed
 int emu_tune_choice(const double* ms, const int* prefer, int ncand, int rounds) {

@@ -97,3 +97,12 @@ def test_split_pgs_step_equals_the_oracle(assets, name, n):
         assert np.array_equal(o.get("qvel"), g.get("qvel")), t
     say("  rows up to", rows)
     g.close()
+
+
+@pytest.mark.parametrize("asked,want", [("3", (1, 0, "pgs_split")), ("", (1, 0, "pgs_split")), ("2", (2, 0, "grid"))])
+def test_envs_per_wavefront_from_the_environment(assets, monkeypatch, asked, want):
+    """A value that is not taken leaves a PGS model with the split step."""
+    monkeypatch.setenv("PIPPIN_HIP_ENVS_PER_WG", asked)
+    g = HipPhysics({**mjcf.load_file(assets / "ant.xml"), "solver_kind": 1}, 2)
+    assert g.launch_shape() == want
+    g.close()

@@ -1,8 +1,28 @@
 """The host's launch rules (pippin_amd/csrc/launch_rules.hpp), without a device."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from tests.emu.pyemu import _p, lib
+
+GRID, SPLIT = 0, 3
+
+
+@pytest.mark.parametrize("kib,packed,asked,want", [
+    (4, False, None, (4, GRID)), (16, False, None, (4, GRID)), (17, False, None, (2, GRID)),
+    (33, False, None, (1, GRID)), (4, True, None, (1, SPLIT)), (33, True, None, (1, SPLIT)),
+    # a number of envs per wavefront that is asked for, with or without room
+    (4, False, b"2", (2, GRID)), (4, True, b"4", (4, GRID)), (4, True, b"1", (1, GRID)),
+    (40, False, b"4", (4, GRID)), (41, False, b"4", (1, GRID)), (41, True, b"4", (1, SPLIT)),
+    # and values that are not taken: the shape is as if nothing had been asked for
+    (4, False, b"3", (4, GRID)), (4, True, b"3", (1, SPLIT)), (4, True, b"", (1, SPLIT)), (4, True, b"no", (1, SPLIT)),
+    (4, True, b"-4", (1, SPLIT)), (4, True, b"0", (1, SPLIT)),
+])
+def test_the_shape_a_sim_starts_with(kib, packed, asked, want):
+    k, sched = C.c_int(-1), C.c_int(-1)
+    lib().emu_start_shape(kib * 1024, packed, 160 * 1024, asked, C.byref(k), C.byref(sched))
+    assert (k.value, sched.value) == want
 
 
 @pytest.mark.parametrize("envs", [1, 7, 1023, 1024, 1025, 5120, 8192, 16384])
