@@ -32,6 +32,41 @@ inline StartShape start_shape(int64_t lds_bytes, bool packed_pgs, int64_t lds_ma
   return {1, PH_SCHED_GRID};
 }
 
+// Envs per wavefront of the split PGS step's front and back and of the pose
+// kernel, for envs of lds_bytes each. A round of wavefronts takes about
+// 1 : 1.2 : 1.5 for 1, 2 and 4 envs (the generic Ant kernel: 344, 410 and 520 us
+// per 4-step round), so the fewest rounds win once the device is full, and one
+// env per wavefront while it is not.
+inline int envs_per_wave_by_rounds(int64_t lds_bytes, int cus, int64_t envs) {
+  const double weight[] = {1.0, 1.2, 1.5};
+  int best = 1;
+  double cost = 0.0;
+  for (int i = 0; i < 3; i++) {
+    const int K = 1 << i;
+    const int64_t lds = K * lds_bytes;
+    if (lds > 64 * 1024) break;
+    const int64_t resident = (int64_t)cus * std::min<int64_t>(4, 160 * 1024 / lds), waves = (envs + K - 1) / K;
+    const double c = weight[i] * (double)((waves + resident - 1) / resident);
+    if (i == 0 || c < cost) {
+      best = K;
+      cost = c;
+    }
+  }
+  return best;
+}
+
+// Envs per wavefront of the step with the learned warm start: the launch
+// shape's, except that the split PGS step's has none to give (its front and back
+// pick theirs by the range) and the learned step runs fused. Several envs of a
+// wavefront wait for each other at every row there, so with several dof blocks
+// one env is the best throughout (six-body pile, 4096 envs, 4 steps: 11.4 ms with
+// 1, 37 with 2, 46 with 4; three boxes 3.7, 6.4, 6.9). A single tree has few rows,
+// and the rounds decide (Ant, 1024 envs: 2.2, 3.7, 4.0 ms; 4096: 8.5, 7.9, 5.3).
+inline int learned_envs_per_wave(int shape_envs, bool split, int nblock, int64_t lds_bytes, int cus, int64_t envs) {
+  if (!split) return shape_envs;
+  return nblock > 1 ? 1 : envs_per_wave_by_rounds(lds_bytes, cus, envs);
+}
+
 // Workgroups of the PGS sweeps over rows that are not packed (k_pgs_sweeps),
 // which follow the packed sweeps: as many as the device holds of them. Usually
 // few envs or none are left to them, and their wavefronts end after reading row

@@ -762,28 +762,6 @@ static unsigned ws_grid(const ph_sim* s, int K, int spec, int64_t nslots) {
   return (unsigned)std::min<int64_t>((int64_t)per_cu * s->cus, nslots);
 }
 
-// Envs per wavefront of the split PGS step's front and back. A round of
-// wavefronts takes about 1 : 1.2 : 1.5 for 1, 2 and 4 envs (the generic Ant
-// kernel: 344, 410 and 520 us per 4-step round), so the fewest rounds win
-// once the device is full, and one env per wavefront while it is not.
-static int split_envs_per_wave(const ph_sim* s, int64_t envs) {
-  const double weight[] = {1.0, 1.2, 1.5};
-  int best = 1;
-  double cost = 0.0;
-  for (int i = 0; i < 3; i++) {
-    const int K = 1 << i;
-    const int64_t lds = (int64_t)K * s->M.L.bytes;
-    if (lds > 64 * 1024) break;
-    const int64_t resident = (int64_t)s->cus * std::min<int64_t>(4, 160 * 1024 / lds), waves = (envs + K - 1) / K;
-    const double c = weight[i] * (double)((waves + resident - 1) / resident);
-    if (i == 0 || c < cost) {
-      best = K;
-      cost = c;
-    }
-  }
-  return best;
-}
-
 // The step without the learned warm start in the given launch shape, with
 // optional per-step controls and qpos outputs (Batch::rollout). Only kernels
 // go on the stream, so the sequence can be captured in a graph.
@@ -796,7 +774,7 @@ static hipError_t launch_plain(ph_sim* s, const ph_launch_shape& sh, int64_t beg
   const DState* sp = s->d_state.p;
   if (sh.schedule == PH_SCHED_PGS_SPLIT) {  // front, sweeps and back of each physics step
     const int64_t envs = end - begin;
-    const int FK = split_envs_per_wave(s, envs);
+    const int FK = envs_per_wave_by_rounds(s->M.L.bytes, s->cus, envs);
     const unsigned grid = (unsigned)((envs + FK - 1) / FK);
     const size_t flds = (size_t)FK * s->M.L.bytes;
     double* vel = s->d_pgs_vel.p;
@@ -859,7 +837,8 @@ static ph_launch_shape current_shape(const ph_sim* s) {
 static hipError_t launch_step(ph_sim* s, int64_t begin, int64_t end, int64_t nstep, const Real* ctrl,
                               Real* qpos_out) {
   if (!s->M.mlp.mode) return launch_plain(s, current_shape(s), begin, end, nstep, ctrl, qpos_out);
-  const int K = s->envs_per_wg;
+  const int K = learned_envs_per_wave(s->envs_per_wg, s->sched == PH_SCHED_PGS_SPLIT, s->M.nblock, s->M.L.bytes, s->cus,
+                                      end - begin);
   const unsigned grid = (unsigned)((end - begin + K - 1) / K);
   const size_t lds = step_lds(s, K);
   phm::launch_step(K, s->spec, grid, lds, s->stream, s->d_model.p, s->d_state.p, begin, end, nstep, ctrl, qpos_out);
@@ -1223,7 +1202,7 @@ extern "C" int pippin_hip_reset_noalloc(ph_sim* s, const int64_t* envs, int64_t 
 static int refresh_poses(const ph_sim* s) {
   if (!s->poses_stale && !s->qpos_shared) return PH_OK;
   HIPCHK(hipSetDevice(s->device));
-  const int K = split_envs_per_wave(s, s->n);
+  const int K = envs_per_wave_by_rounds(s->M.L.bytes, s->cus, s->n);
   const dim3 grid((unsigned)((s->n + K - 1) / K));
   const size_t lds = (size_t)K * s->M.L.bytes;
   if (K == 4) hipLaunchKernelGGL(k_kin<4>, grid, dim3(64), lds, s->stream, s->d_model.p, s->d_state.p);

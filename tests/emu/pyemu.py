@@ -29,7 +29,8 @@ def lib():
         L.emu_last_error.restype = C.c_char_p
         L.emu_general_sweep_blocks.restype = C.c_uint
         L.emu_general_sweep_blocks.argtypes = [i64, C.c_int, C.c_int]
-        for n, a in {"emu_start_shape": [i64, C.c_int, i64, C.c_char_p, vp, vp], "emu_tune_choice": [vp, vp, C.c_int, C.c_int],
+        for n, a in {"emu_learned_envs_per_wave": [C.c_int, C.c_int, C.c_int, i64, C.c_int, i64],
+                     "emu_start_shape": [i64, C.c_int, i64, C.c_char_p, vp, vp], "emu_tune_choice": [vp, vp, C.c_int, C.c_int],
                      "emu_timed_by_dispatch": [C.c_int, C.c_int, C.c_int], "emu_step": [vp, i64, i64, i64], "emu_step_split": [vp, i64, i64, i64, i64], "emu_get": [vp, C.c_int, i64, i64, vp],
                      "emu_set": [vp, C.c_int, i64, i64, vp], "emu_ncon": [vp, i64, i64, vp],
                      "emu_iters": [vp, i64, i64, vp], "emu_status": [vp, i64, i64, vp],

@@ -106,3 +106,33 @@ def test_envs_per_wavefront_from_the_environment(assets, monkeypatch, asked, wan
     g = HipPhysics({**mjcf.load_file(assets / "ant.xml"), "solver_kind": 1}, 2)
     assert g.launch_shape() == want
     g.close()
+
+
+def test_learned_pgs_step_is_the_same_for_every_number_of_envs_per_wavefront(assets):
+    """The split step's shape leaves the number to the range: 4 for these 2053
+    Ants (a ragged last wavefront), 1 for the ranges that fit the device."""
+    n = 2053
+    arr = {**mjcf.load_file(assets / "ant.xml"), "solver_kind": 1}
+    rng = np.random.default_rng(2)
+    runs = []
+    for shape in (None, (1, 0, "grid"), (2, 0, "grid"), (4, 0, "grid")):
+        say("learned PGS", shape)
+        g = HipPhysics(arr, n)
+        if shape:
+            g.set_launch_shape(*shape)
+        if not runs:
+            q = g.get("qpos")
+            q[:, 2] = rng.uniform(0.3, 0.6, n)
+            c = rng.uniform(-1, 1, (n, 8))
+        g.set("qpos", 0, n, q)
+        g.set("ctrl", 0, n, c)
+        g.mlp_init(hidden=32, seed=5)
+        g.mlp_mode(3)
+        for b, e, k in [(0, n, 20), (7, 900, 3), (0, n, 2)]:
+            g.step(b, e, k)
+        runs.append([g.get("qpos"), g.get("qvel"), g.ncon(), g.solver_iterations()])
+        g.close()
+    assert runs[0][2].sum() > n
+    for r in runs[1:]:
+        for a, b in zip(runs[0], r):
+            assert np.array_equal(a, b)

@@ -63,3 +63,15 @@ def test_trials_are_timed_alike():
     assert by_dispatch(1, 0, 1) == 1
     assert {by_dispatch(0, trial, grid) for trial in (0, 1) for grid in (0, 1)} == {0}
     assert by_dispatch(1, 0, 0) == 0
+
+
+@pytest.mark.parametrize("nblock,kib,envs,want", [
+    (1, 10, 1, 1), (1, 10, 1024, 1), (1, 10, 1025, 2), (1, 10, 2048, 2), (1, 10, 2049, 4), (1, 10, 4096, 4),
+    (1, 10, 16384, 4), (1, 33, 16384, 1), (1, 17, 4096, 2), (6, 10, 1, 1), (6, 10, 4096, 1), (2, 4, 16384, 1),
+])
+def test_envs_per_wavefront_of_the_learned_warm_start(nblock, kib, envs, want):
+    """Under the split PGS step's shape by the range; else what the shape says."""
+    rule = lib().emu_learned_envs_per_wave
+    assert rule(1, 1, nblock, kib * 1024, 256, envs) == want
+    for k in (1, 2, 4):
+        assert rule(k, 0, nblock, kib * 1024, 256, envs) == k
