@@ -1761,25 +1761,40 @@ PHD int newton_solve(const MT& M, const DState& S, Env& E, int nr, const Real* w
   // mass-factor slot (per island the Hessian factor, then the gathered
   // problem). One after the other, on 16 of the wavefront's 64 lanes, they
   // were 139 us of a 363 us step on the six-body pile, and gathering them 59.
-  auto doubles = [](int k, int q) { return 2 * k * k + q * k + 2 * q + 4 * k; };
-  auto in_lanes = [&](int id) __attribute__((always_inline)) { return ik[id] <= GL && iq[id] <= GL && doubles(ik[id], iq[id]) <= nv * nv; };
+  // The slot of a model of few bodies is small (two: 144 doubles, of which an
+  // island of 6 dofs and 8 rows needs 160), so an island's rows and vectors go
+  // to the row block where they do not fit beside its matrices: to the row
+  // vectors that newton_dense uses, or to all of it when this step's rows are
+  // elsewhere. (Two capsules, 4096 envs, 4 steps: 558 us by newton_dense, 320 us
+  // so.)
+  const bool rows_here = E.J == LD(J);
+  const LP spare = (LP)(rows_here ? LD(jar) : LD(J));
+  const int slot = nv * nv, spare_n = M.nrl * (rows_here ? 5 : nv + 7);
+  auto beside = [](int k, int q) { return q * k + 2 * q + 4 * k; };
+  auto in_lanes = [&](int id) __attribute__((always_inline)) {
+    const int k = ik[id], q = iq[id], left = slot - 2 * k * k;
+    return k <= GL && q <= GL && left >= 0 && beside(k, q) <= (left > spare_n ? left : spare_n);
+  };
   int iters = 0;
   for (int next = 0; next < ni;) {
     // this row's island of the batch: the row()-th that fits after the ones
     // before it
-    int id = -1, o = 0, po = 0, taken = 0, kmax = 0, used = 0, ints = 0;
+    int id = -1, o = 0, ro = -1, po = 0, taken = 0, kmax = 0, used = 0, spare_used = 0, ints = 0;
     for (; next < ni && taken < X::ROWS; next++) {
       const int c = isl[next];
       if (!in_lanes(c)) continue;
-      const int need = doubles(ik[c], iq[c]);
-      if (used + need > nv * nv) break;
+      const int own = 2 * ik[c] * ik[c], rest = beside(ik[c], iq[c]);
+      const bool in_slot = used + own + rest <= slot;
+      if (!in_slot && (used + own > slot || spare_used + rest > spare_n)) break;
       if (taken == X::row()) {
         id = c;
         o = used;
+        ro = in_slot ? -1 : spare_used;
         po = ints;
       }
       kmax = ik[c] > kmax ? ik[c] : kmax;
-      used += need;
+      used += in_slot ? own + rest : own;
+      spare_used += in_slot ? 0 : rest;
       ints += ik[c] + iq[c];
       taken++;
     }
@@ -1790,8 +1805,8 @@ PHD int newton_solve(const MT& M, const DState& S, Env& E, int nr, const Real* w
       int* rows = dofs + ik[id];
       list(id, dofs, rows, &k, &q, &qi);
       X::order();
-      const LP fac = (LP)LD(chol) + o, sqm = fac + k * k, sJ = sqm + k * k, saref = sJ + q * k, sdd = saref + q,
-               sa = sdd + q, swarm = sa + k, sqf = swarm + k, swarm2 = sqf + k;
+      const LP fac = (LP)LD(chol) + o, sqm = fac + k * k, sJ = ro < 0 ? sqm + k * k : spare + ro, saref = sJ + q * k,
+               sdd = saref + q, sa = sdd + q, swarm = sa + k, sqf = swarm + k, swarm2 = sqf + k;
       X::each([&](int l) {
         if (l < k) {
           const int d = dofs[l];

@@ -118,6 +118,27 @@ GRIPPER = """<mujoco model="gripper">
 """
 
 
+# Free bodies on a plane, named one by one; a "+" after a name puts the next one on top of it.
+# Islands whose gathered problem fits the mass-factor slot (spheres), only with its rows beside
+# the row vectors (two boxes or capsules), in part there (three), or nowhere (a stack of boxes).
+FEW_BODIES = ["sphere sphere", "capsule capsule", "box box", "box capsule", "box box box", "capsule capsule capsule",
+              "box sphere box capsule", "sphere+ sphere sphere", "capsule+ sphere box", "box+ box sphere",
+              "sphere+ sphere+ sphere sphere"]
+
+
+def few_bodies_xml(name: str) -> str:
+    geoms = {"box": '<geom type="box" size=".05 .05 .05"/>', "capsule": '<geom type="capsule" size=".03 .1" euler="0 90 0"/>',
+             "sphere": '<geom type="sphere" size=".05"/>'}
+    bodies, x, z = "", 0.0, 0.0
+    for part in name.split():
+        g = part.rstrip("+")
+        r = 0.03 if g == "capsule" else 0.05
+        bodies += f'<body pos="{x} {0.1 * x * x} {z + r + 0.002}"><freejoint/>{geoms[g]}</body>'
+        x, z = (x + 0.004, z + 2 * r) if part.endswith("+") else (x + 0.5, 0.0)
+    return ('<mujoco><option timestep="0.004"/><worldbody><geom type="plane" size="5 5 .1"/>' + bodies +
+            '</worldbody></mujoco>')
+
+
 from pippin_amd.workloads import random_pile_xml  # noqa: E402,F401  (shared with bench.py)
 
 

@@ -12,8 +12,10 @@ import numpy as np
 import pytest
 
 from oracle import mjcf
+from oracle.pyoracle import OracleSim
 from pippin_amd.physics import HipError, HipPhysics
 from pippin_amd.workloads import random_pile_xml
+from tests.scenes import FEW_BODIES, few_bodies_xml
 
 pytestmark = pytest.mark.gpu
 
@@ -108,6 +110,25 @@ def test_every_shape_matches_on_a_pile(solver):
         say("pile shape", solver, shape)
         got = _run(arr, q, n, shape, 30, 7)
         assert _same(ref, got), shape
+
+
+@pytest.mark.parametrize("name", FEW_BODIES)
+def test_every_shape_matches_the_oracle_on_few_bodies(name):
+    """Islands side by side in the little LDS of models with two to four bodies."""
+    arr = mjcf.load_string(few_bodies_xml(name))
+    n = 5
+    o = OracleSim(arr, n)
+    q = o.get("qpos")
+    q[:, ::7] += 0.001 * np.random.default_rng(4).normal(size=q[:, ::7].shape)
+    o.set("qpos", 0, n, q)
+    ref = []
+    for _ in range(12):
+        o.step(0, n, 4)
+        ref.append((o.get("qpos").copy(), o.ncon().copy()))
+    assert ref[-1][1].min() >= len(name.split())
+    for shape in _valid_shapes(arr, n):
+        say("few bodies", name, shape)
+        assert _same(ref, _run(arr, q, n, shape, 12, 0)), shape
 
 
 def test_autotune_keeps_results_and_caches_its_choice(assets, tmp_path):

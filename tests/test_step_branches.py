@@ -6,6 +6,7 @@ import pytest
 from oracle import mjcf
 from oracle.pyoracle import OracleSim
 from tests.emu.pyemu import EmuSim
+from tests.scenes import FEW_BODIES, few_bodies_xml
 
 
 def _sliders(n, gap, integrator="Euler"):
@@ -43,3 +44,20 @@ def test_contact_copy_past_its_list(n):
         assert np.array_equal(o.ncon(), e.ncon()), t
         assert np.array_equal(o.get("qpos"), e.get("qpos")), t
     assert (o.ncon()[0] > 18 * int(arr["ngeom"])) == (n == 15), o.ncon()
+
+
+@pytest.mark.parametrize("name", FEW_BODIES)
+def test_islands_of_few_bodies(name):
+    arr = mjcf.load_string(few_bodies_xml(name))
+    o, e = OracleSim(arr, 2), EmuSim(arr, 2)
+    q = o.get("qpos")
+    q[1, ::7] += 0.001 * np.arange(q.shape[1] // 7)
+    for s in (o, e):
+        s.set("qpos", 0, 2, q)
+    for t in range(80):
+        for s in (o, e):
+            s.step(0, 2, 1)
+        assert np.array_equal(o.ncon(), e.ncon()), t
+        assert np.array_equal(o.solver_iterations(), e.solver_iterations()), t
+        assert np.array_equal(o.get("qpos"), e.get("qpos")), t
+    assert o.ncon().min() >= len(name.split())
