@@ -118,6 +118,14 @@ GRIPPER = """<mujoco model="gripper">
 """
 
 
+# Boxes on vertical slides over a plane, the first two coupled by a joint equality: PGS rows of
+# one or two dofs, some of them bilateral.
+COUPLED_SLIDERS = ('<mujoco><option timestep="0.004"/><worldbody><geom type="plane" size="5 5 .1"/>' + "".join(
+    f'<body pos="{0.5 * i} 0 {0.11 + 0.01 * i}"><joint name="s{i}" type="slide" axis="0 0 1"/>'
+    f'<geom type="box" size=".1 .1 .1"/></body>' for i in range(3)) +
+    '</worldbody><equality><joint joint1="s0" joint2="s1" polycoef="0.02 0.7 0.1 0 0"/></equality></mujoco>')
+
+
 # Free bodies on a plane, named one by one; a "+" after a name puts the next one on top of it.
 # Islands whose gathered problem fits the mass-factor slot (spheres), only with its rows beside
 # the row vectors (two boxes or capsules), in part there (three), or nowhere (a stack of boxes).

@@ -143,7 +143,8 @@ def test_primitive_pairs_match(name):
 def test_ant_pressed_into_the_floor_matches(assets, shape):
     """Ant states pushed into the floor with bent legs: steps with 17 to 32
     and over 32 constraint rows, more than the 16-row lane solver and LDS row
-    block hold, so they take the dense solver with their rows in HBM. The
+    block hold, so they take the dense solver, past the block with their rows in
+    HBM at 4 envs per wavefront and in the LDS past the layout at 1. The
     Ant-specialised kernel at 4 envs per wavefront and the generic one at 1
     match the oracle bit for bit (contacts, iterations, qpos, qvel)."""
     n, T = 256, 20

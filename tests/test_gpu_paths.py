@@ -6,8 +6,9 @@ import pytest
 
 from oracle import mjcf
 from oracle.pyoracle import OracleSim
-from pippin_amd.physics import HipPhysics
+from pippin_amd.physics import HipError, HipPhysics
 from pippin_amd.workloads import arm_gripper_xml, random_pile_xml
+from tests.scenes import COUPLED_SLIDERS
 
 pytestmark = pytest.mark.gpu
 
@@ -55,19 +56,27 @@ def test_get_and_set_refuse_a_null_buffer(assets, n):
     assert np.array_equal(g.get("qpos"), before)
 
 
-@pytest.mark.parametrize("n", [1, 5, 130])
-@pytest.mark.parametrize("name", ["ant", "pressed", "arm", "pile"])
-def test_split_pgs_step_equals_the_oracle(assets, name, n):
-    """The shape that PGS models start with: one dof block with limits; Ants
-    pressed into the floor, some with more rows than the packed sweeps hold;
-    two blocks with an equality and a tendon; blocks of six dofs."""
+def pgs_model(name, assets):
     if name == "arm":
         arr = mjcf.load_string(arm_gripper_xml(3))
     elif name == "pile":
         arr = mjcf.load_string(random_pile_xml(29))
+    elif name == "sliders":
+        arr = mjcf.load_string(COUPLED_SLIDERS)
     else:
         arr = mjcf.load_file(assets / "ant.xml")
-    arr = {**arr, "solver_kind": 1}
+    return {**arr, "solver_kind": 1}
+
+
+@pytest.mark.parametrize("n", [1, 5, 130])
+@pytest.mark.parametrize("name", ["ant", "pressed", "arm", "pile", "sliders"])
+def test_split_pgs_step_equals_the_oracle(assets, name, n):
+    """The shape that PGS models start with, by the instances of the packed
+    sweeps: one dof block with limits (16 entries, no equality); Ants pressed
+    into the floor, some with more rows than the packed sweeps hold; two blocks
+    with an equality and a tendon (16, equalities); blocks of six dofs (12);
+    blocks of one dof with an equality across two (12, equalities)."""
+    arr = pgs_model(name, assets)
     o, g = OracleSim(arr, n), HipPhysics(arr, n)
     say("split PGS", name, n, g.launch_shape())
     assert g.launch_shape()[2] == "pgs_split"
@@ -96,6 +105,75 @@ def test_split_pgs_step_equals_the_oracle(assets, name, n):
         assert np.array_equal(o.get("qpos"), g.get("qpos")), t
         assert np.array_equal(o.get("qvel"), g.get("qvel")), t
     say("  rows up to", rows)
+    g.close()
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 1e160, 1e200, 1e308])
+@pytest.mark.parametrize("name,dofs", [("pile", (0, 8, 35)), ("ant", (2, 13)), ("arm", (0, 14)), ("sliders", (1,))])
+def test_packed_sweeps_hand_over_what_is_not_finite(assets, name, dofs, value):
+    """A velocity that is not finite before the sweeps, or that overflows at
+    some row of one: the packed sweeps leave the env to the general form from
+    that row on. Equal to the fused step bit for bit, also for the envs that
+    share a wavefront and stay finite."""
+    arr = pgs_model(name, assets)
+    n, before, after = 10, 90, 3
+    say("not finite", name, value)
+    split, fused, calm = HipPhysics(arr, n), HipPhysics(arr, n), HipPhysics(arr, n)
+    assert split.launch_shape()[2] == "pgs_split"
+    fused.set_launch_shape(1, 0, "grid")
+    sims = (split, fused, calm)
+    rng = np.random.default_rng(6)
+    q = split.get("qpos")
+    if name == "pile":
+        q[:, ::7] += rng.normal(0.0, 0.004, q[:, ::7].shape)
+    for s in sims:
+        s.set("qpos", 0, n, q)
+        s.step(0, n, before)
+    hit = [1 + 3 * i for i in range(len(dofs))]  # envs 1, 4, 7: each shares its wavefront with finite ones
+    v = split.get("qvel")
+    for e, d in zip(hit, dofs):
+        v[e, d] = value
+    for s in (split, fused):
+        s.set("qvel", 0, n, v)
+    for _ in range(after):
+        for s in sims:
+            s.step(0, n, 1)
+        for f in ("qpos", "qvel", "qacc"):
+            assert np.array_equal(split.get(f), fused.get(f), equal_nan=True), f
+        for a, b in zip(split.get_history(), fused.get_history()):
+            a, b = ((x if x.dtype.names is None else x["pos"]) for x in (a, b))
+            assert np.array_equal(a, b, equal_nan=True)
+    rest = [e for e in range(n) if e not in hit]
+    assert np.isfinite(split.get("qpos")[rest]).all()
+    assert np.array_equal(split.get("qpos")[rest], calm.get("qpos")[rest])
+    for s in sims:
+        s.close()
+
+
+@pytest.mark.parametrize("steps", [1, 3])
+def test_split_pgs_step_reports_an_env_that_cannot_be_stepped(assets, steps):
+    """A contact capacity that a step of some call exceeds: that call fails, the
+    env keeps its state and reports again, the others go on."""
+    arr = {**mjcf.load_file(assets / "box_drop.xml"), "solver_kind": 1}
+    n = 5
+    g = HipPhysics(arr, n, max_contacts=2)  # a box resting on the plane makes 4
+    assert g.launch_shape()[2] == "pgs_split"
+    q = g.get("qpos")
+    q[1:, [2, 9, 16]] += 5.0  # env 0's bodies land first
+    g.set("qpos", 0, n, q)
+    with pytest.raises(HipError, match=r"capacity exceeded \(env 0\)"):
+        for _ in range(200):
+            g.step(0, n, steps)
+    frozen = g.get("qpos")
+    g.step(1, n, steps)
+    after = g.get("qpos")
+    assert np.array_equal(after[0], frozen[0]) and not (after[1:] == frozen[1:]).all(axis=1).any()
+    with pytest.raises(HipError, match="capacity"):
+        g.step(0, 1, steps)
+    assert np.array_equal(g.get("qpos")[0], frozen[0])
+    g.reset([0])
+    g.step(0, 1, steps)
+    assert not np.array_equal(g.get("qpos")[0], frozen[0])
     g.close()
 
 

@@ -7,7 +7,7 @@ from oracle import mjcf
 from oracle.pyoracle import OracleSim
 from pippin_amd.workloads import arm_gripper_xml, random_pile_xml
 from tests.emu.pyemu import EmuSim
-from tests.scenes import MULTIBODY_SCENES
+from tests.scenes import COUPLED_SLIDERS, MULTIBODY_SCENES
 
 
 def _model(name, assets):
@@ -15,6 +15,8 @@ def _model(name, assets):
         arr = mjcf.load_file(assets / "ant.xml")  # one block of 14 dofs, limits
     elif name == "arm":
         arr = mjcf.load_string(arm_gripper_xml(3))  # blocks of 9 and 6 dofs, an equality, a tendon
+    elif name == "sliders":
+        arr = mjcf.load_string(COUPLED_SLIDERS)  # blocks of 1 dof, an equality across two
     elif name.startswith("seed"):
         arr = mjcf.load_string(random_pile_xml(int(name[4:])))  # blocks of 6 dofs
     else:
@@ -25,7 +27,7 @@ def _model(name, assets):
 
 # capacities: every row packed; none; envs on either side of it
 @pytest.mark.parametrize("cap", [1 << 20, 1, 900])
-@pytest.mark.parametrize("name", ["ant", "arm", "seed3", "seed11", "seed29", *sorted(MULTIBODY_SCENES)])
+@pytest.mark.parametrize("name", ["ant", "arm", "sliders", "seed3", "seed11", "seed29", *sorted(MULTIBODY_SCENES)])
 def test_split_step_equals_the_oracle(assets, name, cap):
     arr = _model(name, assets)
     n, steps = 3, 120
@@ -50,10 +52,11 @@ def test_split_step_equals_the_oracle(assets, name, cap):
 
 
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 1e200, 1e308])
-@pytest.mark.parametrize("dof", [0, 8, 35])
-def test_velocities_that_are_not_finite_spread_as_in_the_general_path(value, dof):
+@pytest.mark.parametrize("name,dof", [("seed29", 0), ("seed29", 8), ("seed29", 35), ("ant", 2), ("ant", 13), ("arm", 0),
+                                      ("arm", 14), ("sliders", 1)])
+def test_velocities_that_are_not_finite_spread_as_in_the_general_path(assets, value, name, dof):
     """A row's zeros outside its blocks still carry 0 * inf = NaN to the other blocks."""
-    arr = {**mjcf.load_string(random_pile_xml(29)), "solver_kind": 1}
+    arr = _model(name, assets)
     n = 2
     a, b = EmuSim(arr, n), EmuSim(arr, n)
     for s in (a, b):
