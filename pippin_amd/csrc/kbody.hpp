@@ -736,8 +736,7 @@ PHD bool factor_solve_blocks(const MT& M, Env& E, const Real* qm, Real h, Real* 
   int* isc = E.si + M.L.i_iscal;
   const int nblock = M.nblock;
   for (int b0 = 0; b0 < nblock; b0 += X::ROWS) {
-    const int blk = b0 + X::row();
-    if (blk < nblock) {
+    PH_ROWS(X, row) if (const int blk = b0 + row; blk < nblock) {
       const int s0 = nblock == 1 ? 0 : M.block_adr[blk], n = nblock == 1 ? nv : M.block_adr[blk + 1] - s0;
       LV r[NM];
 #pragma unroll
@@ -1777,64 +1776,68 @@ PHD int newton_solve(const MT& M, const DState& S, Env& E, int nr, const Real* w
   };
   int iters = 0;
   for (int next = 0; next < ni;) {
-    // this row's island of the batch: the row()-th that fits after the ones
-    // before it
-    int id = -1, o = 0, ro = -1, po = 0, taken = 0, kmax = 0, used = 0, spare_used = 0, ints = 0;
-    for (; next < ni && taken < X::ROWS; next++) {
-      const int c = isl[next];
-      if (!in_lanes(c)) continue;
-      const int own = 2 * ik[c] * ik[c], rest = beside(ik[c], iq[c]);
-      const bool in_slot = used + own + rest <= slot;
-      if (!in_slot && (used + own > slot || spare_used + rest > spare_n)) break;
-      if (taken == X::row()) {
-        id = c;
-        o = used;
-        ro = in_slot ? -1 : spare_used;
-        po = ints;
+    const int from = next;
+    PH_ROWS(X, row) {
+      // this row's island of the batch: the row-th that fits after the ones
+      // before it
+      next = from;
+      int id = -1, o = 0, ro = -1, po = 0, taken = 0, kmax = 0, used = 0, spare_used = 0, ints = 0;
+      for (; next < ni && taken < X::ROWS; next++) {
+        const int c = isl[next];
+        if (!in_lanes(c)) continue;
+        const int own = 2 * ik[c] * ik[c], rest = beside(ik[c], iq[c]);
+        const bool in_slot = used + own + rest <= slot;
+        if (!in_slot && (used + own > slot || spare_used + rest > spare_n)) break;
+        if (taken == row) {
+          id = c;
+          o = used;
+          ro = in_slot ? -1 : spare_used;
+          po = ints;
+        }
+        kmax = ik[c] > kmax ? ik[c] : kmax;
+        used += in_slot ? own + rest : own;
+        spare_used += in_slot ? 0 : rest;
+        ints += ik[c] + iq[c];
+        taken++;
       }
-      kmax = ik[c] > kmax ? ik[c] : kmax;
-      used += in_slot ? own + rest : own;
-      spare_used += in_slot ? 0 : rest;
-      ints += ik[c] + iq[c];
-      taken++;
-    }
-    int it = 0;
-    if (id >= 0) {
-      int k, q, qi;
-      int* dofs = sidx + po;  // the batch's lists, one after the other
-      int* rows = dofs + ik[id];
-      list(id, dofs, rows, &k, &q, &qi);
-      X::order();
-      const LP fac = (LP)LD(chol) + o, sqm = fac + k * k, sJ = ro < 0 ? sqm + k * k : spare + ro, saref = sJ + q * k,
-               sdd = saref + q, sa = sdd + q, swarm = sa + k, sqf = swarm + k, swarm2 = sqf + k;
+      int it = 0;
+      if (id >= 0) {
+        int k, q, qi;
+        int* dofs = sidx + po;  // the batch's lists, one after the other
+        int* rows = dofs + ik[id];
+        list(id, dofs, rows, &k, &q, &qi);
+        X::order();
+        const LP fac = (LP)LD(chol) + o, sqm = fac + k * k, sJ = ro < 0 ? sqm + k * k : spare + ro, saref = sJ + q * k,
+                 sdd = saref + q, sa = sdd + q, swarm = sa + k, sqf = swarm + k, swarm2 = sqf + k;
+        X::each([&](int l) {
+          if (l < k) {
+            const int d = dofs[l];
+            const LP qm = (LP)LD(qm) + d * nv;
+            for (int i = 0; i < k; i++) sqm[l * k + i] = qm[dofs[i]];
+            for (int t = 0; t < q; t++) sJ[t * k + l] = J[rows[t] * nv + d];
+            sa[l] = LD(a)[d];
+            swarm[l] = LD(qacc)[d];
+            if (w2) swarm2[l] = warm2[d];
+          }
+          if (l < q) {
+            saref[l] = E.aref[rows[l]];
+            sdd[l] = E.dd[rows[l]];
+          }
+        });
+        X::order();
+        const NP P{k, q, qi, cap, M.tolerance, sqm, swarm, sa, sqf, fac, swarm2, w2};
+        it = kmax <= 6 ? newton_lanes<X, 6>(M, P, sJ, saref, sdd) : newton_lanes<X, GL>(M, P, sJ, saref, sdd);
+        X::each([&](int l) {
+          if (l < k) {
+            LD(a)[dofs[l]] = sa[l];
+            LD(qfrc_c)[dofs[l]] = sqf[l];
+          }
+        });
+      }
       X::each([&](int l) {
-        if (l < k) {
-          const int d = dofs[l];
-          const LP qm = (LP)LD(qm) + d * nv;
-          for (int i = 0; i < k; i++) sqm[l * k + i] = qm[dofs[i]];
-          for (int t = 0; t < q; t++) sJ[t * k + l] = J[rows[t] * nv + d];
-          sa[l] = LD(a)[d];
-          swarm[l] = LD(qacc)[d];
-          if (w2) swarm2[l] = warm2[d];
-        }
-        if (l < q) {
-          saref[l] = E.aref[rows[l]];
-          sdd[l] = E.dd[rows[l]];
-        }
-      });
-      X::order();
-      const NP P{k, q, qi, cap, M.tolerance, sqm, swarm, sa, sqf, fac, swarm2, w2};
-      it = kmax <= 6 ? newton_lanes<X, 6>(M, P, sJ, saref, sdd) : newton_lanes<X, GL>(M, P, sJ, saref, sdd);
-      X::each([&](int l) {
-        if (l < k) {
-          LD(a)[dofs[l]] = sa[l];
-          LD(qfrc_c)[dofs[l]] = sqf[l];
-        }
+        if (l == 0) its[row] = it;
       });
     }
-    X::each([&](int l) {
-      if (l == 0) its[X::row()] = it;
-    });
     X::sync();
     for (int r = 0; r < X::ROWS; r++) iters = its[r] > iters ? its[r] : iters;
     X::sync();

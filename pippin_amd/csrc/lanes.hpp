@@ -21,6 +21,14 @@ constexpr int GL = 16;  // lanes per environment group
 // in bounds, no branch around the load) and select the value afterwards.
 PHD int clampi(int i, int n) { return i < n ? i : n - 1; }
 
+// A section that each 16-lane row of an env runs for itself: on the device once,
+// with the row that this lane is in; on the host for one row after the other.
+#if defined(__HIP_DEVICE_COMPILE__)
+#define PH_ROWS(X, row) if (const int row = X::row(); true)
+#else
+#define PH_ROWS(X, row) for (int row = 0; row < X::ROWS; row++)
+#endif
+
 // compile-time loop: f(integral_constant<int, I>) for I in [B, E) while f returns true
 template <int B, int E, class F>
 PHD void sfor(F&& f) {
@@ -253,8 +261,8 @@ struct HostLanes {
   static void order() {}
   static void ior(int* p, int v) { *p |= v; }
   static void iadd(int* p, int v) { *p += v; }
-  // 16-lane rows that work on one env, and this lane's (the device policies
-  // own 4, 2 or 1 by their envs per wavefront)
+  // 16-lane rows that work on one env (the device policies own 4, 2 or 1 by
+  // their envs per wavefront); the host takes them in turn (PH_ROWS)
   static constexpr int ROWS = 1;
   static int row() { return 0; }
   template <class P>

@@ -30,6 +30,13 @@ struct HostX : HostLanes {
   static void sync() {}
 };
 
+// One env per wavefront: four 16-lane rows work on it, a block or an island
+// each at a time, and the LDS past the layout takes constraint rows. The rows'
+// sections run one after the other.
+struct HostX4 : HostX {
+  static constexpr int ROWS = 4;
+};
+
 // The network of the learned warm start for one sample, in FP32 with BF16
 // rounding at the device's points (inputs, weights, hidden activations); the
 // sums run sequentially from the bias, where the device's matrix cores
@@ -78,6 +85,7 @@ struct emu_sim {
       grow, islf, gmj;
   std::vector<int> ncon, iters, nrows, status, cgeom, pcgeom, npcon, cost;
   std::vector<double> lds;
+  int rows = 1;  // 16-lane rows per env: 1 or 4
   // learned warm start
   std::vector<float> mlp_P, mlp_feat, mlp_pred, mlp_tgt;
   std::vector<uint16_t> mlp_wbf, mlp_wtbf;
@@ -317,6 +325,16 @@ emu_sim* emu_create(const ph_model_desc* desc, int64_t n) {
 
 void emu_destroy(emu_sim* s) { delete s; }
 
+// 16-lane rows per env of emu_step (without the learned warm start): 4 is one
+// env per wavefront, with exactly the LDS that its launch has
+int emu_rows(emu_sim* s, int rows) {
+  if (rows != 1 && rows != 4) return -1;
+  s->rows = rows;
+  s->lds.assign(s->M.L.bytes / sizeof(double) + (rows == 4 ? s->M.x1 : 16), 0.0);
+  s->lds.shrink_to_fit();
+  return 0;
+}
+
 int emu_step(emu_sim* s, int64_t begin, int64_t end, int64_t nstep) {
   Env E;
   E.s = s->lds.data();
@@ -330,6 +348,8 @@ int emu_step(emu_sim* s, int64_t begin, int64_t end, int64_t nstep) {
     if (poison) std::fill(s->lds.begin(), s->lds.end(), std::numeric_limits<double>::quiet_NaN());
     if (s->M.mlp.mode)
       run_env_mlp<HostXM>(s->M, s->S, E, nstep, nullptr, nullptr, e - begin, true);
+    else if (s->rows == 4)
+      run_env<HostX4>(s->M, s->S, E, nstep, nullptr, nullptr, e - begin);
     else
       run_env<HostX>(s->M, s->S, E, nstep, nullptr, nullptr, e - begin);
   }

@@ -29,7 +29,7 @@ def lib():
         L.emu_last_error.restype = C.c_char_p
         L.emu_general_sweep_blocks.restype = C.c_uint
         L.emu_general_sweep_blocks.argtypes = [i64, C.c_int, C.c_int]
-        for n, a in {"emu_learned_envs_per_wave": [C.c_int, C.c_int, C.c_int, i64, C.c_int, i64],
+        for n, a in {"emu_rows": [vp, C.c_int], "emu_learned_envs_per_wave": [C.c_int, C.c_int, C.c_int, i64, C.c_int, i64],
                      "emu_start_shape": [i64, C.c_int, i64, C.c_char_p, vp, vp], "emu_tune_choice": [vp, vp, C.c_int, C.c_int],
                      "emu_timed_by_dispatch": [C.c_int, C.c_int, C.c_int], "emu_step": [vp, i64, i64, i64], "emu_step_split": [vp, i64, i64, i64, i64], "emu_get": [vp, C.c_int, i64, i64, vp],
                      "emu_set": [vp, C.c_int, i64, i64, vp], "emu_ncon": [vp, i64, i64, vp],
@@ -51,12 +51,14 @@ def _p(a):
 class EmuSim:
     FIELD = {"qpos": 0, "qvel": 1, "ctrl": 2}
 
-    def __init__(self, arrays: dict, n: int):
+    def __init__(self, arrays: dict, n: int, rows: int = 1):
         self.L = lib()
         self.desc = Desc(arrays)
         self.h = self.L.emu_create(self.desc.ptr(), n)
         if not self.h:
             raise RuntimeError(self.L.emu_last_error().decode())
+        if rows != 1 and self.L.emu_rows(self.h, rows) != 0:
+            raise ValueError("rows: 1 or 4")
         self.n = n
         self.nq, self.nv, self.nu = int(arrays["nq"]), int(arrays["nv"]), int(arrays["nu"])
         self.nbody, self.ngeom = int(arrays["nbody"]), int(arrays["ngeom"])
