@@ -329,9 +329,14 @@ enum {
   PH_SCHED_GRID = 0,      /* one workgroup per K envs, dispatched by the hardware */
   PH_SCHED_WS = 1,        /* persistent workgroups taking K envs at a time from a counter */
   PH_SCHED_WS_BUCKET = 2, /* as WS, envs ordered by Newton iterations of their last launch */
-  PH_SCHED_PGS_SPLIT = 3  /* PGS models, K = 1, generic kernel: each physics step as three launches
-                             (up to the sweeps, the sweeps with one env per wavefront and no LDS,
-                             the rest), so that many sweep wavefronts share a SIMD */
+  PH_SCHED_PGS_SPLIT = 3  /* PGS models, generic kernels, given as K = 1: each physics step as a launch up
+                             to the sweeps, the sweeps, and a launch of the rest. A row that touches dof
+                             blocks of at most 16 dofs in all is packed to them, and where every row of a
+                             model can be, the sweeps run four envs per wavefront with their rows in LDS;
+                             a second sweep launch, one env per wavefront in registers, takes the envs with
+                             more rows than that holds (and all envs of other models). The first and last
+                             launches pick 1, 2 or 4 envs per wavefront by the range. Models whose rows
+                             pack start with this schedule. */
 };
 typedef struct ph_launch_shape {
   int32_t envs_per_wave; /* K: 1, 2 or 4 envs per 64-lane wavefront */

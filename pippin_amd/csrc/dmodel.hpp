@@ -97,7 +97,7 @@ struct DModel {
   Real timestep, gravity[3], tolerance, margin, solref[2], solimp[5], impratio, hertz, zeta, slop;
   int ncmax;  // contact capacity per env (the sum of per-pair maxima: never exceeded)
   int nrmax;  // row capacity per env (4 per contact for Newton, 3 for PGS, + limits + equalities)
-  int nrl;    // rows kept in LDS; larger problems use the global row buffers
+  int nrl;    // rows of the LDS row block; more go to the LDS past the layout (x1) or the global row buffers
   // PGS: the most dofs that one row and its M^-1 J^T can hold (the dof blocks of the two
   // bodies of a pair, of a limited joint or of an equality), and the largest such block;
   // 0 when a row can hold more than 16

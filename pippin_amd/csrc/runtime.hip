@@ -507,10 +507,11 @@ extern "C" int pippin_hip_create(const ph_model_desc* desc, int64_t num_envs, co
     if (M.pgs_w > 0) {
       const int64_t rows = 3 * (int64_t)M.ncmax + 2 * hm.nlimited + d.neq;
       const int64_t most = pgs_packed_doubles(M.nv, rows, rows * M.pgs_w);
-      // A single tree of at most 16 dofs meets few contacts: a quarter of the
-      // LDS holds 37 rows of an Ant, and four wavefronts per CU fill its SIMDs
-      // (4096 envs in flight instead of 3072). Piles of bodies need a third
-      // (62 rows of two free bodies).
+      // Models of at most 16 dofs (a tree, or two free bodies) meet few contacts:
+      // a quarter of the LDS holds 36 rows of an Ant, and four wavefronts per CU
+      // fill its SIMDs (4096 envs in flight instead of 3072; the Ant's 4 steps of
+      // 4096 envs 1.99 -> 1.84 ms). Piles of bodies need a third (54 rows of two
+      // bodies each at 36 dofs).
       const int64_t part = (160 * 1024 / (M.nv <= 16 ? 4 : 3) - 512) / 4 / 8;  // 512: the allocation's granularity
       s->pgs_slice = (int)(std::min(most + 1, part) & ~(int64_t)1);
       const void* k = pgs_rows_kernel(M);
