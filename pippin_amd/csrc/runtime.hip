@@ -1113,7 +1113,9 @@ extern "C" int pippin_hip_get(const ph_sim* s, int32_t field, int64_t begin, int
   if (w == 0 || end == begin) return PH_OK;
   if (!out) return fail(PH_ERR_ARG, "null argument");
   const int64_t count = (end - begin) * w;
-  if ((size_t)count * sizeof(double) <= Pinned::STAGE) {
+  // (not once a device pointer to state is out: the direct copy also waits for
+  // work of the null stream, torch's default one, that writes through it)
+  if ((size_t)count * sizeof(double) <= Pinned::STAGE && !s->state_shared) {
     HIPCHK(hipSetDevice(s->device));
     std::lock_guard<std::mutex> lock(s->pin.mu);
     if (s->pin.used) HIPCHK(hipStreamSynchronize(s->stream));  // the staging of set calls

@@ -317,6 +317,32 @@ def test_set_waits_for_the_copies_of_set_device(assets, field):
     assert np.array_equal(g.get("qpos", 0, 2), np.repeat(one, 2, axis=0))
 
 
+@pytest.mark.parametrize("field", ["qpos", "qvel", "ctrl"])
+def test_get_sees_writes_of_the_default_stream(assets, field):
+    """A write through state_device's pointer that is queued on the null stream,
+    behind other work there, is done before a get call returns, however small."""
+    import torch
+
+    n = 4
+    g = HipPhysics(mjcf.load_file(assets / "ant.xml"), n)
+
+    class Field:
+        __cuda_array_interface__ = dict(shape=(n, g.width(field)), typestr="<f8", version=2,
+                                        data=(g.state_ptr(field), False))
+
+    state = torch.as_tensor(Field(), device="cuda")
+    busy = torch.zeros(1 << 26, dtype=torch.float64, device="cuda")
+    new = torch.rand((n, g.width(field)), dtype=torch.float64, device="cuda")
+    want = new.cpu().numpy()
+    for k in range(3):
+        state.zero_()
+        torch.cuda.synchronize()
+        for _ in range(20):  # some milliseconds
+            busy.add_(1.0)
+        state.copy_(new)
+        assert np.array_equal(g.get(field), want), k
+
+
 def test_device_poses_equal_host_poses(assets):
     """pippin_hip_poses_device: the f32 Pose records of every env in device
     memory, for a renderer on the GPU; equal to the host copy of poses() bit
