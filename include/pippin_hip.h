@@ -309,7 +309,10 @@ int pippin_hip_rollout_device(ph_sim* s, int64_t begin, int64_t end, int64_t nst
 int pippin_hip_state_device(ph_sim* s, int32_t field, double** ptr);
 /* Copy `field` (PH_FIELD_QVEL or PH_FIELD_CTRL) for envs [begin, end) from a DEVICE
  * buffer, ordered on the library stream before the next step (no host sync);
- * pippin_hip_get and pippin_hip_set wait for it. */
+ * pippin_hip_get and pippin_hip_set wait for it. What fills the buffer has to be
+ * done before the call: the library stream waits for no other stream. (Step,
+ * rollout_device, get and set return with work that was queued on the null stream
+ * before them done.) */
 int pippin_hip_set_device(ph_sim* s, int32_t field, int64_t begin, int64_t end, const double* src);
 /* Accumulated device time of the step launches and their number since the last
  * reset. A PH_SCHED_GRID launch counts its kernel alone (the dispatch's own time

@@ -712,9 +712,14 @@ static size_t step_lds(const ph_sim* s, int K) {
   return (size_t)K * s->M.L.bytes + (K == 1 ? (size_t)s->M.x1 * sizeof(double) : 0);
 }
 
-// Waits for the sim's stream: no copy of the staging or of set_device is in flight after it.
+// Waits for the sim's stream: no copy of the staging or of set_device is in
+// flight after it. And for the null stream (0.15 us when it is idle): callers
+// queue work on it, torch's default stream, that fills the buffers of their next
+// calls, and the blocking copies that step, get and set made before they used
+// pinned memory had waited for it.
 static hipError_t drain(const ph_sim* s) {
   if (hipError_t e = hipStreamSynchronize(s->stream)) return e;
+  if (hipError_t e = hipStreamSynchronize(nullptr)) return e;
   s->pin.used = 0;
   s->pin.device = false;
   return hipSuccess;
@@ -1149,6 +1154,7 @@ extern "C" int pippin_hip_set(ph_sim* s, int32_t field, int64_t begin, int64_t e
     HIPCHK(hipSetDevice(s->device));
     std::lock_guard<std::mutex> lock(s->pin.mu);
     if (s->pin.used + bytes > Pinned::STAGE) HIPCHK(drain(s));
+    else HIPCHK(hipStreamSynchronize(nullptr));  // see drain
     double* stage = s->pin.stage() + s->pin.used / sizeof(double);
     memcpy(stage, src, bytes);
     s->pin.used += bytes;

@@ -343,6 +343,28 @@ def test_get_sees_writes_of_the_default_stream(assets, field):
         assert np.array_equal(g.get(field), want), k
 
 
+@pytest.mark.parametrize("solver", [0, 1])
+@pytest.mark.parametrize("call", ["step", "rollout", "get", "set"])
+def test_work_of_the_default_stream_is_done_when_a_call_returns(assets, call, solver):
+    """A program that queues its policy on torch's default stream, calls the sim
+    and then hands it the policy's buffer."""
+    import torch
+
+    n = 4
+    g = HipPhysics({**mjcf.load_file(assets / "ant.xml"), "solver_kind": solver}, n)
+    busy = torch.zeros(1 << 26, dtype=torch.float64, device="cuda")
+    ctrl = torch.zeros((n, 2, g.nu), dtype=torch.float64, device="cuda")
+    q = g.get("qpos")
+    calls = dict(step=lambda: g.step(0, n, 1), get=lambda: g.get("qvel"), set=lambda: g.set("qpos", 0, n, q),
+                 rollout=lambda: g.rollout_device(ctrl.data_ptr(), None, 2))
+    for _ in range(3):
+        torch.cuda.synchronize()
+        for _ in range(20):  # some milliseconds
+            busy.add_(1.0)
+        calls[call]()
+        assert torch.cuda.default_stream().query()
+
+
 def test_device_poses_equal_host_poses(assets):
     """pippin_hip_poses_device: the f32 Pose records of every env in device
     memory, for a renderer on the GPU; equal to the host copy of poses() bit
