@@ -455,6 +455,31 @@ bool build_host_model(const ph_model_desc& s, HostModel& m, std::string* err) {
   return true;
 }
 
+bool pairs_can_touch(const HostModel& m) {
+  for (size_t p = 0; p < m.pair_g1.size(); p++) {
+    const int a = m.pair_g1[p], b = m.pair_g2[p];
+    if ((m.geom_contype[a] & m.geom_conaffinity[b]) || (m.geom_contype[b] & m.geom_conaffinity[a])) return true;
+  }
+  return false;
+}
+
+bool rows_can_meet(const HostModel& m, bool contacts) {
+  if (contacts && !m.pair_g1.empty()) return true;
+  std::vector<int> rows(m.block_adr.size(), 0);  // per dof block
+  for (int j = 0; j < m.d.njnt; j++)
+    if (m.jnt_limited[j] && (m.jnt_type[j] == PH_JNT_HINGE || m.jnt_type[j] == PH_JNT_SLIDE))
+      rows[m.dof_block[m.jnt_dofadr[j]]]++;
+  for (int e = 0; e < m.d.neq; e++) {
+    const int b1 = m.dof_block[m.jnt_dofadr[m.eq_joint1[e]]];
+    const int b2 = m.eq_joint2[e] >= 0 ? m.dof_block[m.jnt_dofadr[m.eq_joint2[e]]] : b1;
+    rows[b1]++;
+    if (b2 != b1) rows[b2]++;
+  }
+  for (int n : rows)
+    if (n > 1) return true;
+  return false;
+}
+
 // Scalars, capacities and LDS layout of the device model (pointers are left null).
 void init_dmodel_scalars(const HostModel& hm, int solver, int max_contacts, phk::DModel& M) {
   const ph_model_desc& d = hm.d;

@@ -63,6 +63,11 @@ bool has_implicit_terms(const HostModel& m, const double* dof_damping, const dou
 bool pair_static_ok(const HostModel& m, int g1, int g2);
 // LDS layout for one env: nrl rows kept in LDS, npair candidate pairs, ncmax contacts.
 phk::Layout make_layout(const HostModel& m, int nrl, int npair, int ncmax, int isl_ints);
+// Whether the model's own masks let any candidate pair touch.
+bool pairs_can_touch(const HostModel& m);
+// Whether several constraint rows of a step can act on the same dofs: those of a
+// contact (three or more), or limits and equalities of one dof block.
+bool rows_can_meet(const HostModel& m, bool contacts);
 void init_dmodel_scalars(const HostModel& hm, int solver, int max_contacts, phk::DModel& M);
 
 }  // namespace phh

@@ -12,21 +12,24 @@
 namespace phk {
 
 // The shape a sim starts with: as many envs per wavefront as fit 64 KiB of LDS
-// (lds_bytes each), on the grid schedule. PGS models with packed rows start with
-// the split step: fused, the sweeps of several envs wait for each other at every
-// row (Ant, 4096 envs, 4 steps: 9.9 ms fused, 1.84 ms split; six-body pile, 8192
-// envs: 125 and 11.0 ms). envs_per_wave (PIPPIN_HIP_ENVS_PER_WG; null: not set)
+// (lds_bytes each), on the grid schedule. PGS models whose rows pack and can meet
+// on the same dofs (split) start with the split step: fused, the sweeps of several
+// envs wait for each other at every row (Ant, 4096 envs, 4 steps: 9.9 ms fused,
+// 1.84 ms split; six-body pile, 8192 envs: 125 and 11.0 ms). Where each dof block
+// has one row at most, a sweep or two is all there is, and four launches a step
+// are more than one (1024 envs, 20 steps: cartpole 530 us fused, 907 split; a
+// hinge with a limit 485 and 892). envs_per_wave (PIPPIN_HIP_ENVS_PER_WG; null: not set)
 // asks for 1, 2 or 4 envs on the grid schedule and is ignored where it is another
 // value or more than the device's LDS per workgroup, lds_max, holds.
 struct StartShape {
   int envs_per_wave, schedule;
 };
-inline StartShape start_shape(int64_t lds_bytes, bool packed_pgs, int64_t lds_max, const char* envs_per_wave) {
+inline StartShape start_shape(int64_t lds_bytes, bool split, int64_t lds_max, const char* envs_per_wave) {
   if (envs_per_wave) {
     const int k = std::atoi(envs_per_wave);
     if ((k == 1 || k == 2 || k == 4) && k * lds_bytes <= lds_max) return {k, PH_SCHED_GRID};
   }
-  if (packed_pgs) return {1, PH_SCHED_PGS_SPLIT};
+  if (split) return {1, PH_SCHED_PGS_SPLIT};
   for (int k : {4, 2})
     if (k * lds_bytes <= 64 * 1024) return {k, PH_SCHED_GRID};
   return {1, PH_SCHED_GRID};

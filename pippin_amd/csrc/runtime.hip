@@ -270,6 +270,9 @@ struct ph_sim {
   int envs_per_wg = 1;  // environments packed into one k_step workgroup
   int spec = 0;         // 1: the model matches SpecAnt (compile-time sizes and layout)
   int sched = PH_SCHED_GRID;  // schedule of the plain step (PH_SCHED_*)
+  bool shape_chosen = false;  // set or tuned: no longer the one that the sim started with
+  bool contacts = false;      // some env's masks can let a pair touch
+  int64_t lds_max = 0;        // LDS per workgroup of the device
   int cus = 0;                // compute units of the device
   int pgs_per_cu = 0;         // wavefronts of the packed PGS sweeps that a CU holds
   int pgs_wide_per_cu = 0;    // and of the sweeps over rows that are not packed
@@ -446,6 +449,16 @@ static int variant_clone(ph_sim* s, int src) {
   return V.nvar++;
 }
 
+// The launch shape to start with (start_shape), also taken when parameters let
+// geoms touch that the model's own masks kept apart, unless a shape was set or tuned.
+static void take_start_shape(ph_sim* s) {
+  if (s->shape_chosen) return;
+  const bool split = s->M.solver_kind == 1 && s->M.pgs_w > 0 && phh::rows_can_meet(s->hm, s->contacts);
+  const StartShape first = start_shape(s->M.L.bytes, split, s->lds_max, std::getenv("PIPPIN_HIP_ENVS_PER_WG"));
+  s->envs_per_wg = first.envs_per_wave;
+  s->sched = first.schedule;
+}
+
 extern "C" int pippin_hip_create(const ph_model_desc* desc, int64_t num_envs, const ph_options* opt, ph_sim** out) {
   if (!desc || !out || num_envs < 0) return fail(PH_ERR_ARG, "null argument or negative env count");
   std::unique_ptr<ph_sim> s(new ph_sim());
@@ -472,10 +485,9 @@ extern "C" int pippin_hip_create(const ph_model_desc* desc, int64_t num_envs, co
   hipDeviceProp_t prop;
   HIPCHK(hipGetDeviceProperties(&prop, s->device));
   const int64_t lds_max = (int64_t)prop.sharedMemPerBlock;
-  const StartShape first = start_shape(M.L.bytes, M.solver_kind == 1 && M.pgs_w > 0, lds_max,
-                                       std::getenv("PIPPIN_HIP_ENVS_PER_WG"));
-  s->envs_per_wg = first.envs_per_wave;
-  s->sched = first.schedule;
+  s->lds_max = lds_max;
+  s->contacts = phh::pairs_can_touch(hm);
+  take_start_shape(s.get());
   // model-specialised kernel when the model's sizes and layout match one built
   // in (PIPPIN_HIP_SPEC=0 forces the generic kernel)
   s->spec = SpecAnt::matches(M) && M.solver_kind == 0 ? 1 : 0;
@@ -907,6 +919,7 @@ static void tune_finish(ph_sim* s) {
     s->envs_per_wg = sh.envs_per_wave;
     s->spec = sh.specialised;
     s->sched = sh.schedule;
+    s->shape_chosen = true;
     if (!s->tune_cache.empty())
       if (FILE* f = fopen(s->tune_cache.c_str(), "a")) {
         fprintf(f, "%s : %d %d %d\n", tune_key(s).c_str(), sh.envs_per_wave, sh.specialised, sh.schedule);
@@ -930,6 +943,7 @@ extern "C" int pippin_hip_set_launch_shape(ph_sim* s, const ph_launch_shape* sh)
   s->envs_per_wg = sh->envs_per_wave;
   s->spec = sh->specialised;
   s->sched = sh->schedule;
+  s->shape_chosen = true;
   s->tune_cand.clear();
   s->tune_ms.clear();
   s->tune_rounds = 0;
@@ -1449,6 +1463,11 @@ extern "C" int pippin_hip_set_param(ph_sim* s, int32_t p, int64_t id, int64_t be
     bool sc = false;
     param_apply(s, v, p, id, values + i * w, true, &sc);
     if (sc) recompute.push_back(v);
+  }
+  if ((p == PH_PARAM_GEOM_CONTYPE || p == PH_PARAM_GEOM_CONAFFINITY) && !s->contacts &&
+      std::any_of(values, values + (end - begin) * w, [](double x) { return x != 0.0; })) {
+    s->contacts = true;
+    take_start_shape(s);
   }
   HIPCHK(up(s->d_env_var, s->env_var, &s->M.env_var));
   if (int rc = upload_variants(s)) return rc;

@@ -109,6 +109,7 @@ int emu_start_shape(int64_t lds_bytes, int packed_pgs, int64_t lds_max, const ch
 int emu_learned_envs_per_wave(int shape_envs, int split, int nblock, int64_t lds_bytes, int cus, int64_t envs) {
   return learned_envs_per_wave(shape_envs, split, nblock, lds_bytes, cus, envs);
 }
+int emu_rows_can_meet(emu_sim* s) { return phh::rows_can_meet(s->hm, phh::pairs_can_touch(s->hm)); }
 int emu_timed_by_dispatch(int plain, int trial, int grid) { return timed_by_dispatch(plain, trial, grid); }
 // ms: ncand x rounds, a negative time for a launch that was not timed
 int emu_tune_choice(const double* ms, const int* prefer, int ncand, int rounds) {

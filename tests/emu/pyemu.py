@@ -29,7 +29,7 @@ def lib():
         L.emu_last_error.restype = C.c_char_p
         L.emu_general_sweep_blocks.restype = C.c_uint
         L.emu_general_sweep_blocks.argtypes = [i64, C.c_int, C.c_int]
-        for n, a in {"emu_rows": [vp, C.c_int], "emu_learned_envs_per_wave": [C.c_int, C.c_int, C.c_int, i64, C.c_int, i64],
+        for n, a in {"emu_rows": [vp, C.c_int], "emu_rows_can_meet": [vp], "emu_learned_envs_per_wave": [C.c_int, C.c_int, C.c_int, i64, C.c_int, i64],
                      "emu_start_shape": [i64, C.c_int, i64, C.c_char_p, vp, vp], "emu_tune_choice": [vp, vp, C.c_int, C.c_int],
                      "emu_timed_by_dispatch": [C.c_int, C.c_int, C.c_int], "emu_step": [vp, i64, i64, i64], "emu_step_split": [vp, i64, i64, i64, i64], "emu_get": [vp, C.c_int, i64, i64, vp],
                      "emu_set": [vp, C.c_int, i64, i64, vp], "emu_ncon": [vp, i64, i64, vp],

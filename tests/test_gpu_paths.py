@@ -214,3 +214,38 @@ def test_learned_pgs_step_is_the_same_for_every_number_of_envs_per_wavefront(ass
     for r in runs[1:]:
         for a, b in zip(runs[0], r):
             assert np.array_equal(a, b)
+
+
+def test_pgs_models_whose_rows_cannot_meet_start_fused(assets):
+    """One launch for all steps; masks that parameters open later bring the
+    split step, a shape that was set stays."""
+    arr = {**mjcf.load_file(assets / "cartpole.xml"), "solver_kind": 1}
+    g = HipPhysics(arr, 2)
+    assert g.launch_shape() == (4, 0, "grid")
+    g.close()
+    xml = (assets / "box_drop.xml").read_text().replace("<worldbody>",
+                                                        '<default><geom contype="0" conaffinity="0"/></default><worldbody>', 1)
+    arr = {**mjcf.load_string(xml), "solver_kind": 1}
+    assert not np.any(arr["geom_contype"])
+    g, fixed, o = HipPhysics(arr, 3), HipPhysics(arr, 3), OracleSim(arr, 3)
+    first = g.launch_shape()
+    assert first[2] == "grid"
+    fixed.set_launch_shape(2, 0, "grid")
+    for s in (g, fixed, o):
+        s.step(0, 3, 2)
+        for gi in range(int(arr["ngeom"])):
+            s.set_param("geom_contype", gi, 0, 3, [0.0, 0.0, 0.0])
+    assert g.launch_shape() == first
+    for s in (g, fixed, o):
+        for gi in range(int(arr["ngeom"])):
+            s.set_param("geom_contype", gi, 1, 2, [1.0])
+            s.set_param("geom_conaffinity", gi, 1, 2, [1.0])
+    assert g.launch_shape() == (1, 0, "pgs_split") and fixed.launch_shape() == (2, 0, "grid")
+    for _ in range(60):
+        for s in (g, fixed, o):
+            s.step(0, 3, 2)
+        assert np.array_equal(g.get("qpos"), o.get("qpos"))
+        assert np.array_equal(fixed.get("qpos"), o.get("qpos"))
+    assert o.ncon()[1] > 0
+    for s in (g, fixed):
+        s.close()

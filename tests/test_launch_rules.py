@@ -4,7 +4,9 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from tests.emu.pyemu import _p, lib
+from oracle import mjcf
+from tests.emu.pyemu import EmuSim, _p, lib
+from tests.scenes import COUPLED_SLIDERS
 
 GRID, SPLIT = 0, 3
 
@@ -75,3 +77,27 @@ def test_envs_per_wavefront_of_the_learned_warm_start(nblock, kib, envs, want):
     assert rule(1, 1, nblock, kib * 1024, 256, envs) == want
     for k in (1, 2, 4):
         assert rule(k, 0, nblock, kib * 1024, 256, envs) == k
+
+
+_HINGES = ('<mujoco><compiler angle="radian"/><default><geom contype="0" conaffinity="0"/></default><worldbody>'
+           '<body pos="0 0 1"><joint name="a" type="hinge" axis="0 1 0" {a}/><geom type="sphere" size=".1" pos=".2 0 0"/>'
+           '<body pos=".4 0 0"><joint name="b" type="hinge" axis="0 1 0" {b}/><geom type="sphere" size=".1" pos=".2 0 0"/>'
+           '</body></body><body pos="0 1 1"><joint name="c" type="hinge" axis="0 1 0" {c}/>'
+           '<geom type="sphere" size=".1" pos=".2 0 0"/></body></worldbody>{eq}</mujoco>')
+_LIM = 'limited="true" range="-1 1"'
+
+
+@pytest.mark.parametrize("name,want", [("cartpole.xml", 0), ("pendulum.xml", 0), ("arm3d.xml", 0), ("box_drop.xml", 1), ("ant.xml", 1)])
+def test_rows_of_the_assets_that_can_meet(assets, name, want):
+    assert lib().emu_rows_can_meet(EmuSim(mjcf.load_file(assets / name), 1).h) == want
+
+
+@pytest.mark.parametrize("a,b,c,eq,want", [
+    ("", "", "", "", 0), (_LIM, "", "", "", 0), (_LIM, "", _LIM, "", 0), (_LIM, _LIM, "", "", 1),
+    ("", "", "", "ab", 0), ("", "", "", "ac", 0), (_LIM, "", "", "ab", 1), ("", "", _LIM, "ab", 0), ("", "", _LIM, "ac", 1),
+])
+def test_limits_and_equalities_that_can_meet(a, b, c, eq, want):
+    """More than one row on a dof block: a and b are one, c another."""
+    eq = f'<equality><joint joint1="{eq[0]}" joint2="{eq[1]}"/></equality>' if eq else ""
+    assert lib().emu_rows_can_meet(EmuSim(mjcf.load_string(_HINGES.format(a=a, b=b, c=c, eq=eq)), 1).h) == want
+    assert lib().emu_rows_can_meet(EmuSim(mjcf.load_string(COUPLED_SLIDERS), 1).h) == 1
