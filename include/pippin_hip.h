@@ -339,7 +339,9 @@ enum {
                              a second sweep launch, one env per wavefront in registers, takes the envs with
                              more rows than that holds (and all envs of other models). The first and last
                              launches pick 1, 2 or 4 envs per wavefront by the range. Models whose rows
-                             pack start with this schedule. */
+                             pack start with this schedule, if contacts, or several limits and
+                             equalities of one dof block, can act on the same dofs; masks opened by
+                             pippin_hip_set_param bring it in, unless a shape was set or tuned. */
 };
 typedef struct ph_launch_shape {
   int32_t envs_per_wave; /* K: 1, 2 or 4 envs per 64-lane wavefront */
