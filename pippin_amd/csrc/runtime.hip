@@ -228,7 +228,11 @@ static const void* pgs_rows_kernel(const DModel& M) {
 // stream. (A blocking copy to or from pageable memory took 12 to 20 us of the
 // 125 us of a host-driven step of one env.)
 struct Pinned {
-  static constexpr size_t STAGE = 256 * 1024;  // bytes; larger calls copy directly
+  static constexpr size_t STAGE = 256 * 1024;  // bytes that set calls stage; larger ones copy directly
+  // get calls that stage are smaller. The runtime's blocking copy out takes 14 to
+  // 16.6 us up to a little over 16 KiB, a staged one 14.5 to 15.5; above that the
+  // runtime copies in place in 11 us (117 KiB 16.0), a staged one in 15.5 (19.4)
+  static constexpr size_t GET_STAGE = 17 * 1024;
   char* p = nullptr;
   size_t used = 0;  // staging bytes whose copies may still be in flight
   bool device = false;  // copies of set_device may still be in flight
@@ -1134,7 +1138,7 @@ extern "C" int pippin_hip_get(const ph_sim* s, int32_t field, int64_t begin, int
   const int64_t count = (end - begin) * w;
   // (not once a device pointer to state is out: the direct copy also waits for
   // work of the null stream, torch's default one, that writes through it)
-  if ((size_t)count * sizeof(double) <= Pinned::STAGE && !s->state_shared) {
+  if ((size_t)count * sizeof(double) < Pinned::GET_STAGE && !s->state_shared) {
     HIPCHK(hipSetDevice(s->device));
     std::lock_guard<std::mutex> lock(s->pin.mu);
     if (s->pin.used) HIPCHK(hipStreamSynchronize(s->stream));  // the staging of set calls

@@ -20,9 +20,10 @@ def say(*a):
 
 @pytest.mark.parametrize("shared", [False, True])
 def test_get_and_set_on_both_sides_of_the_staging(assets, shared):
-    """Up to 256 KiB (2184 Ants' qpos) go through pinned staging, which several
-    calls in a row fill; more is copied directly, as is every set call after a
-    device pointer to state was handed out."""
+    """Set calls of up to 256 KiB (2184 Ants' qpos) go through pinned staging,
+    which several calls in a row fill, and get calls below 17 KiB (145 Ants);
+    more is copied directly, as is every call after a device pointer to state
+    was handed out."""
     n = 2300
     say("staging, shared", shared)
     arr = mjcf.load_file(assets / "ant.xml")
@@ -40,7 +41,7 @@ def test_get_and_set_on_both_sides_of_the_staging(assets, shared):
         want[b:e] = x
         x[:] = np.nan  # the caller's array is free again when the call returns
     assert np.array_equal(g.get("qpos"), want)
-    for b, e in [(0, 1), (2299, 2300), (0, 2184), (0, 2185), (116, 2300)]:
+    for b, e in [(0, 1), (2299, 2300), (0, 145), (0, 146), (7, 152), (0, 2184), (0, 2185), (116, 2300)]:
         assert np.array_equal(g.get("qpos", b, e), want[b:e]), (b, e)
     g.close()
 
